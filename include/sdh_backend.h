@@ -113,8 +113,9 @@ int sdh_gemm_nt_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda
 /* backend_cuda.h:45-47 conv2d(); tensor.h:159 (tensor.cpp:520-560).
  * x [N, Cin, H, W], w [Cout, Cin, kh, kw] fp32, bias [Cout] or NULL,
  * out [N, Cout, Ho, Wo] with Ho = (H + 2 pad - kh) / stride + 1 (and Wo
- * alike); zero padding. Patches gathered per pixel chunk, then the fp32
- * GEMM: completes the reference's backend interface, not a tuned path. */
+ * alike); zero padding. out must not overlap the inputs. An implicit GEMM with
+ * fp32 accuracy; it takes scratch of about the size of x and w, or at most
+ * 128 MB where the arena has no more. */
 int sdh_conv2d(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, const float* w, int64_t Cout, int64_t kh,
                int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo);
 /* Tensor::to_bf16 (tensor.cpp:131-137) on device memory: y[i] = bf16 bits of

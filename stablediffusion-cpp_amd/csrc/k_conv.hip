@@ -1,16 +1,16 @@
-// k_conv.hip - conv2d (backend_cuda.h:45-47; tensor.cpp:520-560) as gather +
-// library GEMM, so that backend_hip covers every function of the reference's
-// backend interface and tensor.cpp's device branches run unchanged on it.
+// k_conv.hip - conv2d (backend_cuda.h:45-47; tensor.cpp:520-560).
 //
-// Not a tuned path (convolutions are outside this backend's elementwise /
-// reduction scope): per sample, pixels are taken in chunks of at most 2^25
-// gathered floats; k_gather_patches writes cols[p, (ci, ky, kx)] (the patch
-// that output pixel p sees, zero over the padding; (ci, ky, kx) is the
-// [Cout, Cin, kh, kw] weight's own order, so the weight is already a
-// [Cout, K] matrix); then out[Cout, pixels] = W cols^T through
-// sdh_gemm_nt_f32 (hipBLASLt with fp32 operands), written straight into the
-// NCHW output (ldc = Ho * Wo); the bias is added per output channel after
-// the last chunk (sdh_add_channel_bias).
+// The implicit GEMM on split fp16 operands (k_gemm_split.hip) takes it, at every
+// size measured ([1,256,512,512] to 256 channels, 3x3: 6.4 ms with the path below,
+// 0.90-0.96 ms; [2,4,64,64] to 320: 32 and 22 us). What follows runs where that
+// one's scratch (about the size of x and w) does not fit the arena or would have
+// to grow during a capture, in at most 128 MB: per sample, pixels in chunks of at
+// most 2^25 gathered floats; k_gather_patches writes cols[p, (ci, ky, kx)] (the
+// patch that output pixel p sees, zero over the padding; (ci, ky, kx) is the
+// [Cout, Cin, kh, kw] weight's own order, so the weight is already a [Cout, K]
+// matrix); then out[Cout, pixels] = W cols^T through sdh_gemm_nt_f32, written
+// straight into the NCHW output (ldc = Ho * Wo); the bias is added per output
+// channel after the last chunk (sdh_add_channel_bias).
 #include <algorithm>
 
 #include "sdh_backend.h"
@@ -57,6 +57,10 @@ void run_conv2d(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     check_range(w, (size_t)(Cout * K) * 4, op, "w");
     check_range(out, (size_t)(N * Cout * HW) * 4, op, "out");
     if (bias) check_range(bias, (size_t)Cout * 4, op, "bias");
+    if (split_conv(x, N, Cin, H, W, w, Cout, kh, kw, bias, stride, pad, out, Ho, Wo)) {
+        launched(op);
+        return;
+    }
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(HW, kChunkFloats / K));
     float* cols = (float*)scratch((size_t)(chunk * K) * 4);
     for (int64_t n = 0; n < N; ++n) {

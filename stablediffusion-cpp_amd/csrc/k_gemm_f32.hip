@@ -1,15 +1,14 @@
 // k_gemm_f32.hip - the linear layer with fp32 weights: C[M,N] = A[M,K] * B[N,K]^T
 // (+ C) (+ bias[N]) in fp32 (backend_cuda.h:38-40, gemm_nt_f32; the reference's
 // device path is an fp32 SGEMM, backend_cuda.cu:453-464, its CPU path fp32
-// micro-kernels, tensor.cpp:354-406). Z-Image keeps every weight under 2^20
-// elements in fp32 (safetensors.cpp:110-116 with keep_bf16, pipeline.cpp:113):
-// the patch and caption embedders' small relatives, the timestep MLP, the
-// final layer's modulation and projection. Those layers are small (at most
-// about 1 GFLOP at 1024x1024), so this is a plain register-blocked fp32 FMA
-// kernel on the vector ALUs, exact in fp32 like both reference paths:
-// 64 x 64 output tile per 256-thread workgroup, 4 x 4 per thread, K in steps
-// of 16 through LDS (A and B tiles stored k-major, so a thread's four rows or
-// columns are one float4 read).
+// micro-kernels, tensor.cpp:354-406): every linear of SD 1.x's UNet and text
+// encoder and of the VAE, and Z-Image's weights under 2^20 elements
+// (safetensors.cpp:110-116 with keep_bf16, pipeline.cpp:113). Large products run
+// on split fp16 operands (k_gemm_split.hip), small ones on the library's fp32
+// GEMM; what neither takes on the kernel below, a plain register-blocked fp32
+// FMA kernel on the vector ALUs: 64 x 64 output tile per 256-thread workgroup,
+// 4 x 4 per thread, K in steps of 16 through LDS (A and B tiles stored k-major,
+// so a thread's four rows or columns are one float4 read).
 //
 // Also sdh_to_bf16: float32 -> bf16 bits on the device with the reference's
 // rounding (nearest even; inf and NaN keep their top bits; tensor.cpp:114-121).
@@ -116,9 +115,24 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     }
     check_range(C, (size_t)((M - 1) * ldc + N) * 4, op, "C");
     if (bias) check_range(bias, (size_t)N * 4, op, "bias");
+    const bool lt = K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) &&
+                    aligned(C, 16) && (!bias || aligned(bias, 16));
+    // Split operands from the size where their pack and second launch pay
+    // (MI355X, us, the library's fp32 GEMM in front): [4096,512] x [512,512] 22.8 /
+    // 22.2 alone and 5 us more among other calls, [512,1280] x [1280,1280] 21.9 /
+    // 28.8, [64,1280] x [10240,1280] 25 / 38, [512,640] x [5120,640] 42 / 32,
+    // [256,1280] x [10240,1280] 69 / 49, [8192,320] x [2560,320] 131 / 65,
+    // [4224,2560] x [3840,2560] 610 / 238. Operands that the library path does not
+    // take: from the size where the kernel below is slower ([130,33] x [70,33]
+    // 8.6 / 9.3, [257,321] x [300,321] 31.6 / 10.8).
+    const bool large = 2.0 * (double)M * (double)N * (double)K >= 3e9 && M >= 128 && N >= 128;
+    if (K > 0 && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
+        split_gemm(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
+        launched(op);
+        return;
+    }
     // the library GEMM for aligned operands (fp32 products, fp32 accumulation)
-    if (K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) && aligned(C, 16) &&
-        (!bias || aligned(bias, 16)) && blaslt_gemm(true, M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
+    if (lt && blaslt_gemm(true, M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
         launched(op);
         return;
     }

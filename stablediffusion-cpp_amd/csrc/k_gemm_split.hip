@@ -1,0 +1,833 @@
+// k_gemm_split.hip - fp32 matrix products on the fp16 matrix cores: the linear
+// layer with fp32 weights (backend_cuda.h:38-40, gemm_nt_f32) and conv2d
+// (backend_cuda.h:45-47; tensor.cpp:520-560) as an implicit GEMM.
+//
+// What bounds these: gfx950's fp32 MFMA runs at 157 TFLOP/s, 1/16 of the fp16
+// rate. Every operand is therefore split as in the attention kernels: a block
+// of values is scaled by a power of two 2^-e that brings its largest magnitude
+// into [2^14, 2^15), each scaled value x becomes hi = rne16(x) and
+// lo = rne16(x - hi), and a product is lo_a hi_b + hi_a lo_b + hi_a hi_b with
+// fp32 accumulation: three fp16 MFMAs per fp32 product. |x - hi - lo| is at most
+// 2^-23 |x| while |x| >= 2^-16 of the block's largest value and at most 2^-39
+// of that value below it; the dropped lo_a lo_b is at most 2^-24 of the product.
+// Against 64-bit results the products come out closer than the fp32 MFMA's,
+// whose K additions round one by one where these round once per 16 products.
+//   linear  a block is one row of A, one row of B (one output feature)
+//   conv2d  a block is one output channel's weights; one sample of x
+// The exponents are exact and are applied to the accumulators at the end.
+// A tile that meets a row holding an infinity or a NaN, or (conv2d) a run of
+// 256 pixels whose values are all below 2^-14 of the sample's largest (where
+// the bound above would be looser than fp32's), is computed by plain fp32
+// FMAs from the original operands instead, so such inputs give what fp32 gives.
+//
+// Packed operands (library scratch): K is cut into steps of 32; a step of a row
+// is 128 bytes, 32 hi halves then 32 lo halves, and all rows of a step lie
+// together (a plane). For conv2d a row is a pixel and a step 32 input channels
+// under one kernel tap: the planes of x hold each pixel once and a step reads
+// them at the tap's offset (one more row of zeros stands for the padding), so
+// no patch matrix is written; the weights are packed in the steps' order
+// (channels slowest, so that the nine taps of 32 channels follow each other
+// and find the same pixels in L2).
+//
+// Product kernel: BM x BN tile, operands from global memory straight into LDS
+// (buffer loads, two stages), rows of 128 bytes with 16-byte chunk c of row r at
+// c ^ ((r >> 1) & 7): fragment reads of 16 consecutive rows hit 16 distinct chunks.
+// v_mfma_f32_32x32x16_f16: lane l holds row l % 32 of A and of B, k (l / 32) * 8 .. + 7;
+// result column l % 32, rows (i / 4) * 8 + (l / 32) * 4 + i % 4.
+#include <algorithm>
+
+#include "sdh_internal.hpp"
+
+namespace sdh {
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16;
+using dev::f4;
+
+constexpr int kStep = 32;            // K per step
+constexpr int kRowBytes = 128;       // one row of one step: 32 hi, 32 lo
+constexpr int kBad = 1 << 20;        // exponent of a row that holds an infinity or a NaN
+constexpr unsigned kInf = 0x7F800000u;
+constexpr int kBufferWord3 = 0x00020000;  // raw buffer resource, 32-bit data format
+constexpr int kPixBlock = 256, kChanBlock = 32;  // conv2d: x's maxima are kept per this many pixels and channels
+
+__device__ __forceinline__ unsigned absbits(float x) { return __float_as_uint(x) & 0x7FFFFFFFu; }
+
+// The exponent of a block whose largest magnitude has these bits: scaled by
+// 2^-e it lies in [2^14, 2^15). kBad if it is not finite.
+__device__ __forceinline__ int exp_of(unsigned bits) {
+    if (bits >= kInf) return kBad;
+    if (bits == 0) return 0;
+    return max((int)(bits >> 23), 1) - 141;
+}
+
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
+    return v;
+}
+
+// Eight values scaled by 2^s and split.
+__device__ __forceinline__ void split8(const float* x, int s, h8& hi, h8& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float v = __builtin_amdgcn_ldexpf(x[e], s);
+        hi[e] = (_Float16)v;
+        lo[e] = (_Float16)(v - (float)hi[e]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Pack of dense rows: X [rows, K] (ld) -> planes, exps. One wave per row: the
+// row's largest magnitude first, then (from L1/L2) eight values per lane and turn.
+// ---------------------------------------------------------------------------
+struct PackRows {
+    const float* X;
+    int64_t ld;
+    u16* P;
+    int* exps;
+    int rows, K;
+};
+
+__device__ __forceinline__ unsigned umax4(const f4& v) {
+    return max(max(absbits(v.x), absbits(v.y)), max(absbits(v.z), absbits(v.w)));
+}
+__device__ __forceinline__ void store_split(u16* o, const float* v, int s) {
+    h8 hi, lo;
+    split8(v, s, hi, lo);
+    *(h8*)o = hi;
+    *(h8*)(o + kStep) = lo;
+}
+
+// TURNS > 0: float4 loads (K, ld and X aligned for them) of a row of at most
+// 512 TURNS values, all in flight at once and kept in registers. TURNS = 0:
+// any row, read twice.
+template <int TURNS>
+__device__ __forceinline__ void pack_row(const PackRows& a, int row, int lane) {
+    const float* x = a.X + (int64_t)row * a.ld;
+    const int kp = (a.K + kStep - 1) / kStep * kStep;
+    auto out = [&](int k) __attribute__((always_inline)) {
+        return a.P + ((int64_t)(k / kStep) * a.rows + row) * (kRowBytes / 2) + (k % kStep);
+    };
+    unsigned m = 0;
+    if constexpr (TURNS > 0) {
+        f4 v[TURNS][2];
+#pragma unroll
+        for (int j = 0; j < TURNS; ++j) {  // past the row: its last four values, dropped below
+            const int k = (j * 64 + lane) * 8;
+            v[j][0] = *(const f4*)(x + min(k, a.K - 4));
+            v[j][1] = *(const f4*)(x + min(k + 4, a.K - 4));
+        }
+#pragma unroll
+        for (int j = 0; j < TURNS; ++j) m = max(m, max(umax4(v[j][0]), umax4(v[j][1])));
+        const int e = exp_of(wave_umax(m));
+        if (lane == 0) a.exps[row] = e;
+#pragma unroll
+        for (int j = 0; j < TURNS; ++j) {
+            const int k = (j * 64 + lane) * 8;
+            if (k >= kp) continue;
+            float f[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = k + i < a.K ? v[j][i / 4][i % 4] : 0.f;
+            store_split(out(k), f, e == kBad ? 0 : -e);
+        }
+    } else {
+        for (int k = lane; k < a.K; k += 64) m = max(m, absbits(x[k]));
+        const int e = exp_of(wave_umax(m));
+        if (lane == 0) a.exps[row] = e;
+        for (int k = lane * 8; k < kp; k += 512) {
+            float f[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = k + i < a.K ? x[k + i] : 0.f;
+            store_split(out(k), f, e == kBad ? 0 : -e);
+        }
+    }
+}
+
+// Both operands in one launch: the first ba workgroups take A's rows, the rest B's.
+template <int TURNS>
+__global__ __launch_bounds__(256) void k_split_pack(PackRows a, PackRows b, int ba) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const bool first = (int)blockIdx.x < ba;
+    const PackRows& p = first ? a : b;
+    const int row = ((int)blockIdx.x - (first ? 0 : ba)) * 4 + w;
+    if (row < p.rows) pack_row<TURNS>(p, row, lane);
+}
+
+// ---------------------------------------------------------------------------
+// conv2d's pack. Launch 1: the maxima of x per (sample, 32 channels, 256
+// pixels), and the weights. Launch 2: the pixels, with the sample's exponent.
+// ---------------------------------------------------------------------------
+struct ConvPack {
+    const float* x;       // [N, Cin, HW]
+    const float* w;       // [Cout, Cin, taps]
+    unsigned* maxima;     // [N, ncb, npb]
+    u16* X;               // planes of N * HW + 1 pixels
+    u16* Wp;              // planes of Cout rows
+    int* ex;              // [N]
+    int* ew;              // [Cout]
+    unsigned* bad;        // [N, npb]: this run of pixels needs the fp32 path
+    int N, Cin, HW, Cout, taps;
+    int ncb, npb, chunks;  // 32-channel blocks, 256-pixel blocks, 32-channel steps
+    int per;               // 32-channel steps that a workgroup of launch 2 packs
+};
+
+__global__ __launch_bounds__(256) void k_conv_prep(ConvPack a, int nmax, int in_lds) {
+    extern __shared__ float row[];
+    __shared__ unsigned red[4];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    unsigned m = 0;
+    if ((int)blockIdx.x < nmax) {
+        const int pb = blockIdx.x % a.npb, cb = blockIdx.x / a.npb % a.ncb, n = blockIdx.x / (a.npb * a.ncb);
+        const int c0 = cb * kChanBlock, p = min(pb * kPixBlock + t, a.HW - 1);  // past the last pixel: that one again
+        const float* x = a.x + ((int64_t)n * a.Cin + c0) * a.HW + p;
+        float v[kChanBlock];
+#pragma unroll
+        for (int c = 0; c < kChanBlock; ++c) v[c] = x[(int64_t)min(c, a.Cin - 1 - c0) * a.HW];
+#pragma unroll
+        for (int c = 0; c < kChanBlock; ++c) m = max(m, absbits(v[c]));
+        m = wave_umax(m);
+        if (lane == 0) red[wv] = m;
+        __syncthreads();
+        if (t == 0) a.maxima[blockIdx.x] = max(max(red[0], red[1]), max(red[2], red[3]));
+        return;
+    }
+    // one output channel's weights: [Cin][taps] -> steps (32 channels, tap),
+    // through LDS where the launch gave it room for them
+    const int co = blockIdx.x - nmax, K = a.Cin * a.taps;
+    const float* w = a.w + (int64_t)co * K;
+    if (in_lds) {
+#pragma unroll 8
+        for (int k = t; k < K; k += 256) {
+            const float v = w[k];
+            row[k] = v;
+            m = max(m, absbits(v));
+        }
+    } else {
+#pragma unroll 8
+        for (int k = t; k < K; k += 256) m = max(m, absbits(w[k]));
+    }
+    m = wave_umax(m);
+    if (lane == 0) red[wv] = m;
+    __syncthreads();
+    const int e = exp_of(max(max(red[0], red[1]), max(red[2], red[3])));
+    if (t == 0) a.ew[co] = e;
+    const int tasks = a.chunks * a.taps * 4;
+    for (int i = t; i < tasks; i += 256) {  // eight channels of one step
+        const int g = i & 3, step = i >> 2, chunk = step / a.taps, tap = step - chunk * a.taps, c0 = chunk * kStep + g * 8;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = (c0 + j) * a.taps + tap;
+            v[j] = c0 + j < a.Cin ? (in_lds ? row[k] : w[k]) : 0.f;
+        }
+        store_split(a.Wp + ((int64_t)step * a.Cout + co) * (kRowBytes / 2) + g * 8, v, e == kBad ? 0 : -e);
+    }
+}
+
+// One workgroup: 64 pixels of a sample, `per` steps of 32 channels; each step
+// through LDS, so that x is read in runs of 64 pixels and a step of 64 pixels is
+// written as 8 KB in a row. Grid: (pixel tiles, channel groups, samples).
+__global__ __launch_bounds__(256) void k_conv_pack(ConvPack a) {
+    __shared__ unsigned red[4];
+    __shared__ __attribute__((aligned(16))) u16 tile[64 * 64];
+    const int t = threadIdx.x, lane = t & 63, g = t >> 6, n = blockIdx.z;
+    const unsigned* mx = a.maxima + (int64_t)n * a.ncb * a.npb;
+    unsigned m = 0;
+    for (int i = t; i < a.ncb * a.npb; i += 256) {
+        const unsigned v = mx[i];
+        if (v < kInf) m = max(m, v);
+    }
+    m = wave_umax(m);
+    if (lane == 0) red[g] = m;
+    __syncthreads();
+    m = max(max(red[0], red[1]), max(red[2], red[3]));
+    const int e = exp_of(m);
+    const int p0 = blockIdx.x * 64, pix = p0 + lane;
+    if (blockIdx.y == 0 && t == 0) {
+        if (p0 == 0) a.ex[n] = e;
+        if (p0 % kPixBlock == 0) {
+            const int pb = p0 / kPixBlock;
+            unsigned b = 0;
+            for (int c = 0; c < a.ncb; ++c) b = max(b, mx[c * a.npb + pb]);
+            // not finite, or all of it below 2^-14 of the sample's largest (14 << 23 in exponent bits)
+            a.bad[n * a.npb + pb] = b >= kInf || (b != 0 && b + (14u << 23) < m) ? 1u : 0u;
+        }
+    }
+    const int64_t prows = (int64_t)a.N * a.HW + 1;
+    const int s0 = blockIdx.y * a.per, s1 = min(a.chunks, s0 + a.per);
+    float v[8];
+    auto load = [&](int s) __attribute__((always_inline)) {  // channels past the last: that one again, dropped below
+        const int c0 = s * kStep + g * 8;
+        const float* x = a.x + (int64_t)n * a.Cin * a.HW + min(pix, a.HW - 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = x[(int64_t)min(c0 + j, a.Cin - 1) * a.HW];
+    };
+    load(s0);
+    for (int s = s0; s < s1; ++s) {
+        const int c0 = s * kStep + g * 8;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = c0 + j < a.Cin ? v[j] : 0.f;
+        h8 hi, lo;
+        split8(v, -e, hi, lo);
+        if (s + 1 < s1) load(s + 1);
+        __syncthreads();  // the previous step's tile is read
+        *(h8*)(tile + lane * 64 + ((g ^ (lane & 7)) << 3)) = hi;
+        *(h8*)(tile + lane * 64 + (((g + 4) ^ (lane & 7)) << 3)) = lo;
+        __syncthreads();
+        u16* out = a.X + ((int64_t)s * prows + (int64_t)n * a.HW + p0) * 64;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int i = t + j * 256, r = i >> 3, c = i & 7;
+            if (p0 + r < a.HW) *(h8*)(out + i * 8) = *(const h8*)(tile + r * 64 + ((c ^ (r & 7)) << 3));
+        }
+        if (n == a.N - 1 && p0 + 64 >= a.HW && t < 8)  // the row of zeros
+            *(u32x4*)(a.X + ((int64_t)s * prows + prows - 1) * 64 + t * 8) = u32x4{0, 0, 0, 0};
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The product
+// ---------------------------------------------------------------------------
+struct SplitArgs {
+    const u16* A;
+    const u16* B;
+    int64_t planeA, planeB;  // bytes from one step's rows to the next's
+    const int* ea;           // per row
+    const int* eb;           // per column; conv2d: per sample
+    float* C;
+    int64_t ldc;
+    const float* bias;       // per column; conv2d: per row
+    int M, N, K;
+    int steps, accumulate;
+    int tm, tn, splits;      // tiles, parts of K
+    float* part;             // splits > 1: [splits][tm * BM][tn * BN] sums without the exponents
+    unsigned* slow;          // splits > 1: [tm * tn], the tile was computed by the fp32 path
+    // the original operands
+    const float* A0;
+    const float* B0;
+    int64_t lda, ldb;
+    // conv2d
+    const unsigned* bad;
+    int H, W, Wo, HWo, kh, kw, stride, pad, taps, Cin, Cout, npb, zero;
+};
+
+// One element by fp32 FMAs from the original operands.
+template <bool CONV>
+__device__ __forceinline__ float dot_fp32(const SplitArgs& p, int row, int col) {
+    float s = 0.f;
+    if constexpr (CONV) {
+        const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
+        const int iy0 = oy * p.stride - p.pad, ix0 = ox * p.stride - p.pad;
+        const float* w = p.A0 + (int64_t)row * p.Cin * p.taps;
+        for (int ci = 0; ci < p.Cin; ++ci) {
+            const float* x = p.B0 + ((int64_t)n * p.Cin + ci) * p.H * p.W;
+            for (int ky = 0; ky < p.kh; ++ky)
+                for (int kx = 0; kx < p.kw; ++kx, ++w) {
+                    const int iy = iy0 + ky, ix = ix0 + kx;
+                    const bool in = (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
+                    s = fmaf(*w, in ? x[(int64_t)iy * p.W + ix] : 0.f, s);
+                }
+        }
+    } else {
+        const float* a = p.A0 + (int64_t)row * p.lda;
+        const float* b = p.B0 + (int64_t)col * p.ldb;
+        for (int k = 0; k < p.K; ++k) s = fmaf(a[k], b[k], s);
+    }
+    return s;
+}
+
+// Where element (row, col) lies, and what is added to it.
+template <bool CONV>
+__device__ __forceinline__ float* place(const SplitArgs& p, int row, int col) {
+    if constexpr (CONV) {
+        const int n = col / p.HWo;
+        return p.C + ((int64_t)n * p.Cout + row) * p.HWo + (col - n * p.HWo);
+    } else {
+        return p.C + (int64_t)row * p.ldc + col;
+    }
+}
+template <bool CONV>
+__device__ __forceinline__ void store(const SplitArgs& p, int row, int col, float* cp, float v) {
+    if (p.accumulate) v += *cp;
+    if (p.bias) v += p.bias[CONV ? row : col];
+    *cp = v;
+}
+
+// COUNT loads of 64 x 16 bytes into LDS, one after the other from dst on: lane l
+// of load j reads base + v[j] (a buffer of `bytes` bytes) for dst + 512 j + 8 l.
+template <int COUNT>
+__device__ __forceinline__ void load_lds(const char* base, int bytes, const int* v, u16* dst) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, bytes, kBufferWord3);
+#pragma unroll
+    for (int j = 0; j < COUNT; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst + j * 512), 16, v[j],
+                                                 0, 0, 0);
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, bool CONV>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1 : BM * BN == 128 * 128 ? 2 : 3) void k_split_mm(SplitArgs p) {
+    static_assert(STAGES == 2 || STAGES == 3, "LDS stages");
+    constexpr int NW = (BM / WM) * (BN / WN), T = 64 * NW;
+    constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;  // loads per wave and stage: 8 rows each
+    constexpr int RA = WM / 32, RB = WN / 32;
+    __shared__ __attribute__((aligned(1024))) u16 sA0[BM * 64];
+    __shared__ __attribute__((aligned(1024))) u16 sA1[BM * 64];
+    __shared__ __attribute__((aligned(1024))) u16 sA2[STAGES > 2 ? BM * 64 : 8];
+    __shared__ __attribute__((aligned(1024))) u16 sB0[BN * 64];
+    __shared__ __attribute__((aligned(1024))) u16 sB1[BN * 64];
+    __shared__ __attribute__((aligned(1024))) u16 sB2[STAGES > 2 ? BN * 64 : 8];
+    __shared__ __attribute__((aligned(16))) int sea[BM];  // exponents of the rows, of the columns
+    __shared__ int seb[BN];
+    __shared__ float sbias[CONV ? BM : BN];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = w / (BN / WN), wn = w % (BN / WN);
+    const int fr = lane & 31, fh = lane >> 5;
+    // Workgroups go to the 8 XCDs round robin: renumbered so that each XCD runs
+    // one contiguous range of tiles; within it, eight row tiles by all columns.
+    const int nblk = gridDim.x, xcd = blockIdx.x & 7, per = nblk >> 3, rem = nblk & 7;
+    const int lb = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+    const int tiles = p.tm * p.tn, z = lb / tiles, lt = lb - z * tiles;
+    const int gsz = 8 * p.tn, grp = lt / gsz, in = lt - grp * gsz, gm = min(8, p.tm - grp * 8);
+    const int mt = grp * 8 + in % gm, nt = in / gm;
+    const int m0 = mt * BM, n0 = nt * BN;
+
+    // rows and columns that need the fp32 path
+    bool bad = false;
+    for (int i = t; i < BM; i += T) {
+        const int row = min(m0 + i, p.M - 1), e = p.ea[row];
+        sea[i] = e;
+        if (CONV) sbias[i] = p.bias ? p.bias[row] : 0.f;
+        bad |= e == kBad;
+    }
+    for (int i = t; i < BN; i += T) {
+        const int col = min(n0 + i, p.N - 1);
+        if constexpr (CONV) {
+            const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
+            seb[i] = p.eb[n];
+            const int xa = min(max(ox * p.stride - p.pad, 0), p.W - 1);
+            const int xb = min(max(ox * p.stride - p.pad + p.kw - 1, 0), p.W - 1);
+            for (int ky = 0; ky < p.kh; ++ky) {
+                const int iy = min(max(oy * p.stride - p.pad + ky, 0), p.H - 1);
+                for (int b = (iy * p.W + xa) / kPixBlock; b <= (iy * p.W + xb) / kPixBlock; ++b)
+                    bad |= p.bad[n * p.npb + b] != 0;
+            }
+        } else {
+            const int e = p.eb[col];
+            seb[i] = e;
+            sbias[i] = p.bias ? p.bias[col] : 0.f;
+            bad |= e == kBad;
+        }
+    }
+    if (__syncthreads_or(bad)) {
+        if (z == 0) {
+            if (p.splits > 1 && t == 0) p.slow[lt] = 1;
+            for (int i = t; i < BM * BN; i += T) {
+                const int row = m0 + i / BN, col = n0 + i % BN;
+                if (row < p.M && col < p.N) store<CONV>(p, row, col, place<CONV>(p, row, col), dot_fp32<CONV>(p, row, col));
+            }
+        }
+        return;
+    }
+    if (p.splits > 1 && z == 0 && t == 0) p.slow[lt] = 0;
+
+    // this lane's source row in each of the wave's loads; rows past the matrix
+    // read its last row (their results are not stored)
+    const int lr = lane >> 3;
+    int va[AI], vb[BI];
+    int iy0[CONV ? BI : 1], ix0[CONV ? BI : 1];
+#pragma unroll
+    for (int j = 0; j < AI; ++j) {
+        const int r = (w * AI + j) * 8 + lr;
+        va[j] = min(m0 + r, p.M - 1) * kRowBytes + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
+#pragma unroll
+    for (int j = 0; j < BI; ++j) {
+        const int r = (w * BI + j) * 8 + lr, col = min(n0 + r, p.N - 1);
+        const int chunk = ((lane & 7) ^ ((r >> 1) & 7)) << 4;
+        if constexpr (CONV) {
+            const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
+            iy0[j] = oy * p.stride - p.pad;
+            ix0[j] = ox * p.stride - p.pad;
+            vb[j] = (n * p.H * p.W + iy0[j] * p.W + ix0[j]) * kRowBytes + chunk;  // may lie before the sample
+        } else {
+            vb[j] = col * kRowBytes + chunk;
+        }
+    }
+    const int bytesA = p.M * kRowBytes, bytesB = (CONV ? p.zero + 1 : p.N) * kRowBytes;
+    auto issue = [&](int step, u16* dA, u16* dB) __attribute__((always_inline)) {
+        int chunk = step, tap = 0;
+        if constexpr (CONV) {
+            chunk = step / p.taps;
+            tap = step - chunk * p.taps;
+        }
+        load_lds<AI>((const char*)p.A + step * p.planeA, bytesA, va, dA + w * AI * 512);
+        int v[BI];
+        const int ky = CONV ? tap / p.kw : 0, kx = tap - ky * (CONV ? p.kw : 0);
+#pragma unroll
+        for (int j = 0; j < BI; ++j) {
+            v[j] = vb[j];
+            if constexpr (CONV) {
+                const bool ok = (unsigned)(iy0[j] + ky) < (unsigned)p.H && (unsigned)(ix0[j] + kx) < (unsigned)p.W;
+                v[j] = ok ? v[j] + (ky * p.W + kx) * kRowBytes : p.zero * kRowBytes + (v[j] & 127);
+            }
+        }
+        load_lds<BI>((const char*)p.B + chunk * p.planeB, bytesB, v, dB + w * BI * 512);
+    };
+
+    f32x16 acc[RA][RB];
+#pragma unroll
+    for (int a = 0; a < RA; ++a)
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+
+    // Fragment addresses: rows 32 apart share their swizzle, so a lane has one
+    // chunk offset for each (slice, hi or lo).
+    const int offA = (wm * WM + fr) * 64, offB = (wn * WN + fr) * 64;
+    int at[2][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int l = 0; l < 2; ++l) at[s][l] = ((s * 2 + l * 4 + fh) ^ ((fr >> 1) & 7)) << 3;
+    // A stage is 2 RA turns (slice of 16 k, 32 rows of A) of 3 RB MFMAs; the
+    // fragments of a turn are read one turn ahead.
+    auto compute = [&](const u16* tA, const u16* tB) __attribute__((always_inline)) {
+        h8 ah[2], al[2], bh[2][RB], bl[2][RB];
+        auto fragA = [&](int i, h8& hi, h8& lo) __attribute__((always_inline)) {
+            hi = *(const h8*)(tA + offA + (i % RA) * 2048 + at[i / RA][0]);
+            lo = *(const h8*)(tA + offA + (i % RA) * 2048 + at[i / RA][1]);
+        };
+        auto fragB = [&](int s, h8* hi, h8* lo) __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < RB; ++b) {
+                hi[b] = *(const h8*)(tB + offB + b * 2048 + at[s][0]);
+                lo[b] = *(const h8*)(tB + offB + b * 2048 + at[s][1]);
+            }
+        };
+        fragB(0, bh[0], bl[0]);
+        fragA(0, ah[0], al[0]);
+#pragma unroll
+        for (int i = 0; i < 2 * RA; ++i) {
+            const int s = i / RA, a = i % RA, q = i & 1;
+            if (i + 1 < 2 * RA) fragA(i + 1, ah[q ^ 1], al[q ^ 1]);
+            if (i + 1 == RA) fragB(1, bh[1], bl[1]);
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[q], bh[s][b], acc[a][b], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[q], bl[s][b], acc[a][b], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[q], bh[s][b], acc[a][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // this part's steps
+    const int s0 = (int)((int64_t)p.steps * z / p.splits), s1 = (int)((int64_t)p.steps * (z + 1) / p.splits);
+    // One step: its stage has landed and every wave is past the buffer that the
+    // step STAGES - 1 ahead now goes to (past the end: the last step again, so
+    // that the count of loads in flight stays the same), then its products.
+    auto turn = [&](int s, u16* cA, u16* cB, u16* nA, u16* nB) __attribute__((always_inline)) {
+        // not __syncthreads(), which waits for every copy into LDS
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * (AI + BI)) : "memory");
+        issue(min(s + STAGES - 1, s1 - 1), nA, nB);
+        compute(cA, cB);
+    };
+    issue(s0, sA0, sB0);
+    if (STAGES == 3) issue(min(s0 + 1, s1 - 1), sA1, sB1);
+    int s = s0;
+    if constexpr (STAGES == 3) {
+        for (; s + 3 <= s1; s += 3) {
+            turn(s, sA0, sB0, sA2, sB2);
+            turn(s + 1, sA1, sB1, sA0, sB0);
+            turn(s + 2, sA2, sB2, sA1, sB1);
+        }
+        if (s < s1) turn(s, sA0, sB0, sA2, sB2);
+        if (s + 1 < s1) turn(s + 1, sA1, sB1, sA0, sB0);
+    } else {
+        for (; s + 2 <= s1; s += 2) {
+            turn(s, sA0, sB0, sA1, sB1);
+            turn(s + 1, sA1, sB1, sA0, sB0);
+        }
+        if (s < s1) turn(s, sA0, sB0, sA1, sB1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing is on its way into LDS when the workgroup ends
+
+    if (p.splits > 1) {
+        float* o = p.part + ((int64_t)z * p.tm * BM + m0 + wm * WM) * ((int64_t)p.tn * BN) + n0 + wn * WN + fr;
+#pragma unroll
+        for (int a = 0; a < RA; ++a)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int r = a * 32 + (i >> 2) * 8 + fh * 4 + (i & 3);
+#pragma unroll
+                for (int b = 0; b < RB; ++b) o[(int64_t)r * p.tn * BN + b * 32] = acc[a][b][i];
+            }
+        return;
+    }
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+        const int cl = wn * WN + b * 32 + fr, col = n0 + cl;
+        if (col >= p.N) continue;
+        const int ec = seb[cl];
+        const float bc = CONV ? 0.f : sbias[cl];
+        float* cp = place<CONV>(p, m0 + wm * WM + fh * 4, col);
+        const int64_t ld = CONV ? p.HWo : p.ldc;
+#pragma unroll
+        for (int a = 0; a < RA; ++a)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int rl = wm * WM + a * 32 + g * 8 + fh * 4;  // four rows from here
+                const int4 er = *(const int4*)(sea + rl);
+                f4 v = {__builtin_amdgcn_ldexpf(acc[a][b][g * 4], er.x + ec),
+                        __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 1], er.y + ec),
+                        __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 2], er.z + ec),
+                        __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 3], er.w + ec)};
+                float* q = cp + (a * 32 + g * 8) * ld;
+                const int left = p.M - m0 - rl;
+                if (!CONV && p.accumulate) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] += q[min(i, max(left - 1, 0)) * ld];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i < left) q[i * ld] = v[i] + (CONV ? sbias[rl + i] : bc);
+            }
+    }
+}
+
+// The sum of the parts of K, in their order, with the exponents, bias and C:
+// one column and four rows per thread (grid: columns / 256, rows / 4).
+template <bool CONV>
+__global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) {
+    const int col = blockIdx.x * 256 + threadIdx.x, row0 = blockIdx.y * 4;
+    if (col >= p.N) return;
+    // the tile's number as k_split_mm counts it
+    const int mt = row0 / BM, nt = col / BN, grp = mt / 8, gm = min(8, p.tm - grp * 8);
+    if (p.slow[grp * 8 * p.tn + nt * gm + mt % 8]) return;
+    const int64_t ld = (int64_t)p.tn * BN, plane = (int64_t)p.tm * BM * ld;
+    const float* s = p.part + row0 * ld + col;  // whole tiles: rows past the matrix are there
+    float v[4] = {s[0], s[ld], s[2 * ld], s[3 * ld]};
+#pragma unroll 4
+    for (int z = 1; z < p.splits; ++z)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += s[z * plane + i * ld];
+    const int ec = p.eb[CONV ? col / p.HWo : col];
+    float* q = place<CONV>(p, row0, col);
+    const int64_t ldo = CONV ? p.HWo : p.ldc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (row0 + i < p.M) store<CONV>(p, row0 + i, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], p.ea[row0 + i] + ec));
+}
+
+size_t up(size_t n) { return (n + 255) / 256 * 256; }
+
+// The tiles of k_split_mm, with what a launch of it costs on MI355X. A CU holds
+// `cu` workgroups of a tile; a round of workgroups takes `full` us per step with
+// every CU full, `idle` us with few workgroups, and `once` us to start and to
+// store; parts of K add a launch and the traffic of their sums. The constants are
+// a fit (6 % rms) to 270 timings of 33 shapes, M and N from 64 to 262144 and 3 to
+// 720 steps, under every tile and 1 to 8 parts: over these shapes the tile and
+// the parts with the lowest estimate were the fastest measured, or within 4 % of
+// it in 30 and 13 % in all. Measured at the ends of the range, best tile in
+// front: [4096,320] x [320,320] 14.6 us with 64 x 64, 20.0 with 128 x 128;
+// conv [1,256,256,256] to 256 channels 226 us with 256 x 256, 246 with 128 x 256,
+// 273 with 128 x 128; conv [2,2560,8,8] to 1280 channels 119 us with 64 x 64 in
+// 8 parts, 307 in one.
+struct Tile {
+    int bm, bn, cu;
+    float full, idle, once;
+};
+constexpr Tile kTiles[] = {
+    {256, 256, 1, 1.52f, 1.52f, 5.6f}, {128, 256, 1, 0.90f, 0.90f, 5.3f}, {128, 128, 2, 0.88f, 0.58f, 3.5f},
+    {64, 64, 3, 0.52f, 0.27f, 2.3f}};
+constexpr int kParts[] = {1, 2, 3, 4, 6, 8, 12, 16};
+
+struct Plan {
+    int tile;
+    int tm, tn, splits;
+    int bm() const { return kTiles[tile].bm; }
+    int bn() const { return kTiles[tile].bn; }
+    size_t part_bytes() const { return splits > 1 ? up((size_t)splits * tm * tn * bm() * bn() * 4) : 0; }
+};
+Plan plan_of(int64_t M, int64_t N, int64_t steps) {
+    Plan best{};
+    double least = 0;
+    for (int i = 0; i < 4; ++i) {
+        const Tile& t = kTiles[i];
+        const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn, slots = (int64_t)num_cus() * t.cu;
+        for (const int parts : kParts) {
+            // a part has at least four steps; parts only where one round of workgroups is not full
+            if (parts > 1 && (steps < 4 * parts || tm * tn >= slots)) break;
+            const int64_t n = tm * tn * parts, rest = n % slots;
+            const double k = (double)steps / parts;
+            double us = (double)(n / slots) * (k * t.full + t.once);
+            if (rest) us += k * (t.idle + (t.full - t.idle) * rest / slots) + t.once;
+            if (parts > 1) us += 3.0 + (double)(parts + 1) * tm * t.bm * tn * t.bn * 4 / 4.4e6;
+            if (least == 0 || us < least) {
+                least = us;
+                best = Plan{i, (int)tm, (int)tn, parts};
+            }
+        }
+    }
+    return best;
+}
+
+template <bool CONV>
+void launch_mm(const Plan& q, SplitArgs& p) {
+    const unsigned grid = (unsigned)(q.tm * q.tn * q.splits);
+    if (q.tile == 0)
+        k_split_mm<256, 256, 128, 64, 2, CONV><<<grid, 512, 0, stream()>>>(p);
+    else if (q.tile == 1)
+        k_split_mm<128, 256, 64, 64, 3, CONV><<<grid, 512, 0, stream()>>>(p);
+    else if (q.tile == 2)
+        k_split_mm<128, 128, 64, 64, 2, CONV><<<grid, 256, 0, stream()>>>(p);
+    else
+        k_split_mm<64, 64, 32, 32, 3, CONV><<<grid, 256, 0, stream()>>>(p);
+    if (q.splits > 1)
+        k_split_sum<CONV><<<dim3((unsigned)((p.N + 255) / 256), (unsigned)((p.M + 3) / 4)), 256, 0, stream()>>>(
+            p, q.bm(), q.bn());
+}
+
+constexpr size_t kRowLds = 48 << 10;  // weights of one output channel that k_conv_prep takes through LDS
+constexpr int64_t kMost = int64_t(1) << 31;
+
+}  // namespace
+
+// C = A B^T (+ C) (+ bias), all fp32, on the split operands. Checked arguments.
+// False where the general path has to take it (scratch, or sizes past 32-bit
+// offsets or one launch's grid).
+bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                int64_t ldc, const float* bias, bool accumulate) {
+    const int64_t steps = (K + kStep - 1) / kStep;
+    if (M * kRowBytes >= kMost || N * kRowBytes >= kMost || K >= kMost) return false;
+    const Plan q = plan_of(M, N, steps);
+    if ((int64_t)q.tm * q.tn * q.splits * 512 >= kMost) return false;
+    const size_t pa = up((size_t)steps * M * kRowBytes), pb = up((size_t)steps * N * kRowBytes);
+    const size_t ea = up((size_t)M * 4), eb = up((size_t)N * 4), sl = up((size_t)q.tm * q.tn * 4);
+    char* s = (char*)try_scratch(pa + pb + ea + eb + sl + q.part_bytes());
+    if (!s) return false;
+    SplitArgs p{};
+    PackRows ra{A, lda, (u16*)s, (int*)(s + pa + pb), (int)M, (int)K};
+    PackRows rb{B, ldb, (u16*)(s + pa), (int*)(s + pa + pb + ea), (int)N, (int)K};
+    const unsigned ba = blocks_for(M, 4), bb = blocks_for(N, 4);
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && aligned16(A) && aligned16(B);
+    const int turns = !vec || K > 4096 ? 0 : K > 2048 ? 8 : K > 1024 ? 4 : K > 512 ? 2 : 1;
+    auto pack = turns == 8 ? k_split_pack<8> : turns == 4 ? k_split_pack<4> : turns == 2 ? k_split_pack<2>
+                                           : turns == 1   ? k_split_pack<1>
+                                                          : k_split_pack<0>;
+    pack<<<ba + bb, 256, 0, stream()>>>(ra, rb, (int)ba);
+    p.A = ra.P;
+    p.B = rb.P;
+    p.planeA = M * kRowBytes;
+    p.planeB = N * kRowBytes;
+    p.ea = ra.exps;
+    p.eb = rb.exps;
+    p.C = C;
+    p.ldc = ldc;
+    p.bias = bias;
+    p.M = (int)M;
+    p.N = (int)N;
+    p.K = (int)K;
+    p.steps = (int)steps;
+    p.accumulate = accumulate ? 1 : 0;
+    p.tm = q.tm;
+    p.tn = q.tn;
+    p.splits = q.splits;
+    p.slow = (unsigned*)(s + pa + pb + ea + eb);
+    p.part = (float*)(s + pa + pb + ea + eb + sl);
+    p.A0 = A;
+    p.B0 = B;
+    p.lda = lda;
+    p.ldb = ldb;
+    launch_mm<false>(q, p);
+    return true;
+}
+
+// conv2d of checked arguments; false as above.
+bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, const float* w, int64_t Cout, int64_t kh,
+                int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo) {
+    const int64_t HW = H * W, HWo = Ho * Wo, taps = kh * kw, chunks = (Cin + kStep - 1) / kStep, steps = chunks * taps;
+    const int64_t cols = N * HWo, prows = N * HW + 1;
+    // 32-bit offsets, also of a padded tile's first pixel
+    if ((N * HW + (int64_t)pad * (W + 1) + 1) * kRowBytes >= kMost || cols >= kMost - 256 || Cout * kRowBytes >= kMost ||
+        steps >= kMost || Cin * taps >= kMost || N > 65535 || N * Cin * HW >= kMost * 64)
+        return false;
+    const Plan q = plan_of(Cout, cols, steps);
+    if ((int64_t)q.tm * q.tn * q.splits * 512 >= kMost) return false;
+    ConvPack a{};
+    a.ncb = (int)((Cin + kChanBlock - 1) / kChanBlock);
+    a.npb = (int)((HW + kPixBlock - 1) / kPixBlock);
+    const size_t px = up((size_t)chunks * prows * kRowBytes), pw = up((size_t)steps * Cout * kRowBytes);
+    const size_t mx = up((size_t)N * a.ncb * a.npb * 4), bd = up((size_t)N * a.npb * 4);
+    const size_t ex = up((size_t)N * 4), ew = up((size_t)Cout * 4), sl = up((size_t)q.tm * q.tn * 4);
+    char* s = (char*)try_scratch(px + pw + mx + bd + ex + ew + sl + q.part_bytes());
+    if (!s) return false;
+    a.x = x;
+    a.w = w;
+    a.X = (u16*)s;
+    a.Wp = (u16*)(s += px);
+    a.maxima = (unsigned*)(s += pw);
+    a.bad = (unsigned*)(s += mx);
+    a.ex = (int*)(s += bd);
+    a.ew = (int*)(s += ex);
+    a.N = (int)N;
+    a.Cin = (int)Cin;
+    a.HW = (int)HW;
+    a.Cout = (int)Cout;
+    a.taps = (int)taps;
+    a.chunks = (int)chunks;
+    const int nmax = (int)(N * a.ncb * a.npb), pt = (int)((HW + 63) / 64);
+    // all channels of a pixel tile in one workgroup where that leaves at least four workgroups per CU
+    const int64_t groups = std::min<int64_t>(chunks, std::max<int64_t>(1, (4 * num_cus() + pt * N - 1) / (pt * N)));
+    a.per = (int)((chunks + groups - 1) / groups);
+    const size_t row = (size_t)(Cin * taps) * 4;
+    const bool in_lds = row <= kRowLds;
+    k_conv_prep<<<(unsigned)(nmax + Cout), 256, in_lds ? row : 0, stream()>>>(a, nmax, in_lds ? 1 : 0);
+    k_conv_pack<<<dim3((unsigned)pt, (unsigned)((chunks + a.per - 1) / a.per), (unsigned)N), 256, 0, stream()>>>(a);
+    SplitArgs p{};
+    p.A = a.Wp;
+    p.B = a.X;
+    p.planeA = Cout * kRowBytes;
+    p.planeB = prows * kRowBytes;
+    p.ea = a.ew;
+    p.eb = a.ex;
+    p.C = out;
+    p.bias = bias;
+    p.M = (int)Cout;
+    p.N = (int)cols;
+    p.K = (int)(Cin * taps);
+    p.steps = (int)steps;
+    p.tm = q.tm;
+    p.tn = q.tn;
+    p.splits = q.splits;
+    p.slow = (unsigned*)(s += ew);
+    p.part = (float*)(s + sl);
+    p.A0 = w;
+    p.B0 = x;
+    p.bad = a.bad;
+    p.H = (int)H;
+    p.W = (int)W;
+    p.Wo = (int)Wo;
+    p.HWo = (int)HWo;
+    p.kh = (int)kh;
+    p.kw = (int)kw;
+    p.stride = stride;
+    p.pad = pad;
+    p.taps = (int)taps;
+    p.Cin = (int)Cin;
+    p.Cout = (int)Cout;
+    p.npb = a.npb;
+    p.zero = (int)(prows - 1);
+    launch_mm<true>(q, p);
+    return true;
+}
+
+}  // namespace sdh

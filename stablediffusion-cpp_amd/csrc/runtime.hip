@@ -165,6 +165,11 @@ struct Runtime {
     std::map<uintptr_t, size_t> external;
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
+    // Scratch blocks that grew out of use while captured graphs were alive: a
+    // graph keeps the pointers it was captured with, so they are given back
+    // only when the last graph is destroyed.
+    std::vector<void*> retired_scratch;
+    int live_graphs = 0;
     unsigned* counters = nullptr;
     size_t counter_count = 0;
     void* workspace = nullptr;
@@ -374,23 +379,53 @@ void check_range(const void* p, size_t bytes, const char* op, const char* what) 
     range_check_locked(r, p, bytes, op, what);
 }
 
+namespace {
+
+// Returns the scratch block to an exhausted arena (the next op that needs
+// scratch asks for it again); false where there is none or a graph holds it.
+bool give_back_scratch_locked(Runtime& r) {
+    if (!r.scratch || r.capturing || r.live_graphs > 0) return false;
+    hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
+    r.arena.release(r.scratch);
+    r.scratch = nullptr;
+    r.scratch_bytes = 0;
+    return true;
+}
+
+// Replaces the scratch block by one of at least `bytes`; false when the arena
+// cannot hold it (there is then no scratch block).
+bool grow_scratch_locked(Runtime& r, size_t bytes) {
+    if (r.scratch) {
+        if (r.live_graphs > 0) {
+            r.retired_scratch.push_back(r.scratch);
+        } else {
+            // Work queued earlier may still read the old scratch.
+            hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
+            r.arena.release(r.scratch);
+        }
+    }
+    r.scratch_bytes = round_up(std::max(bytes, (size_t)1 << 20), kAlign);
+    r.scratch = r.arena.alloc(r.scratch_bytes);
+    if (!r.scratch) r.scratch_bytes = 0;
+    return r.scratch != nullptr;
+}
+
+}  // namespace
+
 void* scratch(size_t bytes) {
     Runtime& r = rt();
     std::lock_guard<std::mutex> lk(r.mu);
     if (bytes > r.scratch_bytes) {
         not_capturing_locked(r, "backend_hip scratch");
-        if (r.scratch) {
-            // Work queued earlier may still read the old scratch.
-            hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
-            r.arena.release(r.scratch);
-        }
-        r.scratch_bytes = round_up(std::max(bytes, (size_t)1 << 20), kAlign);
-        r.scratch = r.arena.alloc(r.scratch_bytes);
-        if (!r.scratch) {
-            r.scratch_bytes = 0;
-            fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating scratch");
-        }
+        if (!grow_scratch_locked(r, bytes)) fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating scratch");
     }
+    return r.scratch;
+}
+
+void* try_scratch(size_t bytes) {
+    Runtime& r = rt();
+    std::lock_guard<std::mutex> lk(r.mu);
+    if (bytes > r.scratch_bytes && (r.capturing || !grow_scratch_locked(r, bytes))) return nullptr;
     return r.scratch;
 }
 
@@ -405,6 +440,7 @@ void* workspace(size_t bytes) {
         }
         r.workspace_bytes = round_up(bytes, kAlign);
         r.workspace = r.arena.alloc(r.workspace_bytes);
+        if (!r.workspace && give_back_scratch_locked(r)) r.workspace = r.arena.alloc(r.workspace_bytes);
         if (!r.workspace) {
             r.workspace_bytes = 0;
             fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating the GEMM workspace");
@@ -531,6 +567,7 @@ int sdh_shutdown(void) {
         r.external.clear();
         r.scratch = nullptr;
         r.scratch_bytes = 0;
+        r.retired_scratch.clear();
         r.counters = nullptr;
         r.counter_count = 0;
         r.ones = nullptr;
@@ -559,6 +596,7 @@ int sdh_malloc(size_t bytes, void** out) {
         Runtime& r = rt();
         std::lock_guard<std::mutex> lk(r.mu);
         void* p = r.arena.alloc(bytes);
+        if (!p && give_back_scratch_locked(r)) p = r.arena.alloc(bytes);
         if (!p)
             fail(SDH_ERR_OOM, "sdh_malloc: arena exhausted (" + std::to_string(bytes) + " bytes requested, " +
                                   std::to_string(r.arena.in_use) + " in use, " + std::to_string(r.arena.reserved) +
@@ -743,6 +781,7 @@ int sdh_capture_end(void** graph) {
         const hipError_t ie = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         hip_check(ie, "hipGraphInstantiate");
+        ++r.live_graphs;
         *graph = (void*)e;
     });
 }
@@ -767,6 +806,10 @@ int sdh_graph_destroy(void* graph) {
         // a launch of it may still be queued
         hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
         hip_check(hipGraphExecDestroy((hipGraphExec_t)graph), "hipGraphExecDestroy");
+        if (--r.live_graphs == 0) {
+            for (void* p : r.retired_scratch) r.arena.release(p);
+            r.retired_scratch.clear();
+        }
     });
 }
 

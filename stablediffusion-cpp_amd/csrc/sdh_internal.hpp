@@ -77,6 +77,9 @@ void check_range(const void* p, size_t bytes, const char* op, const char* what);
 // Per-call device scratch of at least `bytes`, owned by the library, valid
 // until the next call that asks for scratch (ops are serialised on one stream).
 void* scratch(size_t bytes);
+// As scratch, but null instead of an error where the arena cannot hold that
+// much, or where the block would have to grow during a capture.
+void* try_scratch(size_t bytes);
 // A persistent library-owned device block of at least `bytes` for a library
 // routine's workspace (the BLAS GEMM), distinct from scratch().
 void* workspace(size_t bytes);
@@ -85,6 +88,12 @@ void* workspace(size_t bytes);
 // (k_gemm.hip). False when hipBLASLt has no algorithm for the shape.
 bool blaslt_gemm(bool f32, int64_t M, int64_t N, int64_t K, const void* P, int64_t ldp, const void* B, int64_t ldb,
                  float* C, int64_t ldc, const float* bias, bool accumulate);
+// The fp32 product and conv2d on split fp16 operands (k_gemm_split.hip), with
+// checked arguments; false where the caller's general path has to run.
+bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                int64_t ldc, const float* bias, bool accumulate);
+bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, const float* w, int64_t Cout, int64_t kh,
+                int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo);
 // y = silu(gate) * up over n floats (the SwiGLU kernel of sdh_swiglu, no checks).
 void launch_swiglu(const float* gate, const float* up, float* y, int64_t n);
 // sdh_softmax_rows on [rows, cols] (k_softmax.hip), errors named after `op`.

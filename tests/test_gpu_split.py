@@ -1,0 +1,214 @@
+"""GPU tests of the fp32 products on split fp16 operands (k_gemm_split.hip):
+sdh_gemm_nt_f32 at sizes that it takes, and sdh_conv2d, against the float64
+oracle within the rigorous fp32 summation bound, element by element: at the
+edges of every tile, K remainders, parts of K, padding and strides; rows of
+extreme scale; infinities and NaN (what fp32 gives); a run of pixels far
+below the sample's largest value; a captured graph replayed after the scratch
+block it uses has been outgrown; and an arena too small for the scratch."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from tolerances import assert_gemm
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+def run_gemm(be, orc, M, N, K, seed, lda=None, bias=True, acc=False, edit=None):
+    lda = lda or K
+    A = orc.randn((M, lda), seed)
+    W = orc.randn((N, K), seed + 1, 0.0, 1.0 / np.sqrt(K))
+    if edit:
+        edit(A, W)
+    b = orc.randn((N,), seed + 2) if bias else None
+    c0 = orc.randn((M, N), seed + 3) if acc else None
+    dC = be.array(c0) if acc else be.empty((M, N))
+    be.gemm_nt_f32(M, N, K, be.array(A), lda, be.array(W), K, dC, N, be.array(b) if bias else None, acc)
+    return dC.download(), A[:, :K], W, b, c0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,lda,bias,acc", [
+    (257, 300, 321, None, True, False),      # odd K and ld, 64 x 64 tiles
+    (65, 63, 65, 70, False, True),           # one past a tile, one short, one past a step
+    (16, 16, 64, None, True, True),          # the smallest that an unaligned call sends here
+    (1024, 1032, 1000, 1004, True, True),    # 64 x 64 or 128 x 128, K not a multiple of 32
+    (130, 4100, 2052, None, True, False),    # few rows
+    (700, 260, 8192, None, False, False),    # parts of K
+    (4097, 2049, 128, None, True, False),    # 128 x 128, one past the tiles (unaligned C rows)
+    (3000, 5000, 160, None, True, True),     # 256 x 256 with remainders
+])
+def test_gemm(be, orc, M, N, K, lda, bias, acc):
+    got, A, W, b, c0 = run_gemm(be, orc, M, N, K, 4000 + M + K, lda, bias, acc)
+    want, S = orc.gemm_nt_f32(A, W, b, c0, acc)
+    assert_gemm(got, want, S, K + 2, f"split gemm {M}x{N}x{K}")
+
+
+@pytest.mark.gpu
+def test_gemm_rows_of_any_scale(be, orc):
+    """Each row has its own exponent: 2^+-120, subnormal rows, a zero row, and
+    rows whose values span 2^16 (the range that keeps every bit)."""
+    def edit(A, W):
+        A[::7] *= np.float32(2.0 ** 100)
+        A[1::7] *= np.float32(2.0 ** -100)
+        A[2] = np.float32(2.0 ** -140) * np.rint(A[2] * 100)  # subnormal, exact
+        A[3] = 0
+        A[4] *= np.float32(2.0) ** np.linspace(0, 16, A.shape[1]).astype(np.float32)
+        W[5] *= np.float32(2.0 ** 20)
+        W[6] *= np.float32(2.0 ** -20)
+
+    got, A, W, b, _ = run_gemm(be, orc, 300, 333, 340, 4500, bias=False, edit=edit)
+    want, S = orc.gemm_nt_f32(A, W, None, None, False)
+    assert_gemm(got, want, S + 2.0 ** -126, 342, "rows of any scale")  # results below 2^-126 round to its grid
+
+
+@pytest.mark.gpu
+def test_gemm_infinities_and_nan(be, orc):
+    """Rows that hold them give what fp32 gives; all others are untouched."""
+    def edit(A, W):
+        A[10, 3], A[11, 5], A[12, 7], A[12, 9] = np.inf, np.nan, np.inf, -np.inf
+        W[200, 3] = -np.inf
+        W[201] = 0
+        W[:, 5][::2] = 0
+
+    got, A, W, b, _ = run_gemm(be, orc, 300, 333, 340, 4600, edit=edit)
+    with np.errstate(invalid="ignore"):
+        want = A.astype(np.float64) @ W.astype(np.float64).T + b
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    fine = np.isfinite(want)
+    with np.errstate(invalid="ignore"):
+        S = np.abs(A.astype(np.float64)) @ np.abs(W.astype(np.float64)).T + np.abs(b)
+    assert np.array_equal(np.isfinite(got), fine)
+    assert_gemm(got[fine], want[fine], S[fine], 342, "beside rows that are not finite")
+
+
+CONVS = [  # N, Cin, H, W, Cout, kh, kw, stride, pad
+    (1, 1, 1, 1, 1, 1, 1, 1, 0), (3, 33, 17, 19, 65, 3, 3, 1, 1), (2, 64, 16, 16, 64, 3, 3, 1, 1),
+    (1, 31, 12, 40, 129, 5, 3, 1, 2), (2, 70, 21, 23, 66, 3, 3, 2, 1), (1, 96, 9, 31, 40, 1, 3, 3, 2),
+    (2, 40, 5, 5, 20, 3, 3, 1, 4),      # pixels that see padding only
+    (1, 320, 33, 31, 100, 1, 1, 1, 0), (2, 260, 8, 8, 300, 3, 3, 1, 1),  # parts of K
+    (1, 36, 300, 260, 257, 3, 3, 1, 1),  # 256 x 256 tiles over rows and runs of 256 pixels
+    (1, 70, 200, 140, 128, 3, 3, 1, 1),  # 128 x 256
+    (2, 4, 66, 62, 3, 3, 3, 1, 1),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Cin,H,W,Cout,kh,kw,stride,pad", CONVS)
+def test_conv(be, orc, N, Cin, H, W, Cout, kh, kw, stride, pad):
+    x = orc.randn((N, Cin, H, W), 4700 + Cin + H) * np.exp2(np.arange(N, dtype=np.float32) * 9)[:, None, None, None]
+    w = orc.randn((Cout, Cin, kh, kw), 4701 + Cout, 0.0, 1.0 / np.sqrt(Cin * kh * kw))
+    b = orc.randn((Cout,), 4702)
+    Ho, Wo = (H + 2 * pad - kh) // stride + 1, (W + 2 * pad - kw) // stride + 1
+    out = be.empty((N, Cout, Ho, Wo))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, kh, kw, be.array(b), stride, pad, out, Ho, Wo)
+    want, S = orc.conv2d(x, w, b, stride, pad)
+    assert_gemm(out.download(), want, S, Cin * kh * kw + 2, f"conv2d {x.shape} k{kh}x{kw} s{stride} p{pad}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("special", [None, np.inf, np.nan])
+def test_conv_far_pixels_and_specials(be, orc, special):
+    """One value of 2^20 (or an infinity, or NaN) in a corner of an image whose
+    far half lies at 2^-10: every output still within the fp32 bound of its own
+    terms, and what sees the special value as fp32 has it."""
+    N, Cin, H, W, Cout = 2, 40, 48, 50, 70
+    x = orc.randn((N, Cin, H, W), 4800)
+    x[:, :, H // 2:] *= np.float32(2.0 ** -10)
+    x[1, 7, 2, 3] = 2.0 ** 20 if special is None else special
+    w = orc.randn((Cout, Cin, 3, 3), 4801, 0.0, 0.05)
+    b = np.zeros(Cout, np.float32)
+    out = be.empty((N, Cout, H, W))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, 3, 3, be.array(b), 1, 1, out, H, W)
+    got = out.download()
+    with np.errstate(invalid="ignore"):
+        want, S = orc.conv2d(x, w, b, 1, 1)
+    fine = np.isfinite(want)
+    assert fine.sum() == want.size - (0 if special is None else 9 * Cout)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    assert_gemm(got[fine], want[fine], S[fine], Cin * 9 + 2, f"conv2d beside {special}")
+
+
+@pytest.mark.gpu
+def test_graph_keeps_its_scratch(be, orc):
+    """A graph holds the scratch block of its capture: the block lives on when
+    a larger one replaces it, and replays over new inputs stay right."""
+    M, N, K = 1000, 1100, 1008
+    W = orc.randn((N, K), 4901, 0.0, 1.0 / np.sqrt(K))
+    dA, dW, dC = be.empty((M, K)), be.array(W), be.empty((M, N))
+    be.gemm_nt_f32(M, N, K, dA.upload(orc.randn((M, K), 4900)), K, dW, K, dC, N)
+    be.capture_begin()
+    be.gemm_nt_f32(M, N, K, dA, K, dW, K, dC, N)
+    graph = be.capture_end()
+    try:
+        x = be.randn((1, 64, 512, 512), 4902)
+        y = be.empty((1, 64, 512, 512))
+        w = be.randn((64, 64, 3, 3), 4903)
+        for i in range(3):
+            A = orc.randn((M, K), 4910 + i)
+            dA.upload(A)
+            be.conv2d(x, 1, 64, 512, 512, w, 64, 3, 3, None, 1, 1, y, 512, 512)
+            be.graph_launch(graph)
+            be.conv2d(x, 1, 64, 512, 512, w, 64, 3, 3, None, 1, 1, y, 512, 512)
+            want, S = orc.gemm_nt_f32(A, W, None, None, False)
+            assert_gemm(dC.download(), want, S, K, f"replay {i}")
+    finally:
+        be.graph_destroy(graph)
+
+
+BODY = r"""
+import sys
+sys.path[:0] = [%r, %r, %r]
+import numpy as np, sdhip
+from oracle import Oracle
+from tolerances import assert_gemm
+MB = 1 << 20
+be, orc = sdhip.Backend(), Oracle()
+x = orc.randn((1, 64, 96, 96), 1); w = orc.randn((80, 64, 3, 3), 2, 0.0, 0.05); b = orc.randn((80,), 3)
+A = orc.randn((2000, 1024), 4); W = orc.randn((600, 1024), 5, 0.0, 0.03)
+dx, dw, db, dy = be.array(x), be.array(w), be.array(b), be.empty((1, 80, 96, 96))
+dA, dW, dC = be.array(A), be.array(W), be.empty((2000, 600))
+want, S = orc.conv2d(x, w, b, 1, 1)
+wg, Sg = orc.gemm_nt_f32(A, W, None, None, False)
+be.gemm_nt_f32(2000, 600, 1024, dA, 1024, dW, 1024, dC, 600)
+assert_gemm(dC.download(), wg, Sg, 1026, 'gemm')
+# what is left of the arena falls in turn below every size that the calls ask for
+hold = []
+for left in (0, 1, 2, 4, 8, 16):
+    try:
+        while True:
+            hold.append(be.malloc(MB))
+    except sdhip.SdhError as e:
+        assert e.status == sdhip.SDH_ERR_OOM, e
+    for _ in range(left):
+        be.free(hold.pop())
+    for f, n in ((lambda: be.conv2d(dx, 1, 64, 96, 96, dw, 80, 3, 3, db, 1, 1, dy, 96, 96), 'conv'),
+                 (lambda: be.gemm_nt_f32(2000, 600, 1024, dA, 1024, dW, 1024, dC, 600), 'gemm')):
+        be.call('sdh_zero', dy.ptr, dy.nbytes); be.call('sdh_zero', dC.ptr, dC.nbytes)
+        try:
+            f()
+            if n == 'conv': assert_gemm(dy.download(), want, S, 578, 'conv with %%d MB left' %% left)
+            else: assert_gemm(dC.download(), wg, Sg, 1026, 'gemm with %%d MB left' %% left)
+            print(n, left, 'MB left: right', flush=True)
+        except sdhip.SdhError as e:
+            assert e.status == sdhip.SDH_ERR_OOM, e
+            print(n, left, 'MB left: reported', flush=True)
+for p in hold: be.free(p)
+be.conv2d(dx, 1, 64, 96, 96, dw, 80, 3, 3, db, 1, 1, dy, 96, 96)
+assert_gemm(dy.download(), want, S, 578, 'conv at the end')
+print('small arena ok', flush=True)
+""" % (os.path.join(ROOT, "stablediffusion-cpp_amd"), os.path.join(ROOT, "oracle"), HERE)
+
+
+@pytest.mark.gpu
+def test_small_arena():
+    r = subprocess.run([sys.executable, "-u", "-c", BODY], capture_output=True, text=True, timeout=110,
+                       env=dict(os.environ, SDH_ARENA_MB="160", SDH_ARENA_LIMIT_MB="160"))
+    print(r.stdout, r.stderr[-3000:])
+    assert r.returncode == 0 and "small arena ok" in r.stdout
