@@ -53,7 +53,8 @@
 // running max a weight is taken against is raised only when a tile's max
 // passes it by 2^1.5 (weights stay below 2^15.5), so O is rescaled on few
 // tiles, and then by exactly the factor between the old and new reference.
-// Head dimensions above 128 take a plain fp32 kernel (one wave per query).
+// Head dimensions above 128 take the score matrix on split operands
+// (k_gemm_split.hip), or with few keys a plain fp32 kernel (one wave per query).
 // Both kernels can store the output rounded to bf16 (sdh_attention_bf16):
 // the operand rounding of the projection that follows (to_out), applied to
 // the same fp32 values, so the next GEMM reads half the bytes and no
@@ -816,16 +817,15 @@ void run_mfma(const float* q, const float* k, const float* v, void* out, int64_t
     launched("sdh_attention");
 }
 
-// Head dimensions above 128 on long sequences (the VAE's one-head attention
-// over 512 channels, modules.cpp:133-141): the score matrix, as the
-// reference's device path forms it (backend_cuda.cu:550-586), on the fp32
-// library GEMM: per (batch, head) and block of query rows, S = q_h k_g^T,
-// the scaled (causal) row softmax in place, then O_h = P v_g as a GEMM
-// against v^T (v transposed once per batch). fp32 products and sums
-// throughout. The score block is bounded to score_bytes() (causal: one block,
-// so the mask's row index is the query's). False, with nothing queued, when
-// the operands do not suit the library GEMM (alignment, Skv % 4) or the
-// causal block would not fit: the caller then runs the one-wave kernel.
+// Head dimensions above 128 where split_attention's scratch does not fit (the
+// packed operands of q, k, v and of the weights come on top of the scores): the
+// score matrix on the fp32 library GEMM, in less scratch: per (batch, head) and
+// block of query rows, S = q_h k_g^T, the scaled (causal) row softmax in place,
+// then O_h = P v_g as a GEMM against v^T (v transposed once per batch). fp32
+// products and sums throughout. The score block is bounded to score_bytes()
+// (causal: one block, so the mask's row index is the query's). False, with
+// nothing queued, when the operands do not suit the library GEMM (alignment,
+// Skv % 4) or the causal block would not fit: the caller then runs the one-wave kernel.
 // The score block's budget: SD_CUDA_ATTN_MB megabytes, at least 64, 1024 when
 // unset, as the reference caps its score buffer (backend_cuda.cu:558-561).
 int64_t score_bytes() {
@@ -922,6 +922,15 @@ void run_attention(const float* q, const float* k, const float* v, void* out, bo
             if (fp16) out16 ? go(D128(), T_(), F_()) : go(D128(), F_(), F_());
             else out16 ? go(D128(), T_(), T_()) : go(D128(), F_(), T_());
         }
+    } else if (Skv > 64 && split_attention(q, k, v, out, out16, N, Sq, Skv, heads, kv_heads, d, causal, scale,
+                                           score_bytes())) {
+        // The score matrix on split operands, from more than one 64-key tile of
+        // the one-wave kernel on (MI355X, us, that kernel in front, or (*) the fp32
+        // library GEMMs that took long sequences of aligned rows): [2,64,8x160]
+        // 16 / 24, [2,256,8x160] to 77 keys 41 / 28, [2,256,8x160] 138 / 35, [1,450,512]
+        // 244 / 33, [1,2745,512] 2997 / 108, [1,4096,512] 329* / 151, [1,16384,512]
+        // 4124* / 1875 (293 TFLOP/s).
+        launched(op);
     } else if (!(Sq * Skv >= (int64_t(1) << 18) &&
                  run_attention_gemm(op, q, k, v, out, out16, N, Sq, Skv, heads, kv_heads, d, causal, scale))) {
         const int64_t gx = (Sq + kGenWaves - 1) / kGenWaves;

@@ -90,6 +90,9 @@ struct PackRows {
     u16* P;
     int* exps;
     int rows, K;
+    // further matrices of the same sizes: matrix i starts at X + (i / inner) outer_ld + (i % inner) inner_ld
+    int inner;
+    int64_t outer_ld, inner_ld;
 };
 
 __device__ __forceinline__ unsigned umax4(const f4& v) {
@@ -102,59 +105,76 @@ __device__ __forceinline__ void store_split(u16* o, const float* v, int s) {
     *(h8*)(o + kStep) = lo;
 }
 
-// TURNS > 0: float4 loads (K, ld and X aligned for them) of a row of at most
-// 512 TURNS values, all in flight at once and kept in registers. TURNS = 0:
-// any row, read twice.
-template <int TURNS>
-__device__ __forceinline__ void pack_row(const PackRows& a, int row, int lane) {
-    const float* x = a.X + (int64_t)row * a.ld;
+// A row of LANES threads' values to steps. TURNS > 0: float4 loads (K, ld and X
+// aligned for them) of at most 8 LANES TURNS values, all in flight at once and
+// kept in registers. TURNS = 0: any row, read twice.
+template <int LANES, int TURNS>
+__device__ __forceinline__ void pack_row(const PackRows& a, const float* x, u16* P, int* exps, int row, int lane,
+                                         unsigned* red) {
     const int kp = (a.K + kStep - 1) / kStep * kStep;
     auto out = [&](int k) __attribute__((always_inline)) {
-        return a.P + ((int64_t)(k / kStep) * a.rows + row) * (kRowBytes / 2) + (k % kStep);
+        return P + ((int64_t)(k / kStep) * a.rows + row) * (kRowBytes / 2) + (k % kStep);
+    };
+    auto exponent = [&](unsigned m) __attribute__((always_inline)) {
+        m = wave_umax(m);
+        if constexpr (LANES > 64) {
+            if ((lane & 63) == 0) red[lane >> 6] = m;
+            __syncthreads();
+            m = max(max(red[0], red[1]), max(red[2], red[3]));
+        }
+        const int e = exp_of(m);
+        if (lane == 0) exps[row] = e;
+        return e == kBad ? 0 : -e;
     };
     unsigned m = 0;
     if constexpr (TURNS > 0) {
         f4 v[TURNS][2];
 #pragma unroll
         for (int j = 0; j < TURNS; ++j) {  // past the row: its last four values, dropped below
-            const int k = (j * 64 + lane) * 8;
+            const int k = (j * LANES + lane) * 8;
             v[j][0] = *(const f4*)(x + min(k, a.K - 4));
             v[j][1] = *(const f4*)(x + min(k + 4, a.K - 4));
         }
 #pragma unroll
         for (int j = 0; j < TURNS; ++j) m = max(m, max(umax4(v[j][0]), umax4(v[j][1])));
-        const int e = exp_of(wave_umax(m));
-        if (lane == 0) a.exps[row] = e;
+        const int e = exponent(m);
 #pragma unroll
         for (int j = 0; j < TURNS; ++j) {
-            const int k = (j * 64 + lane) * 8;
+            const int k = (j * LANES + lane) * 8;
             if (k >= kp) continue;
             float f[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) f[i] = k + i < a.K ? v[j][i / 4][i % 4] : 0.f;
-            store_split(out(k), f, e == kBad ? 0 : -e);
+            store_split(out(k), f, e);
         }
     } else {
-        for (int k = lane; k < a.K; k += 64) m = max(m, absbits(x[k]));
-        const int e = exp_of(wave_umax(m));
-        if (lane == 0) a.exps[row] = e;
-        for (int k = lane * 8; k < kp; k += 512) {
+#pragma unroll 4
+        for (int k = lane; k < a.K; k += LANES) m = max(m, absbits(x[k]));
+        const int e = exponent(m);
+        for (int k = lane * 8; k < kp; k += LANES * 8) {
             float f[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) f[i] = k + i < a.K ? x[k + i] : 0.f;
-            store_split(out(k), f, e == kBad ? 0 : -e);
+            store_split(out(k), f, e);
         }
     }
 }
 
-// Both operands in one launch: the first ba workgroups take A's rows, the rest B's.
-template <int TURNS>
+// Two operands in one launch: the first ba workgroups take a's rows, the rest
+// b's. Four rows per workgroup, a wave each, or (LANES 256) one. grid.y: the matrices.
+template <int LANES, int TURNS>
 __global__ __launch_bounds__(256) void k_split_pack(PackRows a, PackRows b, int ba) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int ROWS = 256 / LANES;
+    __shared__ unsigned red[4];
     const bool first = (int)blockIdx.x < ba;
     const PackRows& p = first ? a : b;
-    const int row = ((int)blockIdx.x - (first ? 0 : ba)) * 4 + w;
-    if (row < p.rows) pack_row<TURNS>(p, row, lane);
+    const int row = ((int)blockIdx.x - (first ? 0 : ba)) * ROWS + (int)threadIdx.x / LANES;
+    if (row >= p.rows) return;  // a whole wave or workgroup
+    const int i = blockIdx.y;
+    const int64_t steps = (p.K + kStep - 1) / kStep;
+    const float* x = p.X + (i / p.inner) * p.outer_ld + (i % p.inner) * p.inner_ld + (int64_t)row * p.ld;
+    pack_row<LANES, TURNS>(p, x, p.P + i * steps * p.rows * (kRowBytes / 2), p.exps + (int64_t)i * p.rows, row,
+                           threadIdx.x % LANES, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -292,10 +312,13 @@ __global__ __launch_bounds__(256) void k_conv_pack(ConvPack a) {
 // ---------------------------------------------------------------------------
 // The product
 // ---------------------------------------------------------------------------
+enum Kind { kDense = 0, kConv = 1, kWeights = 2 };  // kWeights: A holds softmax weights, packed row by row
+
 struct SplitArgs {
     const u16* A;
     const u16* B;
     int64_t planeA, planeB;  // bytes from one step's rows to the next's
+    int rowA;                // bytes from one row of A's step to the next
     const int* ea;           // per row
     const int* eb;           // per column; conv2d: per sample
     float* C;
@@ -306,6 +329,11 @@ struct SplitArgs {
     int tm, tn, splits;      // tiles, parts of K
     float* part;             // splits > 1: [splits][tm * BM][tn * BN] sums without the exponents
     unsigned* slow;          // splits > 1: [tm * tn], the tile was computed by the fp32 path
+    // further products of the same sizes (splits = 1): product i = (o, h) = (i / inner, i % inner)
+    // takes A's matrix i, B's matrix o * kv + h / group and stores at C + o outC + h inC
+    int batches, inner, group, kv;
+    int64_t matA, matB, outC, inC, outA0, inA0, outB0, inB0;
+    int causal, row0;        // kWeights: row r's weights end at column row0 + r
     // the original operands
     const float* A0;
     const float* B0;
@@ -316,10 +344,10 @@ struct SplitArgs {
 };
 
 // One element by fp32 FMAs from the original operands.
-template <bool CONV>
+template <Kind KIND>
 __device__ __forceinline__ float dot_fp32(const SplitArgs& p, int row, int col) {
     float s = 0.f;
-    if constexpr (CONV) {
+    if constexpr (KIND == kConv) {
         const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
         const int iy0 = oy * p.stride - p.pad, ix0 = ox * p.stride - p.pad;
         const float* w = p.A0 + (int64_t)row * p.Cin * p.taps;
@@ -331,6 +359,18 @@ __device__ __forceinline__ float dot_fp32(const SplitArgs& p, int row, int col) 
                     const bool in = (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
                     s = fmaf(*w, in ? x[(int64_t)iy * p.W + ix] : 0.f, s);
                 }
+        }
+    } else if constexpr (KIND == kWeights) {
+        // the softmax weights as they were packed; one too small to be held counts as tiny,
+        // so that it still meets an infinity of B as fp32 has it
+        const int e = p.ea[row];
+        if (e == kBad) return __builtin_nanf("");
+        const float* b = p.B0 + (int64_t)col * p.ldb;
+        const int end = p.causal ? min(p.K, p.row0 + row + 1) : p.K;
+        for (int k = 0; k < end; ++k) {
+            const _Float16* h = (const _Float16*)((const char*)p.A + (int64_t)row * p.rowA + (k / kStep) * p.planeA) + k % kStep;
+            const float w = __builtin_amdgcn_ldexpf((float)h[0] + (float)h[kStep], e);
+            s = fmaf(fmaxf(w, 1e-38f), b[k], s);
         }
     } else {
         const float* a = p.A0 + (int64_t)row * p.lda;
@@ -368,8 +408,9 @@ __device__ __forceinline__ void load_lds(const char* base, int bytes, const int*
                                                  0, 0, 0);
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, bool CONV>
+template <int BM, int BN, int WM, int WN, int STAGES, Kind KIND>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1 : BM * BN == 128 * 128 ? 2 : 3) void k_split_mm(SplitArgs p) {
+    constexpr bool CONV = KIND == kConv;
     static_assert(STAGES == 2 || STAGES == 3, "LDS stages");
     constexpr int NW = (BM / WM) * (BN / WN), T = 64 * NW;
     constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;  // loads per wave and stage: 8 rows each
@@ -390,7 +431,19 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     // one contiguous range of tiles; within it, eight row tiles by all columns.
     const int nblk = gridDim.x, xcd = blockIdx.x & 7, per = nblk >> 3, rem = nblk & 7;
     const int lb = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
-    const int tiles = p.tm * p.tn, z = lb / tiles, lt = lb - z * tiles;
+    const int tiles = p.tm * p.tn, lt = lb % tiles;
+    int z = lb / tiles;
+    if (!CONV && p.batches > 1) {
+        const int o = z / p.inner, h = z - o * p.inner, b = o * p.kv + h / p.group;
+        p.A = (const u16*)((const char*)p.A + z * p.matA);
+        p.B = (const u16*)((const char*)p.B + b * p.matB);
+        p.ea += (int64_t)z * p.M;
+        p.eb += (int64_t)b * p.N;
+        p.C += o * p.outC + h * p.inC;
+        if (KIND == kDense) p.A0 += o * p.outA0 + h * p.inA0;
+        p.B0 += o * p.outB0 + (h / p.group) * p.inB0;
+        z = 0;
+    }
     const int gsz = 8 * p.tn, grp = lt / gsz, in = lt - grp * gsz, gm = min(8, p.tm - grp * 8);
     const int mt = grp * 8 + in % gm, nt = in / gm;
     const int m0 = mt * BM, n0 = nt * BN;
@@ -427,7 +480,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
             if (p.splits > 1 && t == 0) p.slow[lt] = 1;
             for (int i = t; i < BM * BN; i += T) {
                 const int row = m0 + i / BN, col = n0 + i % BN;
-                if (row < p.M && col < p.N) store<CONV>(p, row, col, place<CONV>(p, row, col), dot_fp32<CONV>(p, row, col));
+                if (row < p.M && col < p.N) store<CONV>(p, row, col, place<CONV>(p, row, col), dot_fp32<KIND>(p, row, col));
             }
         }
         return;
@@ -442,7 +495,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
 #pragma unroll
     for (int j = 0; j < AI; ++j) {
         const int r = (w * AI + j) * 8 + lr;
-        va[j] = min(m0 + r, p.M - 1) * kRowBytes + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+        va[j] = min(m0 + r, p.M - 1) * p.rowA + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
     }
 #pragma unroll
     for (int j = 0; j < BI; ++j) {
@@ -457,7 +510,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
             vb[j] = col * kRowBytes + chunk;
         }
     }
-    const int bytesA = p.M * kRowBytes, bytesB = (CONV ? p.zero + 1 : p.N) * kRowBytes;
+    const int bytesA = (p.M - 1) * p.rowA + kRowBytes, bytesB = (CONV ? p.zero + 1 : p.N) * kRowBytes;
     auto issue = [&](int step, u16* dA, u16* dB) __attribute__((always_inline)) {
         int chunk = step, tap = 0;
         if constexpr (CONV) {
@@ -627,6 +680,71 @@ __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) 
         if (row0 + i < p.M) store<CONV>(p, row0 + i, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], p.ea[row0 + i] + ec));
 }
 
+// ---------------------------------------------------------------------------
+// Row softmax whose result is the next product's packed operand, in place:
+// a row of cols scores (ld a multiple of 32) becomes ld / 32 steps of weights
+// (128 bytes take the place of 32 scores), with the row's exponent; the
+// arithmetic is k_softmax.hip's. One workgroup per row, eight consecutive
+// values per thread and turn; every score is read before any is overwritten.
+// Row r's causal mask ends at column row0 + r % period.
+// ---------------------------------------------------------------------------
+template <int TPB, int TURNS>
+__global__ __launch_bounds__(TPB) void k_softmax_split(float* __restrict__ S, int* __restrict__ exps, int cols, int ld,
+                                                      float scale, int causal, int row0, int period) {
+    constexpr int W = TPB / 64;
+    __shared__ float sh[2 * W];
+    const int t = threadIdx.x, row = blockIdx.x;
+    float* x = S + (int64_t)row * ld;
+    const int valid = causal ? min(cols, row0 + row % period + 1) : cols;
+    float v[TURNS][8];
+    float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < TURNS; ++j) {
+        const int k = (j * TPB + t) * 8, kc = min(k, ld - 8);
+        const f4 a = *(const f4*)(x + kc), b = *(const f4*)(x + kc + 4);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[j][i] = k + i < valid ? (i < 4 ? a[i & 3] : b[i & 3]) * scale : -INFINITY;
+            m = fmaxf(m, v[j][i]);
+        }
+    }
+    m = dev::wave_max(m);
+    if constexpr (W > 1) {
+        if ((t & 63) == 0) sh[t >> 6] = m;
+        __syncthreads();
+        m = sh[0];
+#pragma unroll
+        for (int k = 1; k < W; ++k) m = fmaxf(m, sh[k]);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < TURNS; ++j) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[j][i] = expf(v[j][i] - m);
+        s += ((v[j][0] + v[j][1]) + (v[j][2] + v[j][3])) + ((v[j][4] + v[j][5]) + (v[j][6] + v[j][7]));
+    }
+    s = dev::wave_sum(s);
+    if constexpr (W > 1) {
+        if ((t & 63) == 0) sh[W + (t >> 6)] = s;
+        __syncthreads();
+        s = sh[W];
+#pragma unroll
+        for (int k = 1; k < W; ++k) s += sh[W + k];
+    }
+    const float inv = 1.0f / s;  // the largest weight; not finite where a score is not
+    const int e = exp_of(absbits(inv));
+    if (t == 0) exps[row] = e;
+#pragma unroll
+    for (int j = 0; j < TURNS; ++j) {
+        const int k = (j * TPB + t) * 8;
+        if (k >= ld) continue;
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = v[j][i] * inv;
+        store_split((u16*)x + (k / kStep) * (kRowBytes / 2) + (k % kStep), p, e == kBad ? 0 : -e);
+    }
+}
+
 size_t up(size_t n) { return (n + 255) / 256 * 256; }
 
 // The tiles of k_split_mm, with what a launch of it costs on MI355X. A CU holds
@@ -657,7 +775,7 @@ struct Plan {
     int bn() const { return kTiles[tile].bn; }
     size_t part_bytes() const { return splits > 1 ? up((size_t)splits * tm * tn * bm() * bn() * 4) : 0; }
 };
-Plan plan_of(int64_t M, int64_t N, int64_t steps) {
+Plan plan_of(int64_t M, int64_t N, int64_t steps, int64_t batches = 1) {
     Plan best{};
     double least = 0;
     for (int i = 0; i < 4; ++i) {
@@ -665,8 +783,8 @@ Plan plan_of(int64_t M, int64_t N, int64_t steps) {
         const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn, slots = (int64_t)num_cus() * t.cu;
         for (const int parts : kParts) {
             // a part has at least four steps; parts only where one round of workgroups is not full
-            if (parts > 1 && (steps < 4 * parts || tm * tn >= slots)) break;
-            const int64_t n = tm * tn * parts, rest = n % slots;
+            if (parts > 1 && (batches > 1 || steps < 4 * parts || tm * tn >= slots)) break;
+            const int64_t n = tm * tn * parts * batches, rest = n % slots;
             const double k = (double)steps / parts;
             double us = (double)(n / slots) * (k * t.full + t.once);
             if (rest) us += k * (t.idle + (t.full - t.idle) * rest / slots) + t.once;
@@ -680,20 +798,37 @@ Plan plan_of(int64_t M, int64_t N, int64_t steps) {
     return best;
 }
 
-template <bool CONV>
+template <Kind KIND>
 void launch_mm(const Plan& q, SplitArgs& p) {
-    const unsigned grid = (unsigned)(q.tm * q.tn * q.splits);
+    const unsigned grid = (unsigned)(q.tm * q.tn * q.splits * std::max(1, p.batches));
     if (q.tile == 0)
-        k_split_mm<256, 256, 128, 64, 2, CONV><<<grid, 512, 0, stream()>>>(p);
+        k_split_mm<256, 256, 128, 64, 2, KIND><<<grid, 512, 0, stream()>>>(p);
     else if (q.tile == 1)
-        k_split_mm<128, 256, 64, 64, 3, CONV><<<grid, 512, 0, stream()>>>(p);
+        k_split_mm<128, 256, 64, 64, 3, KIND><<<grid, 512, 0, stream()>>>(p);
     else if (q.tile == 2)
-        k_split_mm<128, 128, 64, 64, 2, CONV><<<grid, 256, 0, stream()>>>(p);
+        k_split_mm<128, 128, 64, 64, 2, KIND><<<grid, 256, 0, stream()>>>(p);
     else
-        k_split_mm<64, 64, 32, 32, 3, CONV><<<grid, 256, 0, stream()>>>(p);
+        k_split_mm<64, 64, 32, 32, 3, KIND><<<grid, 256, 0, stream()>>>(p);
     if (q.splits > 1)
-        k_split_sum<CONV><<<dim3((unsigned)((p.N + 255) / 256), (unsigned)((p.M + 3) / 4)), 256, 0, stream()>>>(
+        k_split_sum<KIND == kConv><<<dim3((unsigned)((p.N + 255) / 256), (unsigned)((p.M + 3) / 4)), 256, 0, stream()>>>(
             p, q.bm(), q.bn());
+}
+
+bool vec_rows(const PackRows& a) {
+    return a.K % 4 == 0 && a.ld % 4 == 0 && a.outer_ld % 4 == 0 && a.inner_ld % 4 == 0 && aligned16(a.X);
+}
+// Packs a and b (of the same K; b.rows may be 0), `batches` matrices of each.
+void launch_pack(const PackRows& a, const PackRows& b, int64_t batches) {
+    const bool vec = vec_rows(a) && (!b.rows || vec_rows(b)), wide = a.K > 4096;
+    const int turns = !vec || a.K > 16384 ? 0 : a.K > (wide ? 8192 : 2048) ? 8 : wide || a.K > 1024 ? 4 : a.K > 512 ? 2 : 1;
+    const unsigned ba = blocks_for(a.rows, wide ? 1 : 4), bb = b.rows ? blocks_for(b.rows, wide ? 1 : 4) : 0;
+    auto go = wide ? (turns == 8 ? k_split_pack<256, 8> : turns == 4 ? k_split_pack<256, 4> : k_split_pack<256, 0>)
+                   : (turns == 8   ? k_split_pack<64, 8>
+                      : turns == 4 ? k_split_pack<64, 4>
+                      : turns == 2 ? k_split_pack<64, 2>
+                      : turns == 1 ? k_split_pack<64, 1>
+                                   : k_split_pack<64, 0>);
+    go<<<dim3(ba + bb, (unsigned)batches), 256, 0, stream()>>>(a, b, (int)ba);
 }
 
 constexpr size_t kRowLds = 48 << 10;  // weights of one output channel that k_conv_prep takes through LDS
@@ -715,19 +850,14 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     char* s = (char*)try_scratch(pa + pb + ea + eb + sl + q.part_bytes());
     if (!s) return false;
     SplitArgs p{};
-    PackRows ra{A, lda, (u16*)s, (int*)(s + pa + pb), (int)M, (int)K};
-    PackRows rb{B, ldb, (u16*)(s + pa), (int*)(s + pa + pb + ea), (int)N, (int)K};
-    const unsigned ba = blocks_for(M, 4), bb = blocks_for(N, 4);
-    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && aligned16(A) && aligned16(B);
-    const int turns = !vec || K > 4096 ? 0 : K > 2048 ? 8 : K > 1024 ? 4 : K > 512 ? 2 : 1;
-    auto pack = turns == 8 ? k_split_pack<8> : turns == 4 ? k_split_pack<4> : turns == 2 ? k_split_pack<2>
-                                           : turns == 1   ? k_split_pack<1>
-                                                          : k_split_pack<0>;
-    pack<<<ba + bb, 256, 0, stream()>>>(ra, rb, (int)ba);
+    const PackRows ra{A, lda, (u16*)s, (int*)(s + pa + pb), (int)M, (int)K, 1, 0, 0};
+    const PackRows rb{B, ldb, (u16*)(s + pa), (int*)(s + pa + pb + ea), (int)N, (int)K, 1, 0, 0};
+    launch_pack(ra, rb, 1);
     p.A = ra.P;
     p.B = rb.P;
     p.planeA = M * kRowBytes;
     p.planeB = N * kRowBytes;
+    p.rowA = kRowBytes;
     p.ea = ra.exps;
     p.eb = rb.exps;
     p.C = C;
@@ -747,7 +877,7 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     p.B0 = B;
     p.lda = lda;
     p.ldb = ldb;
-    launch_mm<false>(q, p);
+    launch_mm<kDense>(q, p);
     return true;
 }
 
@@ -797,6 +927,7 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     p.B = a.X;
     p.planeA = Cout * kRowBytes;
     p.planeB = prows * kRowBytes;
+    p.rowA = kRowBytes;
     p.ea = a.ew;
     p.eb = a.ex;
     p.C = out;
@@ -826,7 +957,146 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     p.Cout = (int)Cout;
     p.npb = a.npb;
     p.zero = (int)(prows - 1);
-    launch_mm<true>(q, p);
+    launch_mm<kConv>(q, p);
+    return true;
+}
+
+// Attention through the score matrix (backend_cuda.cu:550-586), for the head
+// dimensions that the fused kernel's registers do not hold: q [N, Sq, heads d],
+// k and v [N, Skv, kv_heads d], fp32, out [N, Sq, heads d] fp32 or bf16, all
+// checked. Per round as many heads, or as many rows of one head, as `budget`
+// bytes of scores hold: S = q k^T, the softmax, which leaves the weights as the
+// packed operand of O = P v, and that product against v^T, packed once. False,
+// with nothing queued, where scratch or sizes do not allow it.
+bool split_attention(const float* q, const float* k, const float* v, void* out, bool out16, int64_t N, int64_t Sq,
+                     int64_t Skv, int heads, int kv_heads, int64_t d, bool causal, float scale, int64_t budget) {
+    const int64_t inner = heads * d, kvi = kv_heads * d, skp = (Skv + kStep - 1) / kStep * kStep;
+    const int64_t dsteps = (d + kStep - 1) / kStep, ssteps = skp / kStep;
+    if (skp > 32768 || Sq * kRowBytes >= kMost || N * heads > 65535) return false;
+    const int group = heads / kv_heads;
+    const int64_t one = Sq * skp * 4, qn = N * heads, kn = N * kv_heads;
+    // heads of a round (whole samples, or groups of one sample's) and rows of a round
+    int64_t nb = 1, rb = Sq;
+    if (one > budget)
+        rb = std::min(Sq, std::max<int64_t>(256, budget / (skp * 4) / 256 * 256));
+    else if (budget / one >= heads)
+        nb = std::min(qn, budget / one / heads * heads);
+    else
+        nb = std::max<int64_t>(1, budget / one / group * group);
+    const Plan p1 = plan_of(rb, Skv, dsteps, nb), p2 = plan_of(rb, d, ssteps, nb);
+    const int64_t most = std::max((int64_t)p1.tm * p1.tn * p1.splits, (int64_t)p2.tm * p2.tn * p2.splits);
+    if (rb * skp * 4 >= kMost || nb * rb >= kMost / 1024 || most * nb * 512 >= kMost) return false;
+    const size_t pq = up((size_t)qn * dsteps * Sq * kRowBytes), pk = up((size_t)kn * dsteps * Skv * kRowBytes);
+    const size_t pv = up((size_t)kn * ssteps * d * kRowBytes), vt = up((size_t)N * kvi * Skv * 4);
+    const size_t sc = up((size_t)nb * rb * skp * 4);
+    const size_t eq = up((size_t)qn * Sq * 4), ek = up((size_t)kn * Skv * 4), ev = up((size_t)kn * d * 4);
+    // these two for any round, so that the budget alone decides what a call holds
+    const size_t ep = up((size_t)qn * Sq * 4), sl = up((size_t)((Sq + 63) / 64) * ((std::max(Skv, d) + 63) / 64) * 4);
+    const size_t parts = std::max(p1.part_bytes(), p2.part_bytes()), o16 = out16 ? up((size_t)N * Sq * inner * 4) : 0;
+    char* s = (char*)try_scratch(pq + pk + pv + vt + sc + eq + ek + ev + ep + sl + o16 + parts);
+    if (!s) return false;
+    auto take = [&](size_t n) {
+        char* r = s;
+        s += n;
+        return r;
+    };
+    const PackRows rq{q, inner, (u16*)take(pq), (int*)take(eq), (int)Sq, (int)d, heads, Sq * inner, d};
+    const PackRows rk{k, kvi, (u16*)take(pk), (int*)take(ek), (int)Skv, (int)d, kv_heads, Skv * kvi, d};
+    float* const tv = (float*)take(vt);
+    const PackRows rv{tv, Skv, (u16*)take(pv), (int*)take(ev), (int)d, (int)Skv, 1, d * Skv, 0};
+    float* const S = (float*)take(sc);
+    int* const exps = (int*)take(ep);
+    unsigned* const slow = (unsigned*)take(sl);
+    float* const o = out16 ? (float*)take(o16) : (float*)out;
+    transpose_device("sdh_attention", v, tv, N, Skv, kvi);
+    const PackRows none{};
+    if (qn == kn) {
+        launch_pack(rq, rk, qn);
+    } else {
+        launch_pack(rq, none, qn);
+        launch_pack(rk, none, kn);
+    }
+    launch_pack(rv, none, kn);
+    auto sized = [](Plan plan, SplitArgs& p) {  // the round's plan, for p's rows
+        p.tm = plan.tm = (p.M + plan.bm() - 1) / plan.bm();
+        p.tn = plan.tn;
+        p.splits = plan.splits;
+        return plan;
+    };
+    int64_t b = 0;
+    for (int64_t b0 = 0; b0 < qn; b0 += b) {
+        const int64_t n0 = b0 / heads, h0 = b0 % heads, kb = n0 * kv_heads + h0 / group;
+        b = nb >= heads ? std::min(nb, qn - b0) : std::min(nb, heads - h0);
+        for (int64_t r0 = 0; r0 < Sq; r0 += rb) {
+            const int64_t m = std::min(rb, Sq - r0);
+            SplitArgs p{};
+            p.batches = (int)b;
+            p.inner = b > 1 ? heads : 1;
+            p.group = b > 1 ? group : 1;
+            p.kv = b > 1 ? kv_heads : 1;
+            p.A = rq.P + (b0 * dsteps * Sq + r0) * (kRowBytes / 2);
+            p.matA = dsteps * Sq * kRowBytes;
+            p.B = rk.P + kb * dsteps * Skv * (kRowBytes / 2);
+            p.matB = dsteps * Skv * kRowBytes;
+            p.planeA = Sq * kRowBytes;
+            p.planeB = Skv * kRowBytes;
+            p.rowA = kRowBytes;
+            p.ea = rq.exps + b0 * Sq + r0;
+            p.eb = rk.exps + kb * Skv;
+            p.C = S;
+            p.ldc = skp;
+            p.outC = heads * m * skp;
+            p.inC = m * skp;
+            p.A0 = q + (n0 * Sq + r0) * inner + h0 * d;
+            p.lda = inner;
+            p.outA0 = Sq * inner;
+            p.inA0 = d;
+            p.B0 = k + n0 * Skv * kvi + h0 / group * d;
+            p.ldb = kvi;
+            p.outB0 = Skv * kvi;
+            p.inB0 = d;
+            p.M = (int)m;
+            p.N = (int)Skv;
+            p.K = (int)d;
+            p.steps = (int)dsteps;
+            p.slow = slow;
+            p.part = (float*)s;
+            launch_mm<kDense>(sized(p1, p), p);
+            auto soft = skp <= 512    ? k_softmax_split<64, 1>
+                        : skp <= 2048 ? k_softmax_split<256, 1>
+                        : skp <= 4096 ? k_softmax_split<512, 1>
+                        : skp <= 8192 ? k_softmax_split<1024, 1>
+                        : skp <= 16384 ? k_softmax_split<1024, 2>
+                                       : k_softmax_split<1024, 4>;
+            const unsigned tpb = skp <= 512 ? 64 : skp <= 2048 ? 256 : skp <= 4096 ? 512 : 1024;
+            soft<<<(unsigned)(b * m), tpb, 0, stream()>>>(S, exps, (int)Skv, (int)skp, scale, causal ? 1 : 0, (int)r0,
+                                                         (int)m);
+            p.A = (const u16*)S;
+            p.matA = m * skp * 4;
+            p.planeA = kRowBytes;
+            p.rowA = (int)(skp * 4);
+            p.ea = exps;
+            p.B = rv.P + kb * ssteps * d * (kRowBytes / 2);
+            p.matB = ssteps * d * kRowBytes;
+            p.planeB = d * kRowBytes;
+            p.eb = rv.exps + kb * d;
+            p.C = o + (n0 * Sq + r0) * inner + h0 * d;
+            p.ldc = inner;
+            p.outC = Sq * inner;
+            p.inC = d;
+            p.B0 = tv + kb * d * Skv;
+            p.ldb = Skv;
+            p.outB0 = kvi * Skv;
+            p.inB0 = d * Skv;
+            p.N = (int)d;
+            p.K = (int)Skv;
+            p.steps = (int)ssteps;
+            p.causal = causal ? 1 : 0;
+            p.row0 = (int)r0;
+            launch_mm<kWeights>(sized(p2, p), p);
+        }
+    }
+    if (out16) to_bf16_device("sdh_attention", o, (uint16_t*)out, N * Sq * inner);
     return true;
 }
 

@@ -94,6 +94,10 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
                 int64_t ldc, const float* bias, bool accumulate);
 bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, const float* w, int64_t Cout, int64_t kh,
                 int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo);
+// Attention of checked arguments through a score matrix of at most `budget`
+// bytes at a time, its products on split operands; false as above.
+bool split_attention(const float* q, const float* k, const float* v, void* out, bool out16, int64_t N, int64_t Sq,
+                     int64_t Skv, int heads, int kv_heads, int64_t d, bool causal, float scale, int64_t budget);
 // y = silu(gate) * up over n floats (the SwiGLU kernel of sdh_swiglu, no checks).
 void launch_swiglu(const float* gate, const float* up, float* y, int64_t n);
 // sdh_softmax_rows on [rows, cols] (k_softmax.hip), errors named after `op`.

@@ -136,6 +136,57 @@ def test_conv_far_pixels_and_specials(be, orc, special):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,Sq,Skv,heads,kvh,d,causal", [
+    (1, 450, 450, 1, 1, 512, False), (2, 70, 65, 4, 2, 160, True), (1, 333, 77, 8, 8, 160, False),
+    (2, 257, 301, 6, 3, 130, True), (1, 129, 2100, 2, 1, 256, False), (1, 40, 4100, 1, 1, 200, True),
+    (1, 33, 16390, 1, 1, 144, False),  # the widest softmax rows
+])
+@pytest.mark.parametrize("out16", [False, True])
+def test_wide_attention(be, orc, N, Sq, Skv, heads, kvh, d, causal, out16):
+    """Head dimensions above 128 through the score matrix: odd sizes, grouped
+    heads, several samples, more keys than queries; the bar of the other routes."""
+    q, k, v = (orc.randn(s, 5000 + i + d) for i, s in enumerate(((N, Sq, heads * d), (N, Skv, kvh * d), (N, Skv, kvh * d))))
+    out = sdhip_array(be, (N, Sq, heads * d), out16)
+    call = be.attention_bf16 if out16 else be.attention
+    call(be.array(q), be.array(k), be.array(v), out, N, Sq, Skv, heads, kvh, d, causal)
+    want = orc.attention(q, k, v, heads, causal, kvh)
+    got = out.download()
+    if out16:
+        from oracle import bf16_to_f32
+
+        got = bf16_to_f32(got).reshape(want.shape)
+    bound = 1e-4 + (2.0 ** -8 * np.abs(want) if out16 else 0)  # bf16: half a step, 2^-9, and its neighbour
+    assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) - bound))
+
+
+def sdhip_array(be, shape, bits16):
+    import sdhip
+
+    return sdhip.DArray(be, shape, dtype=np.uint16 if bits16 else np.float32)
+
+
+@pytest.mark.gpu
+def test_wide_attention_specials(be, orc):
+    """A query and a key with NaN, a value channel with an infinity: what they
+    touch is not finite, as in fp32; the rest is untouched."""
+    S, d = 150, 160
+    q, k, v = (orc.randn((1, S, 2 * d), 5100 + i) for i in range(3))
+    q[0, 20, 5] = np.nan        # row 20 of head 0
+    k[0, 100, d + 3] = np.nan   # head 1: rows 100 and on, by the causal mask
+    v[0, 50, 7] = np.inf        # head 0, channel 7: rows 50 and on
+    out = be.empty((1, S, 2 * d))
+    be.attention(be.array(q), be.array(k), be.array(v), out, 1, S, S, 2, 2, d, True)
+    got = out.download()
+    bad = np.zeros((1, S, 2 * d), bool)
+    bad[0, 20, :d] = bad[0, 100:, d:] = bad[0, 50:, 7] = True
+    assert np.array_equal(~np.isfinite(got), bad)
+    assert np.all(got[0, [r for r in range(50, S) if r != 20], 7] == np.inf)
+    q[0, 20, 5] = k[0, 100, d + 3] = v[0, 50, 7] = 0
+    want = orc.attention(q, k, v, 2, True, 2)
+    assert np.max(np.abs(got - want)[~bad]) <= 1e-4
+
+
+@pytest.mark.gpu
 def test_graph_keeps_its_scratch(be, orc):
     """A graph holds the scratch block of its capture: the block lives on when
     a larger one replaces it, and replays over new inputs stay right."""
