@@ -483,6 +483,10 @@ void run_gemm(const char* op, int64_t M, int64_t N, int64_t K, const float* A, i
     }
     check_range(C, (size_t)((M - 1) * ldc + N) * 4, op, EPI == E_SWIGLU ? "y" : "C");
     if (bias) check_range(bias, (size_t)N * 4, op, "bias");
+    if (EPI == E_LINEAR && gemv_bf16(M, N, K, A, lda, B0, ldb, C, ldc, bias, accumulate)) {  // a few rows
+        launched(op);
+        return;
+    }
     const bool fast = K > 0 && K % 8 == 0 && lda % 4 == 0 && ldb % 8 == 0 && aligned(A, 16) && aligned(B0, 16) &&
                       (EPI != E_SWIGLU || aligned(B1, 16)) && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31);
     if (fast) {

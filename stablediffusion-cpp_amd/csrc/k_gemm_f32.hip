@@ -115,6 +115,10 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     }
     check_range(C, (size_t)((M - 1) * ldc + N) * 4, op, "C");
     if (bias) check_range(bias, (size_t)N * 4, op, "bias");
+    if (gemv_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {  // a few rows
+        launched(op);
+        return;
+    }
     const bool lt = K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) &&
                     aligned(C, 16) && (!bias || aligned(bias, 16));
     // Split operands from the size where their pack and second launch pay

@@ -88,6 +88,12 @@ void* workspace(size_t bytes);
 // (k_gemm.hip). False when hipBLASLt has no algorithm for the shape.
 bool blaslt_gemm(bool f32, int64_t M, int64_t N, int64_t K, const void* P, int64_t ldp, const void* B, int64_t ldb,
                  float* C, int64_t ldc, const float* bias, bool accumulate);
+// Linear layers of at most 8 rows (k_gemv.hip), with checked arguments; false
+// where a GEMM takes them. B fp32, or bf16 with A rounded to it.
+bool gemv_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+              int64_t ldc, const float* bias, bool accumulate);
+bool gemv_bf16(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const uint16_t* B, int64_t ldb, float* C,
+               int64_t ldc, const float* bias, bool accumulate);
 // The fp32 product and conv2d on split fp16 operands (k_gemm_split.hip), with
 // checked arguments; false where the caller's general path has to run.
 bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
