@@ -70,6 +70,7 @@ namespace sdh {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned short u16;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -108,14 +109,19 @@ __device__ __forceinline__ void split(float x, _Float16& hi, _Float16& lo) {
     hi = (_Float16)x;
     lo = (_Float16)(x - (float)hi);
 }
-// Softmax weight p in [0, 2^16) into hi + lo: hi keeps p's leading 11 bits
-// (truncated: exact in fp16 for p >= 2^-14), lo = p - hi exactly in fp32,
-// then rounded to fp16 (|lo| < 2^-10 p, so the pair is within 2^-21 p; below
-// 2^-14, where fp16 is subnormal, within 2^-24 absolutely).
-__device__ __forceinline__ void split_weight(float p, _Float16& hi, _Float16& lo) {
-    const float h = __uint_as_float(__float_as_uint(p) & 0xFFFFE000u);
-    hi = (_Float16)h;
-    lo = (_Float16)(p - h);
+// Two softmax weights in [0, 2^16) into hi + lo: hi is p towards zero in fp16
+// (v_cvt_pkrtz), lo = p - hi rounded to fp16 (|lo| < 2^-10 p, so the pair is
+// within 2^-21 p; below 2^-14, where fp16 is subnormal, within 2^-25
+// absolutely). v_fma_mixlo/mixhi take hi's half as it lies in the packed pair and
+// round the exact difference into a half: three instructions a pair, where
+// masking, subtracting and packing took six.
+__device__ __forceinline__ void split_weights(float p0, float p1, h2& hi, h2& lo) {
+    hi = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+    const unsigned h = __builtin_bit_cast(unsigned, hi);
+    unsigned l;
+    asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l) : "v"(h), "v"(p0));
+    asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l) : "v"(h), "v"(p1));
+    lo = __builtin_bit_cast(h2, l);
 }
 
 // Exponent e of a block whose largest magnitude is amax: amax 2^-e lies in
@@ -131,7 +137,8 @@ __device__ __forceinline__ float pow2(int e) { return __uint_as_float((unsigned)
 // ---------------------------------------------------------------------------
 // Pack: k, v [N, Skv, kv_heads * d] (fp32) -> tiles as described above, and
 // the exponents (e_k, e_v) of every tile. One workgroup per (tile, kv head,
-// batch); 256 threads. VEC: d == DP and 16-B aligned rows (float4 loads).
+// batch); 256 threads. VEC: d a multiple of 8 and 16-B aligned rows (float4
+// loads; a chunk past the head dimension re-reads the last one, zeroed after).
 // ---------------------------------------------------------------------------
 template <int DP, bool VEC, bool SPLIT>
 __global__ __launch_bounds__(256) void k_attn_pack(const float* __restrict__ K, const float* __restrict__ V,
@@ -160,9 +167,9 @@ __global__ __launch_bounds__(256) void k_attn_pack(const float* __restrict__ K, 
             // unconditional loads (rows past the keys re-read the last row,
             // zeroed after the load): a load under a mask splits the kernel
             // into blocks that cost registers
-            const f4* p = (const f4*)(K + (row0 + min(r, nrows - 1)) * kv_inner + col0 + c * 8);
+            const f4* p = (const f4*)(K + (row0 + min(r, nrows - 1)) * kv_inner + col0 + min(c * 8, d - 8));
             f4 a = dev::ld_stream(p), b = dev::ld_stream(p + 1);
-            if (r >= nrows) a = b = f4{0.f, 0.f, 0.f, 0.f};
+            if (r >= nrows || c * 8 >= d) a = b = f4{0.f, 0.f, 0.f, 0.f};
             kx[j][0] = a.x; kx[j][1] = a.y; kx[j][2] = a.z; kx[j][3] = a.w;
             kx[j][4] = b.x; kx[j][5] = b.y; kx[j][6] = b.z; kx[j][7] = b.w;
         } else {
@@ -181,8 +188,8 @@ __global__ __launch_bounds__(256) void k_attn_pack(const float* __restrict__ K, 
         const int i = threadIdx.x + j * 256, r = i / (DP / 4), c = (i % (DP / 4)) * 4;
         f4 x = {0.f, 0.f, 0.f, 0.f};
         if constexpr (VEC) {
-            x = dev::ld_stream((const f4*)(V + (row0 + min(r, nrows - 1)) * kv_inner + col0 + c));
-            if (r >= nrows) x = f4{0.f, 0.f, 0.f, 0.f};
+            x = dev::ld_stream((const f4*)(V + (row0 + min(r, nrows - 1)) * kv_inner + col0 + min(c, d - 4)));
+            if (r >= nrows || c >= d) x = f4{0.f, 0.f, 0.f, 0.f};
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -371,13 +378,13 @@ __global__ __launch_bounds__(256) void k_qkv_prep(float* __restrict__ Q, const f
 // the MFMA work alone (the earlier two-barrier schedule, softmax and O += V P
 // in one segment against S^T in the other, took 8960).
 // ---------------------------------------------------------------------------
-template <int DP, bool CAUSAL, bool OUT16, bool SPLIT>
+template <int DP, int DS, int DT, bool CAUSAL, bool OUT16, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restrict__ Q, const u16* __restrict__ tiles,
                                                           const int2* __restrict__ exps, void* __restrict__ O, int Sq,
                                                           int Skv, int inner, int d, int group, int kv_heads,
                                                           int ntiles, float c2, int qvec, int nqb, int heads) {
-    constexpr int DS = DP / 16;                    // 16-wide head-dim steps of S^T = K Q^T
-    constexpr int DT = DP / 32;                    // 32-row head-dim tiles of O^T
+    // DS 16-wide head-dim steps of S^T = K Q^T, DT 32-row head-dim tiles of O^T
+    static_assert(DS * 16 <= DP && DT * 32 <= DP && DT >= 2, "head dimension steps");
     constexpr int TILE = (SPLIT ? 4 : 2) * kKT * DP, HALF = TILE / 2;  // fp16 values per packed tile, per K or V part
     constexpr int NLD = HALF * 2 / 16 / kThreads;  // 16-B loads per thread per part
     // Four separate LDS objects, each named statically where it is read or
@@ -431,20 +438,34 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
         const float* qp = Q + ((int64_t)nb * Sq + min(qlane, Sq - 1)) * inner + (int64_t)h * d;
         float x[DS][8];
         float qmax = 0.f;
+        if (qvec) {
+            f4 a[DS], b[DS];  // every load first; past the head dimension: its last chunk, dropped below
 #pragma unroll
-        for (int ds = 0; ds < DS; ++ds) {
-            const int c0 = ds * 16 + fh * 8;
-            if (qvec) {
-                const f4 a = *(const f4*)(qp + c0), b = *(const f4*)(qp + c0 + 4);
-                x[ds][0] = a.x; x[ds][1] = a.y; x[ds][2] = a.z; x[ds][3] = a.w;
-                x[ds][4] = b.x; x[ds][5] = b.y; x[ds][6] = b.z; x[ds][7] = b.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[ds][e] = c0 + e < d ? qp[c0 + e] : 0.f;
+            for (int ds = 0; ds < DS; ++ds) {
+                const float* p = qp + min(ds * 16 + fh * 8, d - 8);
+                a[ds] = *(const f4*)p;
+                b[ds] = *(const f4*)(p + 4);
             }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qmax = fmaxf(qmax, fabsf(x[ds][e]));
+            for (int ds = 0; ds < DS; ++ds)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = e < 4 ? a[ds][e & 3] : b[ds][e & 3];
+                    x[ds][e] = ds * 16 + fh * 8 < d ? v : 0.f;
+                }
+        } else {
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int c = ds * 16 + fh * 8 + e;
+                    x[ds][e] = c < d ? qp[c] : 0.f;
+                }
         }
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qmax = fmaxf(qmax, fabsf(x[ds][e]));
         qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
         eq = block_exp(qmax);
         const float sc = pow2(-eq);
@@ -561,29 +582,29 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
+            for (int e = 0; e < 8; e += 2) {
+                const float p0 = s[ks >> 1][(ks & 1) * 8 + e], p1 = s[ks >> 1][(ks & 1) * 8 + e + 1];
                 if constexpr (SPLIT) {
-                    _Float16 hi, lo;
-                    split_weight(s[ks >> 1][(ks & 1) * 8 + e], hi, lo);
-                    ph[ks][e] = hi;
-                    pl[ks][e] = lo;
+                    h2 hi, lo;
+                    split_weights(p0, p1, hi, lo);
+                    ph[ks][e] = hi[0], ph[ks][e + 1] = hi[1];
+                    pl[ks][e] = lo[0], pl[ks][e + 1] = lo[1];
                 } else {
-                    ph[ks][e] = (_Float16)s[ks >> 1][(ks & 1) * 8 + e];
+                    ph[ks][e] = (_Float16)p0, ph[ks][e + 1] = (_Float16)p1;
                 }
             }
     };
-    // O^T += V^T P^T in 2 DT steps of (16-key step ks, pair of 32-row tiles
-    // dt, dt + 1): step i reads the pair's hi/lo V fragments kPipe - 1 steps
+    // O^T += V^T P^T in 2 DT steps of two (16-key step ks, 32-row tile dt) each,
+    // tiles fastest: a step reads its two hi/lo V fragments kPipe - 1 steps
     // ahead of its MFMAs, and interleaves the two accumulator chains
     auto pv = [&](const u16* Vh) __attribute__((always_inline)) {
         const u16* Vl = Vh + DP * kKT;
         constexpr int NS = 2 * DT;
         h8 vf[kPipe][2][2];  // [slot][dt of the pair][hi, lo]
         auto fetch = [&](int i) __attribute__((always_inline)) {
-            const int ks = i / (DT / 2), d0 = (i % (DT / 2)) * 2;
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                const int r = (d0 + u) * 32 + fr;
+                const int ks = (i * 2 + u) / DT, r = (i * 2 + u) % DT * 32 + fr;
                 const int off = r * kKT + (((ks * 2 + fh) ^ swz_v(r)) << 3);
                 vf[i % kPipe][u][0] = *(const h8*)(Vh + off);
                 if constexpr (SPLIT) vf[i % kPipe][u][1] = *(const h8*)(Vl + off);
@@ -595,17 +616,18 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
         for (int i = 0; i < NS; ++i) {
             if (i + kPipe - 1 < NS) fetch(i + kPipe - 1);
             __builtin_amdgcn_sched_barrier(0);
-            const int ks = i / (DT / 2), d0 = (i % (DT / 2)) * 2, sl = i % kPipe;
+            const int sl = i % kPipe;
+            auto mma = [&](int u, const h8& vv, const h8* pp) __attribute__((always_inline)) {
+                const int ks = (i * 2 + u) / DT, dt = (i * 2 + u) % DT;
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv, pp[ks], o[dt], 0, 0, 0);
+            };
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                o[d0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[sl][u][0], ph[ks], o[d0 + u], 0, 0, 0);
+            for (int u = 0; u < 2; ++u) mma(u, vf[sl][u][0], ph);
             if constexpr (SPLIT) {
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
-                    o[d0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[sl][u][0], pl[ks], o[d0 + u], 0, 0, 0);
+                for (int u = 0; u < 2; ++u) mma(u, vf[sl][u][0], pl);
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
-                    o[d0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[sl][u][1], ph[ks], o[d0 + u], 0, 0, 0);
+                for (int u = 0; u < 2; ++u) mma(u, vf[sl][u][1], ph);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -672,7 +694,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
                 // the rounding gemm_nt_bf16 gives its A, applied to the fp32 value above
                 u16* op = (u16*)O + obase;
                 if (qvec) {
-                    *(uint2*)(op + c0) = dev::bf16x4(v);
+                    if (c0 < d) *(uint2*)(op + c0) = dev::bf16x4(v);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -681,7 +703,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
             } else {
                 float* op = (float*)O + obase;
                 if (qvec) {
-                    *(f4*)(op + c0) = v;
+                    if (c0 < d) *(f4*)(op + c0) = v;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -796,24 +818,36 @@ void run_mfma(const float* q, const float* k, const float* v, void* out, int64_t
     }
     if (prep) {
         need(DP == 128, "sdh_qknorm_rope_attention", "internal: fused preparation needs head dim 128");
-    } else if (d == DP && kv_inner % 4 == 0 && aligned16(k) && aligned16(v))
+    } else if (d % 8 == 0 && kv_inner % 4 == 0 && aligned16(k) && aligned16(v))
         k_attn_pack<DP, true, SPLIT><<<pgrid, 256, 0, stream()>>>(k, v, tiles, exps, (int)Skv, (int)kv_inner, (int)d,
                                                            (int)ntiles, kv_heads);
     else
         k_attn_pack<DP, false, SPLIT><<<pgrid, 256, 0, stream()>>>(k, v, tiles, exps, (int)Skv, (int)kv_inner, (int)d,
                                                             (int)ntiles, kv_heads);
     launched("sdh_attention");
-    const int qvec = d == DP && inner % 4 == 0 && aligned16(q) && (OUT16 ? ((uintptr_t)out & 7) == 0 : aligned16(out));
+    const int qvec = d % 8 == 0 && inner % 4 == 0 && aligned16(q) && (OUT16 ? ((uintptr_t)out & 7) == 0 : aligned16(out));
     const int64_t nqb = (Sq + kBM - 1) / kBM, nblk = nqb * heads * N;
     need(nblk * kThreads <= kMaxGridItems, "sdh_attention", "too many query blocks for one launch");
-    if (causal)
-        k_attn_fwd<DP, true, OUT16, SPLIT><<<(unsigned)nblk, kThreads, 0, stream()>>>(
-            q, tiles, exps, out, (int)Sq, (int)Skv, (int)inner, (int)d, heads / kv_heads, kv_heads, (int)ntiles, c2,
-            qvec, (int)nqb, heads);
-    else
-        k_attn_fwd<DP, false, OUT16, SPLIT><<<(unsigned)nblk, kThreads, 0, stream()>>>(
-            q, tiles, exps, out, (int)Sq, (int)Skv, (int)inner, (int)d, heads / kv_heads, kv_heads, (int)ntiles, c2,
-            qvec, (int)nqb, heads);
+    // The steps and tiles that the head dimension fills: SD 1.5's 40 and 80 leave
+    // an eighth and a third of the padded tile's MFMAs out. Measured, together
+    // with float4 loads of q, k and v for every multiple of 8 (element loads under
+    // a mask before): [2,4096,8x40] 187 -> 169 us,
+    // [2,4096,8x40] to 77 keys 25.8 -> 16.0, [2,1024,8x80] 86 -> 57, [1,920,8x80] to
+    // 77 keys 36 -> 17 us; [1,4224,30x128] 640 -> 638.
+    auto fwd = [&](auto ds, auto dt) {
+        constexpr int DS = decltype(ds)::value, DT = decltype(dt)::value;
+        auto go = causal ? k_attn_fwd<DP, DS, DT, true, OUT16, SPLIT> : k_attn_fwd<DP, DS, DT, false, OUT16, SPLIT>;
+        go<<<(unsigned)nblk, kThreads, 0, stream()>>>(q, tiles, exps, out, (int)Sq, (int)Skv, (int)inner, (int)d,
+                                                     heads / kv_heads, kv_heads, (int)ntiles, c2, qvec, (int)nqb, heads);
+    };
+    using std::integral_constant;
+    if constexpr (DP == 64) {
+        if (d <= 48) fwd(integral_constant<int, 3>(), integral_constant<int, 2>());
+        else fwd(integral_constant<int, 4>(), integral_constant<int, 2>());
+    } else {
+        if (d <= 80) fwd(integral_constant<int, 5>(), integral_constant<int, 3>());
+        else fwd(integral_constant<int, 8>(), integral_constant<int, 4>());
+    }
     launched("sdh_attention");
 }
 
