@@ -79,6 +79,7 @@ using dev::f4;
 constexpr int kKT = 64;                     // keys per tile
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
 constexpr int kBM = 32 * kWaves;            // queries per workgroup
+constexpr int kKeyWaves = 4;                // waves per 32 queries of the form for few queries
 constexpr float kLog2e = 1.44269504088896341f;
 constexpr float kNoMax = -1e30f;            // running max before any key: finite, so 2^(m - m') never sees inf - inf
 // The running reference m is raised only when a tile's max passes it by
@@ -378,8 +379,13 @@ __global__ __launch_bounds__(256) void k_qkv_prep(float* __restrict__ Q, const f
 // the MFMA work alone (the earlier two-barrier schedule, softmax and O += V P
 // in one segment against S^T in the other, took 8960).
 // ---------------------------------------------------------------------------
-template <int DP, int DS, int DT, bool CAUSAL, bool OUT16, bool SPLIT>
-__global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restrict__ Q, const u16* __restrict__ tiles,
+// KEYS: the form for few queries. A workgroup of 4 waves takes 32 queries of one
+// head, and its waves every fourth key tile each, read from memory straight into
+// registers (one wave has no other to share a tile with); the waves' sums are
+// put together through LDS at the end. Waits once per tile instead of once per
+// 256 queries' tile: see the rule at the launch.
+template <int DP, int DS, int DT, bool CAUSAL, bool OUT16, bool SPLIT, bool KEYS>
+__global__ __launch_bounds__(KEYS ? 64 * kKeyWaves : kThreads, 1) void k_attn_fwd(const float* __restrict__ Q, const u16* __restrict__ tiles,
                                                           const int2* __restrict__ exps, void* __restrict__ O, int Sq,
                                                           int Skv, int inner, int d, int group, int kv_heads,
                                                           int ntiles, float c2, int qvec, int nqb, int heads) {
@@ -391,10 +397,14 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
     // filled (the loop below is unrolled by two): the compiler then knows
     // which LDS-DMA writes a read can alias, and does not make the read of
     // one buffer wait for the copy into the other.
-    __shared__ __attribute__((aligned(1024))) u16 kbuf0[HALF];
-    __shared__ __attribute__((aligned(1024))) u16 kbuf1[HALF];
-    __shared__ __attribute__((aligned(1024))) u16 vbuf0[HALF];
-    __shared__ __attribute__((aligned(1024))) u16 vbuf1[HALF];
+    constexpr int BUF = KEYS ? 8 : HALF;
+    __shared__ __attribute__((aligned(1024))) u16 kbuf0[BUF];
+    __shared__ __attribute__((aligned(1024))) u16 kbuf1[BUF];
+    __shared__ __attribute__((aligned(1024))) u16 vbuf0[BUF];
+    __shared__ __attribute__((aligned(1024))) u16 vbuf1[BUF];
+    // KEYS: each wave's O, running reference and sum
+    __shared__ float part_o[KEYS ? kKeyWaves : 1][KEYS ? DT * 16 : 1][64];
+    __shared__ float part_m[KEYS ? kKeyWaves : 1][64], part_l[KEYS ? kKeyWaves : 1][64];
 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const bool isY = w >= kWaves / 2;
@@ -406,9 +416,9 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
     const int nblk = gridDim.x, xcd = blockIdx.x & 7, per = nblk >> 3, rem = nblk & 7;
     const int lb = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
     const int qb = lb % nqb, h = (lb / nqb) % heads, nb = lb / (nqb * heads), kh = h / group;
-    const int q0 = qb * kBM, qw0 = q0 + w * 32;
+    const int q0 = qb * (KEYS ? 32 : kBM), qw0 = KEYS ? q0 : q0 + w * 32;
     const int qlane = qw0 + fr;
-    const int qend = min(q0 + kBM, Sq);
+    const int qend = min(q0 + (KEYS ? 32 : kBM), Sq);
     const int T = CAUSAL ? min(ntiles, (qend - 1) / kKT + 1) : ntiles;
     const u16* src = tiles + ((int64_t)nb * kv_heads + kh) * ntiles * TILE;
     const int2* ex = exps + ((int64_t)nb * kv_heads + kh) * ntiles;
@@ -428,7 +438,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
                                                      16, lane * 16, off + chunk * 16, 0, 0);
         }
     };
-    issue(0, 0, kbuf0);
+    if constexpr (!KEYS) issue(0, 0, kbuf0);
 
     // Q fragments (B operand of S^T): query qlane, head dims ds*16 + fh*8 .. +7,
     // scaled by 2^-eq for the query's largest magnitude (lanes l and l^32 hold its two halves)
@@ -632,6 +642,85 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    if constexpr (KEYS) {
+        for (int t = w; t < T; t += kKeyWaves) {
+            const u16 *Kh = src + (int64_t)t * TILE, *Vh = Kh + HALF;
+            constexpr int P = SPLIT ? 2 : 1, NV = 4 * DT;
+            h8 kf[DS][2][2], vf[NV][2];  // the tile's fragments, all on their way at once
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int l = 0; l < P; ++l) {
+                        const int r = j * 32 + fr;
+                        kf[ds][j][l] = *(const h8*)(Kh + l * kKT * DP + r * DP + (((ds * 2 + fh) ^ swz_k<DP>(r)) << 3));
+                    }
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int l = 0; l < P; ++l) {
+                    const int ks = i / DT, r = i % DT * 32 + fr;
+                    vf[i][l] = *(const h8*)(Vh + l * kKT * DP + r * kKT + (((ks * 2 + fh) ^ swz_v(r)) << 3));
+                }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[j][i] = 0.f;
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds][j][0], qh[ds], s[j], 0, 0, 0);
+                if constexpr (SPLIT) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds][j][0], ql[ds], s[j], 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds][j][1], qh[ds], s[j], 0, 0, 0);
+                }
+            }
+            softmax(t);
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int ks = i / DT, dt = i % DT;
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][0], ph[ks], o[dt], 0, 0, 0);
+                if constexpr (SPLIT) {
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][0], pl[ks], o[dt], 0, 0, 0);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][1], ph[ks], o[dt], 0, 0, 0);
+                }
+            }
+        }
+        // every wave's sums on the scale of the largest reference; wave w then
+        // holds the rows of the 8-row groups w DT .. w DT + DT - 1 of O^T
+        part_m[w][lane] = m;
+        part_l[w][lane] = lsum;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) part_o[w][dt * 16 + i][lane] = o[dt][i];
+        __syncthreads();
+        float f[kKeyWaves], best = part_m[0][lane];
+#pragma unroll
+        for (int i = 1; i < kKeyWaves; ++i) best = fmaxf(best, part_m[i][lane]);
+        lsum = 0.f;
+#pragma unroll
+        for (int i = 0; i < kKeyWaves; ++i) {
+            f[i] = __builtin_amdgcn_exp2f(part_m[i][lane] - best);
+            lsum = fmaf(f[i], part_l[i][lane], lsum);
+        }
+#pragma unroll
+        for (int k = 0; k < DT; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = 0.f;
+#pragma unroll
+                for (int i = 0; i < kKeyWaves; ++i) v = fmaf(f[i], part_o[i][(w * DT + k) * 4 + e][lane], v);
+                o[k / 4][k % 4 * 4 + e] = v;
+            }
+    }
     // a wave with no real query, or (causal) whose queries all precede tile t, skips it
     const bool active = qw0 < Sq;
     auto wants = [&](int t) { return active && !(CAUSAL && qw0 + 31 < t * kKT); };
@@ -673,22 +762,25 @@ __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const float* __restric
             if (t < T && wants(t)) scores(kc);
         }
     };
-    for (int t = 0; t <= T; t += 2) {
-        iteration(t, kbuf0, vbuf1, kbuf1, vbuf0);
-        if (t + 1 <= T) iteration(t + 1, kbuf1, vbuf0, kbuf0, vbuf1);
+    if constexpr (!KEYS) {
+        for (int t = 0; t <= T; t += 2) {
+            iteration(t, kbuf0, vbuf1, kbuf1, vbuf0);
+            if (t + 1 <= T) iteration(t + 1, kbuf1, vbuf0, kbuf0, vbuf1);
+        }
+        // the surplus copies must land before the workgroup's LDS is released
+        __builtin_amdgcn_s_waitcnt(kWaitVmBase);
     }
-    // the surplus copies must land before the workgroup's LDS is released
-    __builtin_amdgcn_s_waitcnt(kWaitVmBase);
     if (qlane >= Sq) return;
     lsum += __shfl_xor(lsum, 32, 64);
     // the reference scales P by 1/sum (tensor.cpp:761-764); O^T carries 2^(14-E) sum(p v), lsum 2^14 sum(p)
     const float inv = ldexpf(1.0f / lsum, E);
     const int64_t obase = ((int64_t)nb * Sq + qlane) * inner + (int64_t)h * d;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < (KEYS ? (DT + 3) / 4 : DT); ++dt)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int c0 = dt * 32 + g * 8 + fh * 4;
+            if (KEYS && dt * 4 + g >= DT) break;  // DT groups of eight rows each: see above
+            const int c0 = (KEYS ? w * DT + dt * 4 + g : dt * 4 + g) * 8 + fh * 4;
             const f4 v = {o[dt][g * 4] * inv, o[dt][g * 4 + 1] * inv, o[dt][g * 4 + 2] * inv, o[dt][g * 4 + 3] * inv};
             if constexpr (OUT16) {
                 // the rounding gemm_nt_bf16 gives its A, applied to the fp32 value above
@@ -828,6 +920,16 @@ void run_mfma(const float* q, const float* k, const float* v, void* out, int64_t
     const int qvec = d % 8 == 0 && inner % 4 == 0 && aligned16(q) && (OUT16 ? ((uintptr_t)out & 7) == 0 : aligned16(out));
     const int64_t nqb = (Sq + kBM - 1) / kBM, nblk = nqb * heads * N;
     need(nblk * kThreads <= kMaxGridItems, "sdh_attention", "too many query blocks for one launch");
+    const int64_t nq32 = (Sq + 31) / 32;
+    // The form for few queries while its 32-query workgroups are one round (they
+    // hold a CU each), or two of many tiles: the other form then leaves most CUs
+    // idle. Measured (us, other form / this one): [1,203,32x128] causal 26.3 / 19.8,
+    // [1,96,30x128] 18.5 / 17.5, [2,512,8x40] 26.3 / 16.3, [1,1024,8x40] 41.6 / 20.4,
+    // [1,4096,2x128] 213 / 138 at one round, [1,2048,8x40] 76 / 50 at two of 32
+    // tiles; but [1,512,30x128] 49 / 60 at two of 8, [2,4096,8x40] to 77 keys
+    // 15.6 / 43 at eight, and with a single tile 13.3 / 13.6.
+    const int64_t nwg = nq32 * heads * N;
+    const bool keys = (nwg <= num_cus() && ntiles >= 2) || (nwg <= 2 * num_cus() && ntiles >= 24);
     // The steps and tiles that the head dimension fills: SD 1.5's 40 and 80 leave
     // an eighth and a third of the padded tile's MFMAs out. Measured, together
     // with float4 loads of q, k and v for every multiple of 8 (element loads under
@@ -836,9 +938,11 @@ void run_mfma(const float* q, const float* k, const float* v, void* out, int64_t
     // 77 keys 36 -> 17 us; [1,4224,30x128] 640 -> 638.
     auto fwd = [&](auto ds, auto dt) {
         constexpr int DS = decltype(ds)::value, DT = decltype(dt)::value;
-        auto go = causal ? k_attn_fwd<DP, DS, DT, true, OUT16, SPLIT> : k_attn_fwd<DP, DS, DT, false, OUT16, SPLIT>;
-        go<<<(unsigned)nblk, kThreads, 0, stream()>>>(q, tiles, exps, out, (int)Sq, (int)Skv, (int)inner, (int)d,
-                                                     heads / kv_heads, kv_heads, (int)ntiles, c2, qvec, (int)nqb, heads);
+        auto go = keys ? (causal ? k_attn_fwd<DP, DS, DT, true, OUT16, SPLIT, true> : k_attn_fwd<DP, DS, DT, false, OUT16, SPLIT, true>)
+                       : (causal ? k_attn_fwd<DP, DS, DT, true, OUT16, SPLIT, false> : k_attn_fwd<DP, DS, DT, false, OUT16, SPLIT, false>);
+        go<<<(unsigned)(keys ? nwg : nblk), keys ? 64 * kKeyWaves : kThreads, 0, stream()>>>(
+            q, tiles, exps, out, (int)Sq, (int)Skv, (int)inner, (int)d, heads / kv_heads, kv_heads, (int)ntiles, c2, qvec,
+            (int)(keys ? nq32 : nqb), heads);
     };
     using std::integral_constant;
     if constexpr (DP == 64) {
