@@ -35,6 +35,7 @@
 // v_mfma_f32_32x32x16_f16: lane l holds row l % 32 of A and of B, k (l / 32) * 8 .. + 7;
 // result column l % 32, rows (i / 4) * 8 + (l / 32) * 4 + i % 4.
 #include <algorithm>
+#include <type_traits>
 
 #include "sdh_internal.hpp"
 
@@ -448,6 +449,72 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     const int mt = grp * 8 + in % gm, nt = in / gm;
     const int m0 = mt * BM, n0 = nt * BN;
 
+    // this lane's source row in each of the wave's loads; rows past the matrix
+    // read its last row (their results are not stored)
+    const int lr = lane >> 3;
+    int va[AI], vb[BI];
+    int iy0[CONV ? BI : 1], ix0[CONV ? BI : 1];
+#pragma unroll
+    for (int j = 0; j < AI; ++j) {
+        const int r = (w * AI + j) * 8 + lr;
+        va[j] = min(m0 + r, p.M - 1) * p.rowA + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
+#pragma unroll
+    for (int j = 0; j < BI; ++j) {
+        const int r = (w * BI + j) * 8 + lr, col = min(n0 + r, p.N - 1);
+        const int chunk = ((lane & 7) ^ ((r >> 1) & 7)) << 4;
+        if constexpr (CONV) {
+            const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
+            iy0[j] = oy * p.stride - p.pad;
+            ix0[j] = ox * p.stride - p.pad;
+            vb[j] = (n * p.H * p.W + iy0[j] * p.W + ix0[j]) * kRowBytes + chunk;  // may lie before the sample
+        } else {
+            vb[j] = col * kRowBytes + chunk;
+        }
+    }
+    const int bytesA = (p.M - 1) * p.rowA + kRowBytes, bytesB = (CONV ? p.zero + 1 : p.N) * kRowBytes;
+    // this part's steps, and the one whose stage is issued next: its planes and
+    // (conv2d) its tap, counted on without divisions
+    const int s0 = (int)((int64_t)p.steps * z / p.splits), s1 = (int)((int64_t)p.steps * (z + 1) / p.splits);
+    int left = s1 - s0, ky = 0, kx = 0;  // steps not issued yet
+    const char* pa = (const char*)p.A + s0 * p.planeA;
+    const char* pb = (const char*)p.B + (CONV ? s0 / p.taps : s0) * p.planeB;
+    if (CONV) {
+        const int tap = s0 % p.taps;
+        ky = tap / p.kw;
+        kx = tap - ky * p.kw;
+    }
+    int src[BI];  // the next stage's offsets into B's plane
+    auto aim = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < BI; ++j) {
+            src[j] = vb[j];
+            if constexpr (CONV) {
+                const bool ok = (unsigned)(iy0[j] + ky) < (unsigned)p.H && (unsigned)(ix0[j] + kx) < (unsigned)p.W;
+                const int pad = p.zero * kRowBytes + (vb[j] & 127), at = vb[j] + (ky * p.W + kx) * kRowBytes;
+                src[j] = pad + ((at - pad) & -(int)ok);
+            }
+        }
+    };
+    auto issue = [&](u16* dA, u16* dB) __attribute__((always_inline)) {
+        load_lds<AI>(pa, bytesA, va, dA + w * AI * 512);
+        load_lds<BI>(pb, bytesB, src, dB + w * BI * 512);
+        --left;
+        pa += p.planeA;
+        if (!CONV) {
+            pb += p.planeB;
+        } else if (++kx == p.kw) {
+            kx = 0;
+            if (++ky == p.kh) {
+                ky = 0;
+                pb += p.planeB;
+            }
+        }
+    };
+    // the first stage is on its way while the tile's rows and columns are looked at
+    aim();
+    issue(sA0, sB0);
+
     // rows and columns that need the fp32 path
     bool bad = false;
     for (int i = t; i < BM; i += T) {
@@ -475,7 +542,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
             bad |= e == kBad;
         }
     }
-    if (__syncthreads_or(bad)) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (__syncthreads_or(bad)) {  // the first stage is in LDS behind this
         if (z == 0) {
             if (p.splits > 1 && t == 0) p.slow[lt] = 1;
             for (int i = t; i < BM * BN; i += T) {
@@ -486,50 +554,6 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
         return;
     }
     if (p.splits > 1 && z == 0 && t == 0) p.slow[lt] = 0;
-
-    // this lane's source row in each of the wave's loads; rows past the matrix
-    // read its last row (their results are not stored)
-    const int lr = lane >> 3;
-    int va[AI], vb[BI];
-    int iy0[CONV ? BI : 1], ix0[CONV ? BI : 1];
-#pragma unroll
-    for (int j = 0; j < AI; ++j) {
-        const int r = (w * AI + j) * 8 + lr;
-        va[j] = min(m0 + r, p.M - 1) * p.rowA + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
-    }
-#pragma unroll
-    for (int j = 0; j < BI; ++j) {
-        const int r = (w * BI + j) * 8 + lr, col = min(n0 + r, p.N - 1);
-        const int chunk = ((lane & 7) ^ ((r >> 1) & 7)) << 4;
-        if constexpr (CONV) {
-            const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
-            iy0[j] = oy * p.stride - p.pad;
-            ix0[j] = ox * p.stride - p.pad;
-            vb[j] = (n * p.H * p.W + iy0[j] * p.W + ix0[j]) * kRowBytes + chunk;  // may lie before the sample
-        } else {
-            vb[j] = col * kRowBytes + chunk;
-        }
-    }
-    const int bytesA = (p.M - 1) * p.rowA + kRowBytes, bytesB = (CONV ? p.zero + 1 : p.N) * kRowBytes;
-    auto issue = [&](int step, u16* dA, u16* dB) __attribute__((always_inline)) {
-        int chunk = step, tap = 0;
-        if constexpr (CONV) {
-            chunk = step / p.taps;
-            tap = step - chunk * p.taps;
-        }
-        load_lds<AI>((const char*)p.A + step * p.planeA, bytesA, va, dA + w * AI * 512);
-        int v[BI];
-        const int ky = CONV ? tap / p.kw : 0, kx = tap - ky * (CONV ? p.kw : 0);
-#pragma unroll
-        for (int j = 0; j < BI; ++j) {
-            v[j] = vb[j];
-            if constexpr (CONV) {
-                const bool ok = (unsigned)(iy0[j] + ky) < (unsigned)p.H && (unsigned)(ix0[j] + kx) < (unsigned)p.W;
-                v[j] = ok ? v[j] + (ky * p.W + kx) * kRowBytes : p.zero * kRowBytes + (v[j] & 127);
-            }
-        }
-        load_lds<BI>((const char*)p.B + chunk * p.planeB, bytesB, v, dB + w * BI * 512);
-    };
 
     f32x16 acc[RA][RB];
 #pragma unroll
@@ -547,71 +571,92 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int l = 0; l < 2; ++l) at[s][l] = ((s * 2 + l * 4 + fh) ^ ((fr >> 1) & 7)) << 3;
-    // A stage is 2 RA turns (slice of 16 k, 32 rows of A) of 3 RB MFMAs; the
-    // fragments of a turn are read one turn ahead.
-    auto compute = [&](const u16* tA, const u16* tB) __attribute__((always_inline)) {
-        h8 ah[2], al[2], bh[2][RB], bl[2][RB];
-        auto fragA = [&](int i, h8& hi, h8& lo) __attribute__((always_inline)) {
-            hi = *(const h8*)(tA + offA + (i % RA) * 2048 + at[i / RA][0]);
-            lo = *(const h8*)(tA + offA + (i % RA) * 2048 + at[i / RA][1]);
-        };
-        auto fragB = [&](int s, h8* hi, h8* lo) __attribute__((always_inline)) {
+    // A step is 2 RA turns (slice of 16 k, 32 rows of A) of 3 RB MFMAs; the
+    // fragments of a turn are read one turn ahead. Before the last turn's MFMAs,
+    // when every fragment of the step is in registers, the workgroup meets: the
+    // next step's stage has landed, its first fragments are read behind those
+    // MFMAs, and the buffer just read takes the stage STAGES steps on. Not
+    // __syncthreads(), which waits for every copy into LDS.
+    h8 ah[2], al[2], bh[2][RB], bl[2][RB];
+    auto fragA = [&](const u16* tA, int i) __attribute__((always_inline)) {
+        ah[i & 1] = *(const h8*)(tA + offA + (i % RA) * 2048 + at[i / RA][0]);
+        al[i & 1] = *(const h8*)(tA + offA + (i % RA) * 2048 + at[i / RA][1]);
+    };
+    auto fragB = [&](const u16* tB, int s) __attribute__((always_inline)) {
 #pragma unroll
-            for (int b = 0; b < RB; ++b) {
-                hi[b] = *(const h8*)(tB + offB + b * 2048 + at[s][0]);
-                lo[b] = *(const h8*)(tB + offB + b * 2048 + at[s][1]);
-            }
-        };
-        fragB(0, bh[0], bl[0]);
-        fragA(0, ah[0], al[0]);
+        for (int b = 0; b < RB; ++b) {
+            bh[s][b] = *(const h8*)(tB + offB + b * 2048 + at[s][0]);
+            bl[s][b] = *(const h8*)(tB + offB + b * 2048 + at[s][1]);
+        }
+    };
+    // The step's buffers; nA, nB: the next step's. TAIL: among the last steps, where
+    // the next stages may not exist.
+    auto step = [&](auto tail, int s, u16* cA, u16* cB, u16* nA, u16* nB) __attribute__((always_inline)) {
+        constexpr bool TAIL = decltype(tail)::value;
+        constexpr int AHEAD = (STAGES - 2) * (AI + BI);  // loads of the stage after the next one
 #pragma unroll
         for (int i = 0; i < 2 * RA; ++i) {
-            const int s = i / RA, a = i % RA, q = i & 1;
-            if (i + 1 < 2 * RA) fragA(i + 1, ah[q ^ 1], al[q ^ 1]);
-            if (i + 1 == RA) fragB(1, bh[1], bl[1]);
+            const int sl = i / RA, a = i % RA, q = i & 1;
+            if (i + 1 < 2 * RA) {
+                fragA(cA, i + 1);
+                if (i + 1 == RA) fragB(cB, 1);
+            } else if (!TAIL || s + 1 < s1) {
+                const bool more = !TAIL || s + STAGES < s1;
+                if (more) aim();
+                if (!TAIL || s + 2 < s1)
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(AHEAD) : "memory");
+                else
+                    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                if (more) issue(cA, cB);
+                fragA(nA, 0);
+                fragB(nB, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int b = 0; b < RB; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[q], bh[s][b], acc[a][b], 0, 0, 0);
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[q], bh[sl][b], acc[a][b], 0, 0, 0);
 #pragma unroll
             for (int b = 0; b < RB; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[q], bl[s][b], acc[a][b], 0, 0, 0);
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[q], bl[sl][b], acc[a][b], 0, 0, 0);
 #pragma unroll
             for (int b = 0; b < RB; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[q], bh[s][b], acc[a][b], 0, 0, 0);
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[q], bh[sl][b], acc[a][b], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-
-    // this part's steps
-    const int s0 = (int)((int64_t)p.steps * z / p.splits), s1 = (int)((int64_t)p.steps * (z + 1) / p.splits);
-    // One step: its stage has landed and every wave is past the buffer that the
-    // step STAGES - 1 ahead now goes to (past the end: the last step again, so
-    // that the count of loads in flight stays the same), then its products.
-    auto turn = [&](int s, u16* cA, u16* cB, u16* nA, u16* nB) __attribute__((always_inline)) {
-        // not __syncthreads(), which waits for every copy into LDS
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * (AI + BI)) : "memory");
-        issue(min(s + STAGES - 1, s1 - 1), nA, nB);
-        compute(cA, cB);
-    };
-    issue(s0, sA0, sB0);
-    if (STAGES == 3) issue(min(s0 + 1, s1 - 1), sA1, sB1);
-    int s = s0;
-    if constexpr (STAGES == 3) {
-        for (; s + 3 <= s1; s += 3) {
-            turn(s, sA0, sB0, sA2, sB2);
-            turn(s + 1, sA1, sB1, sA0, sB0);
-            turn(s + 2, sA2, sB2, sA1, sB1);
-        }
-        if (s < s1) turn(s, sA0, sB0, sA2, sB2);
-        if (s + 1 < s1) turn(s + 1, sA1, sB1, sA0, sB0);
-    } else {
-        for (; s + 2 <= s1; s += 2) {
-            turn(s, sA0, sB0, sA1, sB1);
-            turn(s + 1, sA1, sB1, sA0, sB0);
-        }
-        if (s < s1) turn(s, sA0, sB0, sA1, sB1);
+    if (left > 0) {
+        aim();
+        issue(sA1, sB1);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing is on its way into LDS when the workgroup ends
+    if (STAGES == 3 && left > 0) {
+        aim();
+        issue(sA2, sB2);
+    }
+    fragA(sA0, 0);
+    fragB(sB0, 0);
+    int s = s0;
+    std::false_type body;
+    std::true_type tail;
+    if constexpr (STAGES == 3) {
+        for (; s + 6 <= s1; s += 3) {
+            step(body, s, sA0, sB0, sA1, sB1);
+            step(body, s, sA1, sB1, sA2, sB2);
+            step(body, s, sA2, sB2, sA0, sB0);
+        }
+        step(tail, s, sA0, sB0, sA1, sB1);
+        if (s + 1 < s1) step(tail, s + 1, sA1, sB1, sA2, sB2);
+        if (s + 2 < s1) step(tail, s + 2, sA2, sB2, sA0, sB0);
+        if (s + 3 < s1) step(tail, s + 3, sA0, sB0, sA1, sB1);
+        if (s + 4 < s1) step(tail, s + 4, sA1, sB1, sA2, sB2);
+    } else {
+        for (; s + 4 <= s1; s += 2) {
+            step(body, s, sA0, sB0, sA1, sB1);
+            step(body, s, sA1, sB1, sA0, sB0);
+        }
+        step(tail, s, sA0, sB0, sA1, sB1);
+        if (s + 1 < s1) step(tail, s + 1, sA1, sB1, sA0, sB0);
+        if (s + 2 < s1) step(tail, s + 2, sA0, sB0, sA1, sB1);
+    }
 
     if (p.splits > 1) {
         float* o = p.part + ((int64_t)z * p.tm * BM + m0 + wm * WM) * ((int64_t)p.tn * BN) + n0 + wn * WN + fr;
