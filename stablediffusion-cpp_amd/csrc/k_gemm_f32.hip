@@ -122,14 +122,15 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     const bool lt = K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) &&
                     aligned(C, 16) && (!bias || aligned(bias, 16));
     // Split operands from the size where their pack and second launch pay
-    // (MI355X, us, the library's fp32 GEMM in front): [4096,512] x [512,512] 22.8 /
-    // 22.2 alone and 5 us more among other calls, [512,1280] x [1280,1280] 21.9 /
-    // 28.8, [64,1280] x [10240,1280] 25 / 38, [512,640] x [5120,640] 42 / 32,
-    // [256,1280] x [10240,1280] 69 / 49, [8192,320] x [2560,320] 131 / 65,
-    // [4224,2560] x [3840,2560] 610 / 238. Operands that the library path does not
-    // take: from the size where the kernel below is slower ([130,33] x [70,33]
-    // 8.6 / 9.3, [257,321] x [300,321] 31.6 / 10.8).
-    const bool large = 2.0 * (double)M * (double)N * (double)K >= 3e9 && M >= 128 && N >= 128;
+    // (MI355X, us, the library's fp32 GEMM in front): [512,640] x [5120,640] 42 / 32,
+    // [256,1280] x [10240,1280] 69 / 49, [8192,320] x [2560,320] 131 / 63,
+    // [4224,2560] x [3840,2560] 610 / 238; below 3 GFLOP only tall ones, whose packed
+    // weights many rows share: [4096,512] x [512,512] equal, [4800,512] x [512,512] 36 /
+    // 21, but [330,640] x [5120,640] 26 / 33, [512,1280] x [1280,1280] 22 / 29. Operands
+    // that the library path does not take: from the size where the kernel below
+    // is slower ([130,33] x [70,33] 8.6 / 9.3, [257,321] x [300,321] 31.6 / 10.8).
+    const double flops = 2.0 * (double)M * (double)N * (double)K;
+    const bool large = M >= 128 && N >= 128 && (flops >= 3e9 || (flops >= 2e9 && M >= 1024));
     if (K > 0 && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
         split_gemm(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
         launched(op);
