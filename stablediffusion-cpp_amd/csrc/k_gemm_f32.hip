@@ -122,15 +122,18 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     const bool lt = K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) &&
                     aligned(C, 16) && (!bias || aligned(bias, 16));
     // Split operands from the size where their pack and second launch pay
-    // (MI355X, us, the library's fp32 GEMM in front): [512,640] x [5120,640] 42 / 32,
-    // [256,1280] x [10240,1280] 69 / 49, [8192,320] x [2560,320] 131 / 63,
-    // [4224,2560] x [3840,2560] 610 / 238; below 3 GFLOP only tall ones, whose packed
-    // weights many rows share: [4096,512] x [512,512] equal, [4800,512] x [512,512] 36 /
-    // 21, but [330,640] x [5120,640] 26 / 33, [512,1280] x [1280,1280] 22 / 29. Operands
-    // that the library path does not take: from the size where the kernel below
-    // is slower ([130,33] x [70,33] 8.6 / 9.3, [257,321] x [300,321] 31.6 / 10.8).
+    // (MI355X, us, the library's fp32 GEMM in front): [512,640] x [5120,640] 36 / 31,
+    // [256,2560] x [3840,2560] 44 / 42, [256,1280] x [4608,1280] 41 / 27, [8192,320] x
+    // [2560,320] 107 / 67, [4224,2560] x [3840,2560] 583 / 231; with fewer rows the
+    // weights' pack is not won back ([231,2560] x [3840,2560] 41 / 43). From 2.4 GFLOP
+    // only tall ones, whose packed weights many rows share: [6400,320] x [640,320]
+    // 24.5 / 23.9, [2400,512] x [1024,512] 35 / 21, [4800,512] x [512,512] 36 / 23 to 29;
+    // below, [4096,512] x [512,512] 19.5 / 21.4, [1024,1024] x [1024,1024] 18.8 / 22.8,
+    // [330,640] x [5120,640] 23 / 28. Operands that the library path does not take: from
+    // the size where the kernel below is slower ([130,33] x [70,33] 8.6 / 9.3, [257,321] x
+    // [300,321] 31.6 / 10.8).
     const double flops = 2.0 * (double)M * (double)N * (double)K;
-    const bool large = M >= 128 && N >= 128 && (flops >= 3e9 || (flops >= 2e9 && M >= 1024));
+    const bool large = N >= 128 && ((flops >= 3e9 && M >= 256) || (flops >= 2.4e9 && M >= 2048));
     if (K > 0 && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
         split_gemm(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
         launched(op);
