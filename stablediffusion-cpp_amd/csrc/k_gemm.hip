@@ -7,8 +7,9 @@
 // hipBLASLt (bf16 x bf16 -> fp32 with the bias epilogue, the library GEMM,
 // measured 1.35-1.83 PFLOP/s at the Z-Image shapes against 0.88 for the
 // kernels below) whenever the operands are 16-B aligned with aligned leading
-// dimensions; for SwiGLU as two GEMMs into scratch and the elementwise
-// kernel. The hand-written MFMA kernels below cover the other shapes.
+// dimensions. SwiGLU of a short K runs on the main kernel below while its tiles fit
+// the chip at once (the rule stands at the dispatch), else as two library GEMMs into
+// scratch and the elementwise kernel. The kernels below cover the other shapes.
 //
 // Numerics are the reference GPU path's (backend_cuda.cu:236-238, :466-479):
 // A is rounded to bf16 (nearest even; inf/NaN truncated) once per call into
@@ -491,11 +492,23 @@ void run_gemm(const char* op, int64_t M, int64_t N, int64_t K, const float* A, i
                       (EPI != E_SWIGLU || aligned(B1, 16)) && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31);
     if (fast) {
         // hipBLASLt takes the plain GEMM when the operands are 16-B aligned with
-        // aligned leading dimensions; SwiGLU then runs as two GEMMs into scratch
-        // and the elementwise kernel (faster than the fused kernel below, which
-        // stays for the shapes hipBLASLt has no algorithm for)
+        // aligned leading dimensions. SwiGLU with a short K % 64 == 0 runs in one launch
+        // of k_gemm_dl while its tiles (256 rows x 64 hidden) all run at once: the
+        // library's way has two GEMMs and a third launch, 29 us at least. Whole call on
+        // MI355X, us, library / k_gemm_dl, the same bits:
+        //   rows   W1 [512,256]  [1408,512]  [2816,1024]
+        //     64    29.5 / 11      29 / 14
+        //    256    28.7 / 13 (200)           29 / 22
+        //    512    29.3 / 13 (700) 30 / 16   32 / 23
+        //   1024                              40 / 25
+        //   4608    31.7 / 16
+        // With W1 [10240,3840] it gains only while the weights are cached from the call
+        // before (182 rows and the projection back, fresh weights: 124 / 123), and few
+        // tiles of a long K lose (W1 [1536,5120] at 256 rows: 41 / 75).
         const bool lt = ldb % 8 == 0 && ldc % 4 == 0 && aligned(C, 16) && (!bias || aligned(bias, 16));
-        const bool swi_lt = EPI == E_SWIGLU && lt && ldc == N;
+        const int64_t tiles = ((M + kDM - 1) / kDM) * ((N + kDN / 2 - 1) / (kDN / 2));
+        const bool one = EPI == E_SWIGLU && K % 64 == 0 && K <= 1024 && tiles <= num_cus();
+        const bool swi_lt = EPI == E_SWIGLU && lt && ldc == N && !one;
         const size_t pbytes = ((size_t)(M * K) * 2 + 255) / 256 * 256, gbytes = (size_t)(M * N) * 4;
         char* base = (char*)scratch(pbytes + (swi_lt ? 2 * gbytes : 0));
         u16* P = (u16*)base;
