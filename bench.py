@@ -728,15 +728,15 @@ class AttentionVAE(Workload):
     """The VAE decoder's mid-block attention (VAEAttention, modules.cpp:133-141:
     one head over the 512 channels, tokens = the latent's pixels) at the FLUX
     VAE's 1024x1024 decode: q k v [1, 16384, 512] fp32. Head dimensions above
-    128 on long sequences take the score-matrix route on the fp32 library GEMM
-    (score blocks, the row softmax, a GEMM against v^T), so the rate is quoted
-    against the 157.3 TFLOP/s fp32 MFMA peak. Parity: the reference's
+    128 with more than 64 keys take the score-matrix route on split operands
+    (score blocks, the row softmax, a product against v^T), three fp16 products
+    per fp32 product, which pct_mfma_peak counts. Parity: the reference's
     attention on the same arrays, abs 1e-4."""
 
-    name, kernel = "attention_vae", "Cijk"
+    name, kernel = "attention_vae", "k_split_mm"
     S, d = 16384, 512
     flops = 4 * 16384 * 16384 * 512
-    mfma_peak = (157.3, "157.3 TF fp32")
+    mfma_mult = 3
     algo_bytes = 4 * 16384 * 512 * 4
     cpu_time = False
     desc = "VAE mid-block attention, q k v [1,16384,512] fp32, one head (FLUX VAE decode at 1024x1024)"

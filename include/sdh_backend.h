@@ -226,7 +226,8 @@ int sdh_swiglu_bf16(const float* gate, const float* up, uint16_t* y, int64_t n);
  * out = softmax(q k^T / sqrt(d)) v per head, query head h reading key/value
  * head h / (heads / kv_heads); causal keeps keys 0..i for query i.
  * kv_heads <= 0 means kv_heads = heads. out must not overlap the inputs.
- * Fused on the MFMA units (no score matrix in memory) for d <= 128. */
+ * Fused on the MFMA units (no score matrix in memory) for d <= 128; above, with
+ * more than 64 keys, blocks of the score matrix in library scratch. */
 int sdh_attention(const float* q, const float* k, const float* v, float* out, int64_t N, int64_t Sq, int64_t Skv,
                   int heads, int kv_heads, int64_t d, int causal);
 /* FUSED: out = bf16 bits of attention(q, k, v): sdh_attention then the bf16
@@ -257,7 +258,7 @@ int sdh_qknorm_rope_attention(float* q, const float* k, const float* v, void* ou
  * accumulation and softmax statistics. A third of sdh_attention's MFMA work
  * and half its packed bytes; the error is that of fp16 operands (about 2^-12
  * relative per element), for callers whose tolerance allows it (a diffusion
- * step's 2e-2). Head dimensions above 128 run the fp32 kernel. */
+ * step's 2e-2). Head dimensions above 128 run as sdh_attention's. */
 int sdh_attention_fp16(const float* q, const float* k, const float* v, void* out, int out_bf16, int64_t N,
                        int64_t Sq, int64_t Skv, int heads, int kv_heads, int64_t d, int causal);
 
