@@ -10,7 +10,8 @@
 // [Cout, Cin, kh, kw] weight's own order, so the weight is already a [Cout, K]
 // matrix); then out[Cout, pixels] = W cols^T through sdh_gemm_nt_f32, written
 // straight into the NCHW output (ldc = Ho * Wo); the bias is added per output
-// channel after the last chunk (sdh_add_channel_bias).
+// channel after the last chunk (sdh_add_channel_bias). The patches hold the
+// scratch block meanwhile, so the product takes one of its routes without scratch.
 #include <algorithm>
 
 #include "sdh_backend.h"

@@ -20,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "arena.hpp"
 #include "sdh_internal.hpp"
 
 namespace sdh {
@@ -28,12 +29,9 @@ namespace {
 
 thread_local std::string t_last_error;
 
-constexpr size_t kAlign = 256;
 constexpr size_t kStageBytes = 8u << 20;  // per staging buffer
 constexpr int kTimerSlots = 16;
 constexpr size_t kUncachedWords = 64u << 10;  // 256 KiB
-
-size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 size_t env_mb(const char* name, size_t dflt) {
     const char* e = std::getenv(name);
@@ -43,111 +41,14 @@ size_t env_mb(const char* name, size_t dflt) {
     return (end && *end == 0) ? (size_t)v << 20 : dflt;
 }
 
-// Arena: segments of device memory; free ranges indexed by address (for
-// coalescing) and by size (for best fit). Blocks never span segments.
-struct Arena {
-    struct Seg {
-        uintptr_t base;
-        size_t bytes;
-    };
-    std::vector<Seg> segs;
-    std::map<uintptr_t, size_t> free_by_addr;          // addr -> size
-    std::multimap<size_t, uintptr_t> free_by_size;     // size -> addr
-    std::map<uintptr_t, size_t> live;                  // addr -> rounded size
-    std::map<uintptr_t, size_t> requested;             // addr -> bytes asked for
-    size_t reserved = 0, in_use = 0, limit = 0;        // limit 0 = none
-
-    int seg_of(uintptr_t a) const {
-        for (size_t i = 0; i < segs.size(); ++i)
-            if (a >= segs[i].base && a < segs[i].base + segs[i].bytes) return (int)i;
-        return -1;
-    }
-    void erase_free(uintptr_t a, size_t sz) {
-        free_by_addr.erase(a);
-        auto r = free_by_size.equal_range(sz);
-        for (auto it = r.first; it != r.second; ++it)
-            if (it->second == a) {
-                free_by_size.erase(it);
-                return;
-            }
-    }
-    void insert_free(uintptr_t a, size_t sz) {
-        // coalesce with neighbours inside the same segment
-        const int s = seg_of(a);
-        auto next = free_by_addr.lower_bound(a);
-        if (next != free_by_addr.end() && next->first == a + sz && seg_of(next->first) == s) {
-            const uintptr_t na = next->first;
-            const size_t nsz = next->second;
-            erase_free(na, nsz);
-            sz += nsz;
-        }
-        auto prev = free_by_addr.lower_bound(a);
-        if (prev != free_by_addr.begin()) {
-            --prev;
-            if (prev->first + prev->second == a && seg_of(prev->first) == s) {
-                const uintptr_t pa = prev->first;
-                const size_t psz = prev->second;
-                erase_free(pa, psz);
-                a = pa;
-                sz += psz;
-            }
-        }
-        free_by_addr[a] = sz;
-        free_by_size.emplace(sz, a);
-    }
-    bool grow(size_t need) {
-        size_t bytes = round_up(std::max(need, (size_t)256 << 20), (size_t)2 << 20);
-        if (limit && reserved + bytes > limit) {
-            if (reserved + round_up(need, (size_t)2 << 20) > limit) return false;
-            bytes = round_up(need, (size_t)2 << 20);
-        }
-        void* p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess || !p) {
-            (void)hipGetLastError();
-            return false;
-        }
-        segs.push_back({(uintptr_t)p, bytes});
-        reserved += bytes;
-        insert_free((uintptr_t)p, bytes);
-        return true;
-    }
-    void* alloc(size_t bytes) {
-        const size_t sz = round_up(bytes, kAlign);
-        auto it = free_by_size.lower_bound(sz);
-        if (it == free_by_size.end()) {
-            if (!grow(sz)) return nullptr;
-            it = free_by_size.lower_bound(sz);
-            if (it == free_by_size.end()) return nullptr;
-        }
-        const uintptr_t a = it->second;
-        const size_t fsz = it->first;
-        erase_free(a, fsz);
-        if (fsz > sz) insert_free(a + sz, fsz - sz);
-        live[a] = sz;
-        requested[a] = bytes;
-        in_use += sz;
-        return (void*)a;
-    }
-    bool release(void* p) {
-        auto it = live.find((uintptr_t)p);
-        if (it == live.end()) return false;
-        const size_t sz = it->second;
-        live.erase(it);
-        requested.erase((uintptr_t)p);
-        in_use -= sz;
-        insert_free((uintptr_t)p, sz);
-        return true;
-    }
-    void clear() {
-        for (auto& s : segs) (void)hipFree((void*)s.base);
-        segs.clear();
-        free_by_addr.clear();
-        free_by_size.clear();
-        live.clear();
-        requested.clear();
-        reserved = in_use = 0;
-    }
-};
+void* hip_reserve(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess && p) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+void hip_unreserve(void* p) { (void)hipFree(p); }
+void wait_for_stream();
 
 struct Runtime {
     std::mutex mu;
@@ -158,18 +59,12 @@ struct Runtime {
     size_t total_mem = 0;
     int cus = 0;
     hipStream_t stream = nullptr;
-    Arena arena;
+    Arena arena{hip_reserve, hip_unreserve};
     void* stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     hipEvent_t timers[kTimerSlots] = {};
     std::map<uintptr_t, size_t> external;
-    void* scratch = nullptr;
-    size_t scratch_bytes = 0;
-    // Scratch blocks that grew out of use while captured graphs were alive: a
-    // graph keeps the pointers it was captured with, so they are given back
-    // only when the last graph is destroyed.
-    std::vector<void*> retired_scratch;
-    int live_graphs = 0;
+    Scratch scratch{arena, wait_for_stream};
     unsigned* counters = nullptr;
     size_t counter_count = 0;
     void* workspace = nullptr;
@@ -188,6 +83,8 @@ struct Runtime {
     // recorded into a graph, so nothing may wait on it or grow a buffer
     // that queued work could still be reading.
     bool capturing = false;
+    // Entry points open on the thread that holds op_mutex (OpScope).
+    int op_depth = 0;
     // Incremented by every sdh_capture_begin (capture_generation).
     unsigned capture_gen = 0;
     // Uncached device words for cross-workgroup exchange polled through the
@@ -206,6 +103,8 @@ Runtime& rt() {
     static Runtime r;
     return r;
 }
+
+void wait_for_stream() { hip_check(hipStreamSynchronize(rt().stream), "hipStreamSynchronize"); }
 
 }  // namespace
 
@@ -379,54 +278,26 @@ void check_range(const void* p, size_t bytes, const char* op, const char* what) 
     range_check_locked(r, p, bytes, op, what);
 }
 
-namespace {
-
-// Returns the scratch block to an exhausted arena (the next op that needs
-// scratch asks for it again); false where there is none or a graph holds it.
-bool give_back_scratch_locked(Runtime& r) {
-    if (!r.scratch || r.capturing || r.live_graphs > 0) return false;
-    hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
-    r.arena.release(r.scratch);
-    r.scratch = nullptr;
-    r.scratch_bytes = 0;
-    return true;
-}
-
-// Replaces the scratch block by one of at least `bytes`; false when the arena
-// cannot hold it (there is then no scratch block).
-bool grow_scratch_locked(Runtime& r, size_t bytes) {
-    if (r.scratch) {
-        if (r.live_graphs > 0) {
-            r.retired_scratch.push_back(r.scratch);
-        } else {
-            // Work queued earlier may still read the old scratch.
-            hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
-            r.arena.release(r.scratch);
-        }
-    }
-    r.scratch_bytes = round_up(std::max(bytes, (size_t)1 << 20), kAlign);
-    r.scratch = r.arena.alloc(r.scratch_bytes);
-    if (!r.scratch) r.scratch_bytes = 0;
-    return r.scratch != nullptr;
-}
-
-}  // namespace
-
 void* scratch(size_t bytes) {
     Runtime& r = rt();
     std::lock_guard<std::mutex> lk(r.mu);
-    if (bytes > r.scratch_bytes) {
-        not_capturing_locked(r, "backend_hip scratch");
-        if (!grow_scratch_locked(r, bytes)) fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating scratch");
-    }
-    return r.scratch;
+    const Scratch::Answer a = r.scratch.take(bytes, r.capturing);
+    if (a == Scratch::kCapturing) not_capturing_locked(r, "backend_hip scratch");
+    if (a == Scratch::kFull) fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating scratch");
+    if (a == Scratch::kHeld) fail(SDH_ERR_HIP, "backend_hip: internal: an op asked for scratch twice");
+    return r.scratch.block;
 }
 
 void* try_scratch(size_t bytes) {
     Runtime& r = rt();
     std::lock_guard<std::mutex> lk(r.mu);
-    if (bytes > r.scratch_bytes && (r.capturing || !grow_scratch_locked(r, bytes))) return nullptr;
-    return r.scratch;
+    return r.scratch.take(bytes, r.capturing) == Scratch::kHave ? r.scratch.block : nullptr;
+}
+
+OpScope::OpScope() { ++rt().op_depth; }
+OpScope::~OpScope() {
+    Runtime& r = rt();
+    if (--r.op_depth == 0) r.scratch.end_op();
 }
 
 void* workspace(size_t bytes) {
@@ -440,7 +311,7 @@ void* workspace(size_t bytes) {
         }
         r.workspace_bytes = round_up(bytes, kAlign);
         r.workspace = r.arena.alloc(r.workspace_bytes);
-        if (!r.workspace && give_back_scratch_locked(r)) r.workspace = r.arena.alloc(r.workspace_bytes);
+        if (!r.workspace && r.scratch.give_back(r.capturing)) r.workspace = r.arena.alloc(r.workspace_bytes);
         if (!r.workspace) {
             r.workspace_bytes = 0;
             fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating the GEMM workspace");
@@ -565,9 +436,7 @@ int sdh_shutdown(void) {
         hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
         r.arena.clear();
         r.external.clear();
-        r.scratch = nullptr;
-        r.scratch_bytes = 0;
-        r.retired_scratch.clear();
+        r.scratch.clear();
         r.counters = nullptr;
         r.counter_count = 0;
         r.ones = nullptr;
@@ -596,7 +465,7 @@ int sdh_malloc(size_t bytes, void** out) {
         Runtime& r = rt();
         std::lock_guard<std::mutex> lk(r.mu);
         void* p = r.arena.alloc(bytes);
-        if (!p && give_back_scratch_locked(r)) p = r.arena.alloc(bytes);
+        if (!p && r.scratch.give_back(r.capturing)) p = r.arena.alloc(bytes);
         if (!p)
             fail(SDH_ERR_OOM, "sdh_malloc: arena exhausted (" + std::to_string(bytes) + " bytes requested, " +
                                   std::to_string(r.arena.in_use) + " in use, " + std::to_string(r.arena.reserved) +
@@ -781,7 +650,7 @@ int sdh_capture_end(void** graph) {
         const hipError_t ie = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         hip_check(ie, "hipGraphInstantiate");
-        ++r.live_graphs;
+        r.scratch.graph_made();
         *graph = (void*)e;
     });
 }
@@ -806,10 +675,7 @@ int sdh_graph_destroy(void* graph) {
         // a launch of it may still be queued
         hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
         hip_check(hipGraphExecDestroy((hipGraphExec_t)graph), "hipGraphExecDestroy");
-        if (--r.live_graphs == 0) {
-            for (void* p : r.retired_scratch) r.arena.release(p);
-            r.retired_scratch.clear();
-        }
+        r.scratch.graph_gone();
     });
 }
 

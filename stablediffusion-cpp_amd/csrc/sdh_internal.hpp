@@ -34,10 +34,17 @@ void set_last_error(const char* msg);
 // attention, the bf16 GEMM's packed A, conv2d) cannot interleave with
 // another thread's. Recursive: entry points call entry points.
 std::recursive_mutex& op_mutex();
+// An entry point's extent, entered with op_mutex held; the end of the
+// outermost one ends the op's hold on the scratch block.
+struct OpScope {
+    OpScope();
+    ~OpScope();
+};
 
 template <class F>
 int guarded(F&& f) noexcept {
     std::lock_guard<std::recursive_mutex> lk(op_mutex());
+    OpScope scope;
     try {
         f();
         set_last_error("");
@@ -74,11 +81,14 @@ int num_cus();
 // Throws SDH_ERR_INVALID unless [p, p + bytes) lies inside one live arena
 // block or one registered external range. `what` names the argument.
 void check_range(const void* p, size_t bytes, const char* op, const char* what);
-// Per-call device scratch of at least `bytes`, owned by the library, valid
-// until the next call that asks for scratch (ops are serialised on one stream).
+// Per-call device scratch of at least `bytes`, owned by the library and held by
+// the op until its (outermost) entry point ends; ops are serialised on one
+// stream. There is one block: an op asks once, and a second request inside it,
+// also by an entry point that it calls, is an error.
 void* scratch(size_t bytes);
 // As scratch, but null instead of an error where the arena cannot hold that
-// much, or where the block would have to grow during a capture.
+// much, where the block would have to grow during a capture, or where the op
+// holds it already: the caller then takes a route without scratch.
 void* try_scratch(size_t bytes);
 // A persistent library-owned device block of at least `bytes` for a library
 // routine's workspace (the BLAS GEMM), distinct from scratch().
