@@ -311,7 +311,6 @@ void* workspace(size_t bytes) {
         }
         r.workspace_bytes = round_up(bytes, kAlign);
         r.workspace = r.arena.alloc(r.workspace_bytes);
-        if (!r.workspace && r.scratch.give_back(r.capturing)) r.workspace = r.arena.alloc(r.workspace_bytes);
         if (!r.workspace) {
             r.workspace_bytes = 0;
             fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating the GEMM workspace");

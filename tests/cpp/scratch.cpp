@@ -57,10 +57,26 @@ int held() {
     return 0;
 }
 
+// Memory for someone else, inside an op that holds the block: the arena finds
+// none rather than the op's own (the GEMM workspace against the packed input).
+int exhausted() {
+    World w(96 * MB);
+    CHECK(w.s.take(32 * MB, false) == Scratch::kHave);
+    CHECK(!w.arena.alloc(80 * MB));
+    CHECK(!w.s.give_back(false) && !w.arena.alloc(80 * MB));
+    w.s.end_op();
+    CHECK(w.s.give_back(false));  // between ops it is idle
+    void* p = w.arena.alloc(80 * MB);
+    CHECK(p && w.s.take(32 * MB, false) == Scratch::kFull);
+    w.arena.release(p);
+    CHECK(w.s.take(32 * MB, false) == Scratch::kHave);
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-    const std::map<std::string, int (*)()> all = {{"held", held}};
+    const std::map<std::string, int (*)()> all = {{"held", held}, {"exhausted", exhausted}};
     const auto it = all.find(argc > 1 ? argv[1] : "");
     return it == all.end() ? 2 : it->second();
 }
