@@ -6,7 +6,9 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <iterator>
 #include <map>
+#include <set>
 #include <vector>
 
 namespace sdh {
@@ -30,6 +32,7 @@ struct Arena {
     std::map<uintptr_t, size_t> live;                  // addr -> rounded size
     std::map<uintptr_t, size_t> requested;             // addr -> bytes asked for
     size_t reserved = 0, in_use = 0, limit = 0;        // limit 0 = none
+    size_t releases = 0;                               // calls of release that gave a block back
 
     int seg_of(uintptr_t a) const {
         for (size_t i = 0; i < segs.size(); ++i)
@@ -106,8 +109,26 @@ struct Arena {
         live.erase(it);
         requested.erase((uintptr_t)p);
         in_use -= sz;
+        ++releases;
         insert_free((uintptr_t)p, sz);
         return true;
+    }
+    bool has_free(size_t bytes) const { return free_by_size.lower_bound(round_up(bytes, kAlign)) != free_by_size.end(); }
+    // The free range that releasing p would leave.
+    size_t room_around(void* p) const {
+        const auto it = live.find((uintptr_t)p);
+        if (it == live.end()) return 0;
+        const uintptr_t a = it->first;
+        const int s = seg_of(a);
+        size_t n = it->second;
+        auto next = free_by_addr.lower_bound(a);
+        const auto prev = next;
+        if (next != free_by_addr.end() && next->first == a + it->second && seg_of(next->first) == s) n += next->second;
+        if (prev != free_by_addr.begin()) {
+            const auto b = std::prev(prev);
+            if (b->first + b->second == a && seg_of(b->first) == s) n += b->second;
+        }
+        return n;
     }
     void clear() {
         for (auto& s : segs) unreserve((void*)s.base);
@@ -129,22 +150,30 @@ struct Scratch {
     void* block = nullptr;
     size_t bytes = 0;
     bool held = false;
-    // Blocks that grew out of use while captured graphs were alive: a graph
-    // keeps the pointers it was captured with, so they are given back only
-    // when the last graph is destroyed.
+    // A graph keeps the pointers it was captured with: a block that an op asked
+    // for during a capture is replaced, but given back only when the last graph
+    // is destroyed.
+    bool captured = false;
     std::vector<void*> retired;
-    int graphs = 0;
+    std::set<void*> graphs;
+    // The last size that the arena could not hold, and its count of releases
+    // then: until one more, a request that has another route is not tried again.
+    size_t refused = 0, refused_at = 0;
 
     enum Answer { kHave, kHeld, kCapturing, kFull };
 
-    // After kHave `block` holds at least `want` bytes for the op that asks.
-    Answer take(size_t want, bool capturing) {
+    // After kHave `block` holds at least `want` bytes for the op that asks;
+    // after any other answer the block is what it was. `must`: the op has no
+    // route without it.
+    Answer take(size_t want, bool capturing, bool must = true) {
         if (held) return kHeld;
         if (want > bytes) {
             if (capturing) return kCapturing;
+            if (!must && refused && want >= refused && arena.releases == refused_at) return kFull;
             if (!grow(want)) return kFull;
         }
         held = true;
+        captured |= capturing;
         return kHave;
     }
     void end_op() { held = false; }
@@ -153,7 +182,7 @@ struct Scratch {
     // scratch asks for it again); false where there is none, an op holds it
     // or a graph may.
     bool give_back(bool capturing) {
-        if (!block || held || capturing || graphs > 0) return false;
+        if (!block || held || capturing || kept()) return false;
         sync();
         arena.release(block);
         block = nullptr;
@@ -164,34 +193,53 @@ struct Scratch {
     void clear() {
         block = nullptr;
         bytes = 0;
-        held = false;
+        held = captured = false;
         retired.clear();
+        graphs.clear();
+        refused = 0;
     }
 
-    // Replaces the block by one of at least `want` bytes; false when the
-    // arena cannot hold it (there is then no block).
+    // Replaces the block by one of at least `want` bytes; false, and the block
+    // stays, when the arena cannot hold that much. The old block makes room
+    // for the new one only where that is known to be enough, so a refusal
+    // costs no wait and moves nothing: an op whose scratch does not fit asks
+    // on each call and then takes its other route.
     bool grow(size_t want) {
-        if (block) {
-            if (graphs > 0) {
-                retired.push_back(block);
-            } else {
-                // Work queued earlier may still read the old block.
-                sync();
-                arena.release(block);
-            }
+        const size_t size = round_up(std::max(want, (size_t)1 << 20), kAlign);
+        void* old = block;
+        if (old && !kept() && !arena.has_free(size) && arena.room_around(old) >= size) {
+            // work queued earlier may still read the old block
+            sync();
+            arena.release(old);
+            old = nullptr;
         }
-        bytes = round_up(std::max(want, (size_t)1 << 20), kAlign);
-        block = arena.alloc(bytes);
-        if (!block) bytes = 0;
-        return block != nullptr;
+        void* fresh = arena.alloc(size);
+        if (!fresh) {
+            refused = want;
+            refused_at = arena.releases;
+            return false;
+        }
+        if (old && kept()) {
+            retired.push_back(old);
+        } else if (old) {
+            sync();
+            arena.release(old);
+        }
+        block = fresh;
+        bytes = size;
+        captured = false;
+        return true;
     }
 
-    void graph_made() { ++graphs; }
-    void graph_gone() {
-        if (--graphs > 0) return;
+    void graph_made(void* g) { graphs.insert(g); }
+    void graph_gone(void* g) {
+        if (!graphs.erase(g) || !graphs.empty()) return;
         for (void* p : retired) arena.release(p);
         retired.clear();
+        captured = false;
     }
+
+    bool kept() const { return captured && !graphs.empty(); }
 };
 
 }  // namespace sdh

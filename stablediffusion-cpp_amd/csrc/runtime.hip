@@ -291,7 +291,7 @@ void* scratch(size_t bytes) {
 void* try_scratch(size_t bytes) {
     Runtime& r = rt();
     std::lock_guard<std::mutex> lk(r.mu);
-    return r.scratch.take(bytes, r.capturing) == Scratch::kHave ? r.scratch.block : nullptr;
+    return r.scratch.take(bytes, r.capturing, false) == Scratch::kHave ? r.scratch.block : nullptr;
 }
 
 OpScope::OpScope() { ++rt().op_depth; }
@@ -649,7 +649,7 @@ int sdh_capture_end(void** graph) {
         const hipError_t ie = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         hip_check(ie, "hipGraphInstantiate");
-        r.scratch.graph_made();
+        r.scratch.graph_made((void*)e);
         *graph = (void*)e;
     });
 }
@@ -674,7 +674,7 @@ int sdh_graph_destroy(void* graph) {
         // a launch of it may still be queued
         hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
         hip_check(hipGraphExecDestroy((hipGraphExec_t)graph), "hipGraphExecDestroy");
-        r.scratch.graph_gone();
+        r.scratch.graph_gone(graph);
     });
 }
 

@@ -3,7 +3,7 @@ GEMM's scratch cannot be had, in a child process whose arena holds exactly the
 room that the patches need: the product of a chunk at sizes that the fp32
 linear sends to its split operands on its own (many output channels; rows that
 are not a multiple of 16 bytes; a second chunk and a second sample at an
-unaligned place), eagerly and captured. 1x1 kernels, so float64 matrix
+unaligned place), eagerly and captured, and beside a live graph. 1x1 kernels, so float64 matrix
 products on the host are the reference; within the fp32 summation bound."""
 import os
 import subprocess
@@ -88,6 +88,12 @@ for i in range(3):
     be.call('sdh_zero', out.ptr, out.nbytes)
     be.graph_launch(graph)
     check(out.download(), x, w, b, 'captured, replay %%d' %% i)
+used = be.memory_stats()[1]
+for i in range(5):  # with a graph alive: refused again each time, and nothing more held
+    be.call('sdh_zero', out.ptr, out.nbytes)
+    conv(dx, x, dw, w, db, out)
+    check(out.download(), x, w, b, 'beside a graph')
+    assert be.memory_stats()[1] == used
 be.graph_destroy(graph)
 print('gather route ok', flush=True)
 """ % (os.path.join(ROOT, "stablediffusion-cpp_amd"), os.path.join(ROOT, "oracle"), HERE)

@@ -20,7 +20,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["held", "exhausted"])
+@pytest.mark.parametrize("scenario", ["held", "exhausted", "refused", "in_place", "graphs"])
 def test_scratch(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
