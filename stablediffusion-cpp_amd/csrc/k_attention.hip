@@ -1069,6 +1069,7 @@ void run_attention(const float* q, const float* k, const float* v, void* out, bo
         // 244 / 33, [1,2745,512] 2997 / 108, [1,4096,512] 329* / 151, [1,16384,512]
         // 4124* / 1875 (293 TFLOP/s).
         launched(op);
+        reserve_blaslt();
     } else if (!(Sq * Skv >= (int64_t(1) << 18) &&
                  run_attention_gemm(op, q, k, v, out, out16, N, Sq, Skv, heads, kv_heads, d, causal, scale))) {
         const int64_t gx = (Sq + kGenWaves - 1) / kGenWaves;

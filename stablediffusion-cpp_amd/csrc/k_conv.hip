@@ -58,11 +58,13 @@ void run_conv2d(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     check_range(w, (size_t)(Cout * K) * 4, op, "w");
     check_range(out, (size_t)(N * Cout * HW) * 4, op, "out");
     if (bias) check_range(bias, (size_t)Cout * 4, op, "bias");
+    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(HW, kChunkFloats / K));
+    reserve_scratch((size_t)(chunk * K) * 4);
+    reserve_blaslt();
     if (split_conv(x, N, Cin, H, W, w, Cout, kh, kw, bias, stride, pad, out, Ho, Wo)) {
         launched(op);
         return;
     }
-    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(HW, kChunkFloats / K));
     float* cols = (float*)scratch((size_t)(chunk * K) * 4);
     for (int64_t n = 0; n < N; ++n) {
         const float* xn = x + n * Cin * H * W;

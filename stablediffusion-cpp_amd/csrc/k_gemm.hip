@@ -398,11 +398,30 @@ Blas& blas() {
     return b;
 }
 
+// False where hipBLASLt cannot be had. It is not created during a capture, which
+// it answers by ending the process.
+bool blas_handle(Blas& b) {
+    if (!b.tried) {
+        need(!capturing(), "hipBLASLt", "not allowed while the library stream is being captured (sdh_capture_begin); "
+                                        "run the op once before capturing");
+        b.tried = true;
+        if (hipblasLtCreate(&b.h) != HIPBLAS_STATUS_SUCCESS) b.h = nullptr;
+    }
+    return b.h != nullptr;
+}
+
 void blas_check(hipblasStatus_t st, const char* what) {
     if (st != HIPBLAS_STATUS_SUCCESS) fail(SDH_ERR_HIP, std::string(what) + ": hipBLASLt status " + std::to_string((int)st));
 }
 
 }  // namespace
+
+void reserve_blaslt() {
+    if (capturing()) return;
+    Blas& b = blas();
+    std::lock_guard<std::mutex> lk(b.mu);
+    if (blas_handle(b)) (void)try_workspace(kBlasWorkspace);
+}
 
 // C[M,N] = P[M,K] B[N,K]^T (+ bias) (+ C) on hipBLASLt with fp32 accumulation,
 // P and B bf16 (f32 = false) or fp32 (f32 = true; fp32 products). Returns
@@ -412,14 +431,7 @@ bool blaslt_gemm(bool f32, int64_t M, int64_t N, int64_t K, const void* P, int64
                  float* C, int64_t ldc, const float* bias, bool accumulate) {
     Blas& b = blas();
     std::lock_guard<std::mutex> lk(b.mu);
-    if (!b.h) {
-        if (b.tried) return false;
-        b.tried = true;
-        if (hipblasLtCreate(&b.h) != HIPBLAS_STATUS_SUCCESS) {
-            b.h = nullptr;
-            return false;
-        }
-    }
+    if (!blas_handle(b)) return false;
     const auto key = std::make_tuple(M, N, K, ldp, ldb, ldc, bias ? 1 : 0, f32 ? 1 : 0);
     const hipDataType ab = f32 ? HIP_R_32F : HIP_R_16BF;
     auto it = b.plans.find(key);
@@ -484,15 +496,20 @@ void run_gemm(const char* op, int64_t M, int64_t N, int64_t K, const float* A, i
     }
     check_range(C, (size_t)((M - 1) * ldc + N) * 4, op, EPI == E_SWIGLU ? "y" : "C");
     if (bias) check_range(bias, (size_t)N * 4, op, "bias");
-    if (EPI == E_LINEAR && gemv_bf16(M, N, K, A, lda, B0, ldb, C, ldc, bias, accumulate)) {  // a few rows
-        launched(op);
-        return;
-    }
     const bool fast = K > 0 && K % 8 == 0 && lda % 4 == 0 && ldb % 8 == 0 && aligned(A, 16) && aligned(B0, 16) &&
                       (EPI != E_SWIGLU || aligned(B1, 16)) && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31);
+    // hipBLASLt takes the plain GEMM when the operands are 16-B aligned with
+    // aligned leading dimensions
+    const bool lt = fast && ldc % 4 == 0 && aligned(C, 16) && (!bias || aligned(bias, 16));
+    const size_t pbytes = ((size_t)(M * K) * 2 + 255) / 256 * 256, gbytes = (size_t)(M * N) * 4;
+    if (EPI == E_LINEAR && gemv_bf16(M, N, K, A, lda, B0, ldb, C, ldc, bias, accumulate)) {  // a few rows
+        launched(op);
+        if (fast) reserve_scratch(pbytes);
+        if (lt) reserve_blaslt();
+        return;
+    }
     if (fast) {
-        // hipBLASLt takes the plain GEMM when the operands are 16-B aligned with
-        // aligned leading dimensions. SwiGLU with a short K % 64 == 0 runs in one launch
+        // SwiGLU with a short K % 64 == 0 runs in one launch
         // of k_gemm_dl while its tiles (256 rows x 64 hidden) all run at once: the
         // library's way has two GEMMs and a third launch, 29 us at least. Whole call on
         // MI355X, us, library / k_gemm_dl, the same bits:
@@ -505,11 +522,13 @@ void run_gemm(const char* op, int64_t M, int64_t N, int64_t K, const float* A, i
         // With W1 [10240,3840] it gains only while the weights are cached from the call
         // before (182 rows and the projection back, fresh weights: 124 / 123), and few
         // tiles of a long K lose (W1 [1536,5120] at 256 rows: 41 / 75).
-        const bool lt = ldb % 8 == 0 && ldc % 4 == 0 && aligned(C, 16) && (!bias || aligned(bias, 16));
         const int64_t tiles = ((M + kDM - 1) / kDM) * ((N + kDN / 2 - 1) / (kDN / 2));
         const bool one = EPI == E_SWIGLU && K % 64 == 0 && K <= 1024 && tiles <= num_cus();
         const bool swi_lt = EPI == E_SWIGLU && lt && ldc == N && !one;
-        const size_t pbytes = ((size_t)(M * K) * 2 + 255) / 256 * 256, gbytes = (size_t)(M * N) * 4;
+        if (one && lt && ldc == N) {
+            reserve_scratch(pbytes + 2 * gbytes);
+            reserve_blaslt();
+        }
         char* base = (char*)scratch(pbytes + (swi_lt ? 2 * gbytes : 0));
         u16* P = (u16*)base;
         const int64_t kg = K / 8;

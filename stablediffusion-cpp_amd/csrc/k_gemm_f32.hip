@@ -115,12 +115,13 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     }
     check_range(C, (size_t)((M - 1) * ldc + N) * 4, op, "C");
     if (bias) check_range(bias, (size_t)N * 4, op, "bias");
-    if (gemv_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {  // a few rows
-        launched(op);
-        return;
-    }
     const bool lt = K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) &&
                     aligned(C, 16) && (!bias || aligned(bias, 16));
+    if (gemv_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {  // a few rows
+        launched(op);
+        if (lt) reserve_blaslt();
+        return;
+    }
     // Split operands from the size where their pack and second launch pay
     // (MI355X, us, the library's fp32 GEMM in front): [512,640] x [5120,640] 36 / 31,
     // [256,2560] x [3840,2560] 44 / 42, [256,1280] x [4608,1280] 41 / 27, [8192,320] x
@@ -137,6 +138,7 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     if (K > 0 && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
         split_gemm(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
         launched(op);
+        if (lt) reserve_blaslt();
         return;
     }
     // the library GEMM for aligned operands (fp32 products, fp32 accumulation)

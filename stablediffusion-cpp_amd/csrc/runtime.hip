@@ -300,23 +300,35 @@ OpScope::~OpScope() {
     if (--r.op_depth == 0) r.scratch.end_op();
 }
 
-void* workspace(size_t bytes) {
+void reserve_scratch(size_t bytes) {
+    Runtime& r = rt();
+    std::lock_guard<std::mutex> lk(r.mu);
+    if (!r.capturing && r.scratch.take(bytes, false, false) == Scratch::kHave) r.scratch.end_op();
+}
+
+void* try_workspace(size_t bytes) {
     Runtime& r = rt();
     std::lock_guard<std::mutex> lk(r.mu);
     if (bytes > r.workspace_bytes) {
-        not_capturing_locked(r, "backend_hip GEMM workspace");
+        if (r.capturing) return nullptr;
         if (r.workspace) {
             hip_check(hipStreamSynchronize(r.stream), "hipStreamSynchronize");
             r.arena.release(r.workspace);
         }
         r.workspace_bytes = round_up(bytes, kAlign);
         r.workspace = r.arena.alloc(r.workspace_bytes);
-        if (!r.workspace) {
-            r.workspace_bytes = 0;
-            fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating the GEMM workspace");
-        }
+        if (!r.workspace) r.workspace_bytes = 0;
     }
     return r.workspace;
+}
+
+void* workspace(size_t bytes) {
+    void* p = try_workspace(bytes);
+    if (p) return p;
+    Runtime& r = rt();
+    std::lock_guard<std::mutex> lk(r.mu);
+    not_capturing_locked(r, "backend_hip GEMM workspace");
+    fail(SDH_ERR_OOM, "backend_hip: arena exhausted allocating the GEMM workspace");
 }
 
 void arm_device_check(unsigned* word, const char* what, void (*on_failure)()) {

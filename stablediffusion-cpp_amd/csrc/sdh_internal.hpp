@@ -90,14 +90,24 @@ void* scratch(size_t bytes);
 // much, where the block would have to grow during a capture, or where the op
 // holds it already: the caller then takes a route without scratch.
 void* try_scratch(size_t bytes);
+// Sizes the scratch block for a later op, if it can be done now, without
+// holding it: a route that needs less than the op's other route asks for that
+// one's, so that what a program may capture after an op does not depend on the
+// route that the op took.
+void reserve_scratch(size_t bytes);
 // A persistent library-owned device block of at least `bytes` for a library
-// routine's workspace (the BLAS GEMM), distinct from scratch().
+// routine's workspace (the BLAS GEMM), distinct from scratch(); try_workspace
+// is null instead of an error where it cannot be had.
 void* workspace(size_t bytes);
+void* try_workspace(size_t bytes);
 // C[M,N] = P[M,K] B[N,K]^T (+ bias[N]) (+ C) on hipBLASLt, fp32 accumulation;
 // P and B bf16 (f32 false) or fp32 (f32 true), leading dimensions in elements
 // (k_gemm.hip). False when hipBLASLt has no algorithm for the shape.
 bool blaslt_gemm(bool f32, int64_t M, int64_t N, int64_t K, const void* P, int64_t ldp, const void* B, int64_t ldb,
                  float* C, int64_t ldc, const float* bias, bool accumulate);
+// Readies the library GEMM and its workspace, if it can be done now: for the
+// routes that do without it (see reserve_scratch).
+void reserve_blaslt();
 // Linear layers of at most 8 rows (k_gemv.hip), with checked arguments; false
 // where a GEMM takes them. B fp32, or bf16 with A rounded to it.
 bool gemv_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
