@@ -874,11 +874,6 @@ __global__ __launch_bounds__(64 * kGenWaves) void k_attn_generic(const float* __
     }
 }
 
-bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-    return x < y + nb && y < x + na;
-}
-
 // QK-norm + RoPE folded into the pack (k_qkv_prep); q is written back.
 struct QKPrep {
     float* q;

@@ -61,7 +61,9 @@ void run_conv2d(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(HW, kChunkFloats / K));
     reserve_scratch((size_t)(chunk * K) * 4);
     reserve_blaslt();
-    if (split_conv(x, N, Cin, H, W, w, Cout, kh, kw, bias, stride, pad, out, Ho, Wo)) {
+    const size_t ob = (size_t)(N * Cout * HW) * 4;  // out on x: sample by sample below, as the patches are gathered
+    if (!overlaps(out, ob, x, (size_t)(N * Cin * H * W) * 4) && !overlaps(out, ob, w, (size_t)(Cout * K) * 4) &&
+        split_conv(x, N, Cin, H, W, w, Cout, kh, kw, bias, stride, pad, out, Ho, Wo)) {
         launched(op);
         return;
     }

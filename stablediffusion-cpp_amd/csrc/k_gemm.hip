@@ -502,7 +502,9 @@ void run_gemm(const char* op, int64_t M, int64_t N, int64_t K, const float* A, i
     // aligned leading dimensions
     const bool lt = fast && ldc % 4 == 0 && aligned(C, 16) && (!bias || aligned(bias, 16));
     const size_t pbytes = ((size_t)(M * K) * 2 + 255) / 256 * 256, gbytes = (size_t)(M * N) * 4;
-    if (EPI == E_LINEAR && gemv_bf16(M, N, K, A, lda, B0, ldb, C, ldc, bias, accumulate)) {  // a few rows
+    // the kernel of a few rows reads A as it stores C; the others read A's packed copy
+    const bool apart = !overlaps(C, (size_t)((M - 1) * ldc + N) * 4, A, K > 0 ? (size_t)((M - 1) * lda + K) * 4 : 0);
+    if (EPI == E_LINEAR && apart && gemv_bf16(M, N, K, A, lda, B0, ldb, C, ldc, bias, accumulate)) {  // a few rows
         launched(op);
         if (fast) reserve_scratch(pbytes);
         if (lt) reserve_blaslt();

@@ -117,7 +117,11 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     if (bias) check_range(bias, (size_t)N * 4, op, "bias");
     const bool lt = K > 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(B, 16) &&
                     aligned(C, 16) && (!bias || aligned(bias, 16));
-    if (gemv_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {  // a few rows
+    // C on A or B: the routes below that were always there
+    const size_t cbytes = (size_t)((M - 1) * ldc + N) * 4;
+    const bool apart = K == 0 || (!overlaps(C, cbytes, A, (size_t)((M - 1) * lda + K) * 4) &&
+                                  !overlaps(C, cbytes, B, (size_t)((N - 1) * ldb + K) * 4));
+    if (apart && gemv_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {  // a few rows
         launched(op);
         if (lt) reserve_blaslt();
         return;
@@ -135,7 +139,7 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     // [300,321] 31.6 / 10.8).
     const double flops = 2.0 * (double)M * (double)N * (double)K;
     const bool large = N >= 128 && ((flops >= 3e9 && M >= 256) || (flops >= 2.4e9 && M >= 2048));
-    if (K > 0 && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
+    if (K > 0 && apart && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
         split_gemm(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
         launched(op);
         if (lt) reserve_blaslt();

@@ -41,11 +41,6 @@ constexpr int kThreads = 256;
 // [2,960,64,64] 11.4 against 11.9 us).
 constexpr int kStreamThreads = 64;
 
-bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-    return x < y + nb && y < x + na;
-}
-
 unsigned stride_grid(int64_t n) {
     const int64_t want = (n + kThreads - 1) / kThreads;
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)num_cus() * 32));

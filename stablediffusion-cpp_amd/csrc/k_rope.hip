@@ -501,11 +501,6 @@ __global__ __launch_bounds__(kThreads) void k_qknorm_rope_half(QKArgs a, int64_t
     }
 }
 
-bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-    return x < y + nb && y < x + na;
-}
-
 // Returns false when no fused kernel covers the shape (the caller then runs
 // the two ops one after the other).
 bool run_qknorm_rope_fused(float* q, int64_t inner_q, float* k, int64_t inner_k, int64_t N, int64_t S, int64_t dim,

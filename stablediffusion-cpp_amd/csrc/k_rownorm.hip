@@ -1038,11 +1038,6 @@ void run_rownorm(const char* op, int mode, const float* x, float* y, int64_t row
     launched(op);
 }
 
-bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-    return x < y + nb && y < x + na;
-}
-
 void run_rms_mod_bf16(const float* x, uint16_t* y, int64_t rows, int64_t C, const float* gamma, const float* scale,
                       float eps) {
     const char* op = "sdh_rms_norm_modulate_bf16";

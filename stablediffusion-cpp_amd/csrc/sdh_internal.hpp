@@ -158,6 +158,10 @@ void zero_device(void* p, size_t bytes);
 inline void need(bool ok, const char* op, const char* msg) {
     if (!ok) fail(SDH_ERR_INVALID, std::string(op) + ": " + msg);
 }
+inline bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
+}
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline unsigned blocks_for(int64_t items, int64_t per_block) {
     int64_t b = (items + per_block - 1) / per_block;

@@ -54,3 +54,16 @@ def test_conv2d_rejects_bad_output_size(be):
     with pytest.raises(sdhip.SdhError) as e:
         be.conv2d(x, 1, 2, 5, 5, w, 3, 3, 3, None, 1, 0, out, 5, 5)  # pad 0 gives 3 x 3
     assert e.value.status == sdhip.SDH_ERR_INVALID
+
+
+def test_conv2d_in_place(be, orc):
+    """out on x: each sample's patches are gathered before its output is
+    stored, so this gives the convolution of the original (1x1 and 3x3)."""
+    for k, seed in ((1, 8101), (3, 8102)):
+        N, C, H, W = 2, 33, 19, 21
+        x = orc.randn((N, C, H, W), seed)
+        w = orc.randn((C, C, k, k), seed + 10, 0.0, 0.1)
+        dx = be.array(x)
+        be.conv2d(dx, N, C, H, W, be.array(w), C, k, k, None, 1, k // 2, dx, H, W)
+        want, S = orc.conv2d(x, w, None, 1, k // 2)
+        assert_gemm(dx.download(), want, S, C * k * k + 2, f"in place {k}x{k}")

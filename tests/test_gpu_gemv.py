@@ -33,3 +33,22 @@ def test_few_rows(be, orc, M, N, K):
         be.gemm_nt_bf16(M, N, K, dA, lda, be.array(W16), K, dC, N, None if acc else db, acc)
         want, S = orc.gemm_nt_bf16(A[:, :K], W16, None if acc else b, c0 if acc else None, acc)
         assert_gemm(dC.download(), want, S + more[acc], K + 2, f"bf16 {M}x{N}x{K} acc={acc}")
+
+
+@pytest.mark.parametrize("M", [1, 3, 8, 9])
+@pytest.mark.parametrize("N,lda", [(256, 256), (1024, 1024), (4104, 4104), (512, 520)])
+def test_bf16_rows_in_place(be, orc, M, N, lda):
+    """C on A: every value of A is read (and rounded) before C is stored. C
+    within A's rows (lda > N) too, with and without accumulation."""
+    from oracle import f32_to_bf16
+
+    A = orc.randn((M, lda), 6100 + N)
+    W16 = f32_to_bf16(orc.randn((N, N), 6101 + N, 0.0, 1.0 / np.sqrt(N))).reshape(N, N)
+    dW = be.array(W16)
+    for acc in (False, True):
+        dA = be.array(A)
+        be.gemm_nt_bf16(M, N, N, dA, lda, dW, N, dA, lda, None, acc)
+        want, S = orc.gemm_nt_bf16(A[:, :N], W16, None, A[:, :N] if acc else None, acc)
+        got = dA.download()
+        assert_gemm(got[:, :N], want, S + np.abs(A[:, :N]), N + 2, f"in place {M}x{N} acc={acc}")
+        assert np.array_equal(got[:, N:], A[:, N:])
