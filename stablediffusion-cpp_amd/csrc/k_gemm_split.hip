@@ -15,8 +15,8 @@
 //   linear  a block is one row of A, one row of B (one output feature)
 //   conv2d  a block is one output channel's weights; one sample of x
 // The exponents are exact and are applied to the accumulators at the end.
-// A tile that meets a row holding an infinity or a NaN, or (conv2d) a run of
-// 256 pixels whose values are all below 2^-14 of the sample's largest (where
+// A result whose row or column holds an infinity or a NaN, or (conv2d) sees a run
+// of 256 pixels whose values are all below 2^-14 of the sample's largest (where
 // the bound above would be looser than fp32's), is computed by plain fp32
 // FMAs from the original operands instead, so such inputs give what fp32 gives.
 //
@@ -329,7 +329,7 @@ struct SplitArgs {
     int steps, accumulate;
     int tm, tn, splits;      // tiles, parts of K
     float* part;             // splits > 1: [splits][tm * BM][tn * BN] sums without the exponents
-    unsigned* slow;          // splits > 1: [tm * tn], the tile was computed by the fp32 path
+    float* limc;             // conv2d, splits > 1: the columns' limits
     // further products of the same sizes (splits = 1): product i = (o, h) = (i / inner, i % inner)
     // takes A's matrix i, B's matrix o * kv + h / group and stores at C + o outC + h inC
     int batches, inner, group, kv;
@@ -343,43 +343,6 @@ struct SplitArgs {
     const unsigned* bad;
     int H, W, Wo, HWo, kh, kw, stride, pad, taps, Cin, Cout, npb, zero;
 };
-
-// One element by fp32 FMAs from the original operands.
-template <Kind KIND>
-__device__ __forceinline__ float dot_fp32(const SplitArgs& p, int row, int col) {
-    float s = 0.f;
-    if constexpr (KIND == kConv) {
-        const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
-        const int iy0 = oy * p.stride - p.pad, ix0 = ox * p.stride - p.pad;
-        const float* w = p.A0 + (int64_t)row * p.Cin * p.taps;
-        for (int ci = 0; ci < p.Cin; ++ci) {
-            const float* x = p.B0 + ((int64_t)n * p.Cin + ci) * p.H * p.W;
-            for (int ky = 0; ky < p.kh; ++ky)
-                for (int kx = 0; kx < p.kw; ++kx, ++w) {
-                    const int iy = iy0 + ky, ix = ix0 + kx;
-                    const bool in = (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
-                    s = fmaf(*w, in ? x[(int64_t)iy * p.W + ix] : 0.f, s);
-                }
-        }
-    } else if constexpr (KIND == kWeights) {
-        // the softmax weights as they were packed; one too small to be held counts as tiny,
-        // so that it still meets an infinity of B as fp32 has it
-        const int e = p.ea[row];
-        if (e == kBad) return __builtin_nanf("");
-        const float* b = p.B0 + (int64_t)col * p.ldb;
-        const int end = p.causal ? min(p.K, p.row0 + row + 1) : p.K;
-        for (int k = 0; k < end; ++k) {
-            const _Float16* h = (const _Float16*)((const char*)p.A + (int64_t)row * p.rowA + (k / kStep) * p.planeA) + k % kStep;
-            const float w = __builtin_amdgcn_ldexpf((float)h[0] + (float)h[kStep], e);
-            s = fmaf(fmaxf(w, 1e-38f), b[k], s);
-        }
-    } else {
-        const float* a = p.A0 + (int64_t)row * p.lda;
-        const float* b = p.B0 + (int64_t)col * p.ldb;
-        for (int k = 0; k < p.K; ++k) s = fmaf(a[k], b[k], s);
-    }
-    return s;
-}
 
 // Where element (row, col) lies, and what is added to it.
 template <bool CONV>
@@ -396,6 +359,200 @@ __device__ __forceinline__ void store(const SplitArgs& p, int row, int col, floa
     if (p.accumulate) v += *cp;
     if (p.bias) v += p.bias[CONV ? row : col];
     *cp = v;
+}
+
+// ---------------------------------------------------------------------------
+// The fp32 path: elements by fp32 FMAs from the original operands.
+// ---------------------------------------------------------------------------
+// Where column col's patch lies (conv2d): its sample, and its first pixel.
+struct Patch {
+    const float* x;
+    int iy, ix;
+};
+__device__ __forceinline__ Patch patch_of(const SplitArgs& p, int col) {
+    const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
+    return Patch{p.B0 + (int64_t)n * p.Cin * p.H * p.W, oy * p.stride - p.pad, ox * p.stride - p.pad};
+}
+__device__ __forceinline__ float patch_value(const SplitArgs& p, const Patch& a, int ci, int ky, int kx) {
+    const int iy = a.iy + ky, ix = a.ix + kx;
+    const bool in = (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
+    const float v = a.x[((int64_t)ci * p.H + (in ? iy : 0)) * p.W + (in ? ix : 0)];  // no load under a mask
+    return in ? v : 0.f;
+}
+// Softmax weight k of a row as it was packed, with the row's exponent; one too small to be
+// held counts as tiny, so that it still meets an infinity of B as fp32 has it.
+__device__ __forceinline__ float packed_weight(const SplitArgs& p, int row, int e, int k) {
+    const _Float16* h = (const _Float16*)((const char*)p.A + (int64_t)row * p.rowA + (k / kStep) * p.planeA) + k % kStep;
+    return fmaxf(__builtin_amdgcn_ldexpf((float)h[0] + (float)h[kStep], e), 1e-38f);
+}
+__device__ __forceinline__ int weights_of(const SplitArgs& p, int row) {  // how many a row has
+    return p.causal ? min(p.K, p.row0 + row + 1) : p.K;
+}
+
+// Thread t of T's share of one element.
+template <Kind KIND>
+__device__ __forceinline__ float dot_share(const SplitArgs& p, int row, int col, int t, int T) {
+    float s = 0.f;
+    if constexpr (KIND == kConv) {
+        const Patch at = patch_of(p, col);
+        const float* w = p.A0 + (int64_t)row * p.K;
+#pragma unroll 4
+        for (int k = t; k < p.K; k += T) {
+            const int ci = k / p.taps, tap = k - ci * p.taps, ky = tap / p.kw;
+            s = fmaf(w[k], patch_value(p, at, ci, ky, tap - ky * p.kw), s);
+        }
+    } else if constexpr (KIND == kWeights) {
+        const int e = p.ea[row], end = weights_of(p, row);
+        if (e == kBad) return __builtin_nanf("");
+        const float* b = p.B0 + (int64_t)col * p.ldb;
+#pragma unroll 4
+        for (int k = t; k < end; k += T) s = fmaf(packed_weight(p, row, e, k), b[k], s);
+    } else {
+        const float* a = p.A0 + (int64_t)row * p.lda;
+        const float* b = p.B0 + (int64_t)col * p.ldb;
+#pragma unroll 4
+        for (int k = t; k < p.K; k += T) s = fmaf(a[k], b[k], s);
+    }
+    return s;
+}
+
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // four floats at any float's address
+
+// Sixteen elements' sums over [k0, k1), K cut over the waves: rows row[], columns col[].
+template <Kind KIND>
+__device__ __forceinline__ void dot16(const SplitArgs& p, const int* row, const int* col, int k0, int k1,
+                                      float (&s)[4][4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[r][c] = 0.f;
+    auto add = [&](const float* a, const float* b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[r][c] = fmaf(a[r], b[c], s[r][c]);
+    };
+    float a[4], b[4];
+    if constexpr (KIND == kConv) {
+        Patch at[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) at[c] = patch_of(p, col[c]);
+        int ci = k0 / p.taps, ky = (k0 - ci * p.taps) / p.kw, kx = k0 - ci * p.taps - ky * p.kw;
+        constexpr int U = 4;  // so many k's loads on their way at once; past k1: the last one again, not added
+        for (int k = k0; k < k1; k += U) {
+            float va[U][4], vb[U][4];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) va[u][r] = p.A0[(int64_t)row[r] * p.K + min(k + u, k1 - 1)];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) vb[u][c] = patch_value(p, at[c], ci, ky, kx);
+                if (k + u + 1 < k1 && ++kx == p.kw) {
+                    kx = 0;
+                    if (++ky == p.kh) ky = 0, ++ci;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k + u < k1) add(va[u], vb[u]);
+        }
+    } else if constexpr (KIND == kWeights) {
+        int e[4], end[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            e[r] = p.ea[row[r]];
+            end[r] = weights_of(p, row[r]);
+        }
+        for (int k = k0; k < k1; ++k) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) b[c] = p.B0[(int64_t)col[c] * p.ldb + k];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float w = e[r] == kBad ? __builtin_nanf("") : packed_weight(p, row[r], e[r], k);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s[r][c] = k < end[r] ? fmaf(w, b[c], s[r][c]) : s[r][c];
+            }
+        }
+    } else {
+        const float *pa[4], *pb[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            pa[r] = p.A0 + (int64_t)row[r] * p.lda;
+            pb[r] = p.B0 + (int64_t)col[r] * p.ldb;
+        }
+        int k = k0;
+#pragma unroll 2
+        for (; k + 4 <= k1; k += 4) {
+            f4u va[4], vb[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                va[r] = *(const f4u*)(pa[r] + k);
+                vb[r] = *(const f4u*)(pb[r] + k);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[r] = va[r][i], b[r] = vb[r][i];
+                add(a, b);
+            }
+        }
+        for (; k < k1; ++k) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a[r] = pa[r][k], b[r] = pb[r][k];
+            add(a, b);
+        }
+    }
+}
+
+// One element by the workgroup's T threads; `sums`: T / 64 floats of LDS.
+template <Kind KIND, int T>
+__device__ __forceinline__ void element_fp32(const SplitArgs& p, int row, int col, float* sums) {
+    const int t = threadIdx.x;
+    const float s = dev::wave_sum(dot_share<KIND>(p, row, col, t, T));
+    if ((t & 63) == 0) sums[t >> 6] = s;
+    __syncthreads();
+    if (t == 0) {
+        float v = sums[0];
+#pragma unroll
+        for (int i = 1; i < T / 64; ++i) v += sums[i];
+        store<KIND == kConv>(p, row, col, place<KIND == kConv>(p, row, col), v);
+    }
+    __syncthreads();
+}
+
+// 1024 elements by the workgroup: 32 x 32 from (row0, col0) on, or (!SQUARE) 4 x 256.
+// Each wave sums a part of K for all of them, sixteen per lane; `sums`: 1024 floats of LDS.
+template <Kind KIND, int T, bool SQUARE>
+__device__ __forceinline__ void block_fp32(const SplitArgs& p, int row0, int col0, float* sums) {
+    constexpr int NW = T / 64;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    auto row_of = [&](int l, int r) __attribute__((always_inline)) { return row0 + (SQUARE ? (l >> 3) + 8 * r : r); };
+    auto col_of = [&](int l, int c) __attribute__((always_inline)) { return col0 + (SQUARE ? (l & 7) + 8 * c : l + 64 * c); };
+    int row[4], col[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        row[r] = min(row_of(lane, r), p.M - 1);
+        col[r] = min(col_of(lane, r), p.N - 1);
+    }
+    float s[4][4];
+    dot16<KIND>(p, row, col, (int)((int64_t)p.K * w / NW), (int)((int64_t)p.K * (w + 1) / NW), s);
+    for (int i = 0; i < NW; ++i) {
+        if (w == i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    float* q = sums + (r * 4 + c) * 64 + lane;
+                    *q = i ? *q + s[r][c] : s[r][c];
+                }
+        }
+        __syncthreads();
+    }
+    for (int i = t; i < 1024; i += T) {
+        const int rr = row_of(i & 63, i >> 8), cc = col_of(i & 63, (i >> 6) & 3);
+        if (rr < p.M && cc < p.N) store<KIND == kConv>(p, rr, cc, place<KIND == kConv>(p, rr, cc), sums[i]);
+    }
+    __syncthreads();
 }
 
 // COUNT loads of 64 x 16 bytes into LDS, one after the other from dst on: lane l
@@ -425,6 +582,13 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     __shared__ __attribute__((aligned(16))) int sea[BM];  // exponents of the rows, of the columns
     __shared__ int seb[BN];
     __shared__ float sbias[CONV ? BM : BN];
+    // A result stands if its magnitude before the exponents reaches its row's and its column's
+    // limit together; else the fp32 path computes it: one by one from `alone`, or by whole
+    // blocks of 32 x 32 where a block has more than kAlone of them.
+    __shared__ __attribute__((aligned(16))) float slr[BM];
+    __shared__ float slc[BN];
+    constexpr int NB = (BM / 32) * (BN / 32), kAlone = 16;
+    __shared__ int blocks[NB], alone[NB * kAlone], nalone;
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = w / (BN / WN), wn = w % (BN / WN);
     const int fr = lane & 31, fh = lane >> 5;
@@ -515,13 +679,18 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     aim();
     issue(sA0, sB0);
 
-    // rows and columns that need the fp32 path
-    bool bad = false;
+    // the rows' and columns' exponents and limits
+    bool watch = false;
+    auto limit = [&](bool bad) __attribute__((always_inline)) {
+        watch |= bad;
+        return bad ? INFINITY : 0.f;
+    };
+    if (t == 0) nalone = 0;
     for (int i = t; i < BM; i += T) {
         const int row = min(m0 + i, p.M - 1), e = p.ea[row];
         sea[i] = e;
         if (CONV) sbias[i] = p.bias ? p.bias[row] : 0.f;
-        bad |= e == kBad;
+        slr[i] = limit(e == kBad);
     }
     for (int i = t; i < BN; i += T) {
         const int col = min(n0 + i, p.N - 1);
@@ -530,30 +699,23 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
             seb[i] = p.eb[n];
             const int xa = min(max(ox * p.stride - p.pad, 0), p.W - 1);
             const int xb = min(max(ox * p.stride - p.pad + p.kw - 1, 0), p.W - 1);
+            bool bad = false;
             for (int ky = 0; ky < p.kh; ++ky) {
                 const int iy = min(max(oy * p.stride - p.pad + ky, 0), p.H - 1);
                 for (int b = (iy * p.W + xa) / kPixBlock; b <= (iy * p.W + xb) / kPixBlock; ++b)
                     bad |= p.bad[n * p.npb + b] != 0;
             }
+            slc[i] = limit(bad);
+            if (p.splits > 1 && z == 0 && mt == 0 && n0 + i < p.N) p.limc[col] = slc[i];
         } else {
             const int e = p.eb[col];
             seb[i] = e;
             sbias[i] = p.bias ? p.bias[col] : 0.f;
-            bad |= e == kBad;
+            slc[i] = limit(e == kBad);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (__syncthreads_or(bad)) {  // the first stage is in LDS behind this
-        if (z == 0) {
-            if (p.splits > 1 && t == 0) p.slow[lt] = 1;
-            for (int i = t; i < BM * BN; i += T) {
-                const int row = m0 + i / BN, col = n0 + i % BN;
-                if (row < p.M && col < p.N) store<CONV>(p, row, col, place<CONV>(p, row, col), dot_fp32<KIND>(p, row, col));
-            }
-        }
-        return;
-    }
-    if (p.splits > 1 && z == 0 && t == 0) p.slow[lt] = 0;
+    watch = __syncthreads_or(watch);  // the first stage is in LDS behind this
 
     f32x16 acc[RA][RB];
 #pragma unroll
@@ -670,6 +832,40 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
             }
         return;
     }
+    // the elements that the fp32 path takes: one bit for each of a lane's
+    unsigned low[RA * RB] = {};
+    if (watch) {
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            const float lc = slc[wn * WN + b * 32 + fr];
+#pragma unroll
+            for (int a = 0; a < RA; ++a) {
+                const int rl = wm * WM + a * 32;
+                unsigned m = 0;
+                int n = 0;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f4 lr = *(const f4*)(slr + rl + g * 8 + fh * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const bool is = !(fabsf(acc[a][b][g * 4 + i]) >= lr[i] + lc);
+                        m |= (unsigned)is << (g * 4 + i);
+                        n += __builtin_popcountll(__ballot(is));
+                    }
+                }
+                const bool whole = n > kAlone;
+                low[a * RB + b] = whole ? 0xFFFFu : m;
+                if (lane == 0) blocks[(rl / 32) * (BN / 32) + wn * RB + b] = whole;
+                if (!whole && m) {
+                    int at = atomicAdd(&nalone, __builtin_popcount(m));
+                    for (; m; m &= m - 1) {
+                        const int i = __builtin_ctz(m);
+                        alone[at++] = ((rl + (i >> 2) * 8 + fh * 4 + (i & 3)) << 16) | (wn * WN + b * 32 + fr);
+                    }
+                }
+            }
+        }
+    }
 #pragma unroll
     for (int b = 0; b < RB; ++b) {
         const int cl = wn * WN + b * 32 + fr, col = n0 + cl;
@@ -696,20 +892,31 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (i < left) q[i * ld] = v[i] + (CONV ? sbias[rl + i] : bc);
+                    if (i < left && !(low[a * RB + b] >> (g * 4 + i) & 1)) q[i * ld] = v[i] + (CONV ? sbias[rl + i] : bc);
             }
+    }
+    if (!watch) return;
+    __syncthreads();
+    float* sums = (float*)sA0;  // every fragment has been read
+    for (int i = 0; i < nalone; ++i) {
+        const int row = m0 + (alone[i] >> 16), col = n0 + (alone[i] & 0xFFFF);
+        if (row < p.M && col < p.N) element_fp32<KIND, T>(p, row, col, sums);
+    }
+    for (int i = 0; i < NB; ++i) {
+        const int row0 = m0 + i / (BN / 32) * 32, col0 = n0 + i % (BN / 32) * 32;
+        if (blocks[i] && row0 < p.M && col0 < p.N) block_fp32<KIND, T, true>(p, row0, col0, sums);
     }
 }
 
 // The sum of the parts of K, in their order, with the exponents, bias and C:
 // one column and four rows per thread (grid: columns / 256, rows / 4).
-template <bool CONV>
+template <Kind KIND>
 __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) {
-    const int col = blockIdx.x * 256 + threadIdx.x, row0 = blockIdx.y * 4;
-    if (col >= p.N) return;
-    // the tile's number as k_split_mm counts it
-    const int mt = row0 / BM, nt = col / BN, grp = mt / 8, gm = min(8, p.tm - grp * 8);
-    if (p.slow[grp * 8 * p.tn + nt * gm + mt % 8]) return;
+    constexpr bool CONV = KIND == kConv;
+    __shared__ float sums[1024];
+    __shared__ int alone[64], nalone;
+    const int t = threadIdx.x, row0 = blockIdx.y * 4, col = min((int)blockIdx.x * 256 + t, p.N - 1);
+    const bool mine = (int)blockIdx.x * 256 + t < p.N;
     const int64_t ld = (int64_t)p.tn * BN, plane = (int64_t)p.tm * BM * ld;
     const float* s = p.part + row0 * ld + col;  // whole tiles: rows past the matrix are there
     float v[4] = {s[0], s[ld], s[2 * ld], s[3 * ld]};
@@ -718,11 +925,33 @@ __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] += s[z * plane + i * ld];
     const int ec = p.eb[CONV ? col / p.HWo : col];
+    const float lc = CONV ? p.limc[col] : ec == kBad ? INFINITY : 0.f;
+    int er[4];
+    unsigned low = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        er[i] = p.ea[min(row0 + i, p.M - 1)];
+        const bool is = mine && row0 + i < p.M && !(fabsf(v[i]) >= lc + (er[i] == kBad ? INFINITY : 0.f));
+        low |= (unsigned)is << i;
+    }
+    const int n = __syncthreads_count(low);  // threads with such an element
+    if (n > 16) {
+        block_fp32<KIND, 256, false>(p, row0, (int)blockIdx.x * 256, sums);
+        return;
+    }
     float* q = place<CONV>(p, row0, col);
     const int64_t ldo = CONV ? p.HWo : p.ldc;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (row0 + i < p.M) store<CONV>(p, row0 + i, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], p.ea[row0 + i] + ec));
+        if (mine && row0 + i < p.M && !(low >> i & 1))
+            store<CONV>(p, row0 + i, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], er[i] + ec));
+    if (!n) return;
+    if (t == 0) nalone = 0;
+    __syncthreads();
+    for (; low; low &= low - 1) alone[atomicAdd(&nalone, 1)] = (__builtin_ctz(low) << 16) | t;
+    __syncthreads();
+    for (int i = 0; i < nalone; ++i)
+        element_fp32<KIND, 256>(p, row0 + (alone[i] >> 16), (int)blockIdx.x * 256 + (alone[i] & 0xFFFF), sums);
 }
 
 // ---------------------------------------------------------------------------
@@ -855,7 +1084,7 @@ void launch_mm(const Plan& q, SplitArgs& p) {
     else
         k_split_mm<64, 64, 32, 32, 3, KIND><<<grid, 256, 0, stream()>>>(p);
     if (q.splits > 1)
-        k_split_sum<KIND == kConv><<<dim3((unsigned)((p.N + 255) / 256), (unsigned)((p.M + 3) / 4)), 256, 0, stream()>>>(
+        k_split_sum<KIND><<<dim3((unsigned)((p.N + 255) / 256), (unsigned)((p.M + 3) / 4)), 256, 0, stream()>>>(
             p, q.bm(), q.bn());
 }
 
@@ -891,8 +1120,8 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     const Plan q = plan_of(M, N, steps);
     if ((int64_t)q.tm * q.tn * q.splits * 512 >= kMost) return false;
     const size_t pa = up((size_t)steps * M * kRowBytes), pb = up((size_t)steps * N * kRowBytes);
-    const size_t ea = up((size_t)M * 4), eb = up((size_t)N * 4), sl = up((size_t)q.tm * q.tn * 4);
-    char* s = (char*)try_scratch(pa + pb + ea + eb + sl + q.part_bytes());
+    const size_t ea = up((size_t)M * 4), eb = up((size_t)N * 4);
+    char* s = (char*)try_scratch(pa + pb + ea + eb + q.part_bytes());
     if (!s) return false;
     SplitArgs p{};
     const PackRows ra{A, lda, (u16*)s, (int*)(s + pa + pb), (int)M, (int)K, 1, 0, 0};
@@ -916,8 +1145,7 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     p.tm = q.tm;
     p.tn = q.tn;
     p.splits = q.splits;
-    p.slow = (unsigned*)(s + pa + pb + ea + eb);
-    p.part = (float*)(s + pa + pb + ea + eb + sl);
+    p.part = (float*)(s + pa + pb + ea + eb);
     p.A0 = A;
     p.B0 = B;
     p.lda = lda;
@@ -942,8 +1170,8 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     a.npb = (int)((HW + kPixBlock - 1) / kPixBlock);
     const size_t px = up((size_t)chunks * prows * kRowBytes), pw = up((size_t)steps * Cout * kRowBytes);
     const size_t mx = up((size_t)N * a.ncb * a.npb * 4), bd = up((size_t)N * a.npb * 4);
-    const size_t ex = up((size_t)N * 4), ew = up((size_t)Cout * 4), sl = up((size_t)q.tm * q.tn * 4);
-    char* s = (char*)try_scratch(px + pw + mx + bd + ex + ew + sl + q.part_bytes());
+    const size_t ex = up((size_t)N * 4), ew = up((size_t)Cout * 4), lc = q.splits > 1 ? up((size_t)cols * 4) : 0;
+    char* s = (char*)try_scratch(px + pw + mx + bd + ex + ew + lc + q.part_bytes());
     if (!s) return false;
     a.x = x;
     a.w = w;
@@ -984,8 +1212,8 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     p.tm = q.tm;
     p.tn = q.tn;
     p.splits = q.splits;
-    p.slow = (unsigned*)(s += ew);
-    p.part = (float*)(s + sl);
+    p.limc = (float*)(s += ew);
+    p.part = (float*)(s + lc);
     p.A0 = w;
     p.B0 = x;
     p.bad = a.bad;
@@ -1035,10 +1263,9 @@ bool split_attention(const float* q, const float* k, const float* v, void* out, 
     const size_t pv = up((size_t)kn * ssteps * d * kRowBytes), vt = up((size_t)N * kvi * Skv * 4);
     const size_t sc = up((size_t)nb * rb * skp * 4);
     const size_t eq = up((size_t)qn * Sq * 4), ek = up((size_t)kn * Skv * 4), ev = up((size_t)kn * d * 4);
-    // these two for any round, so that the budget alone decides what a call holds
-    const size_t ep = up((size_t)qn * Sq * 4), sl = up((size_t)((Sq + 63) / 64) * ((std::max(Skv, d) + 63) / 64) * 4);
+    const size_t ep = up((size_t)qn * Sq * 4);  // for any round, so that the budget alone decides what a call holds
     const size_t parts = std::max(p1.part_bytes(), p2.part_bytes()), o16 = out16 ? up((size_t)N * Sq * inner * 4) : 0;
-    char* s = (char*)try_scratch(pq + pk + pv + vt + sc + eq + ek + ev + ep + sl + o16 + parts);
+    char* s = (char*)try_scratch(pq + pk + pv + vt + sc + eq + ek + ev + ep + o16 + parts);
     if (!s) return false;
     auto take = [&](size_t n) {
         char* r = s;
@@ -1051,7 +1278,6 @@ bool split_attention(const float* q, const float* k, const float* v, void* out, 
     const PackRows rv{tv, Skv, (u16*)take(pv), (int*)take(ev), (int)d, (int)Skv, 1, d * Skv, 0};
     float* const S = (float*)take(sc);
     int* const exps = (int*)take(ep);
-    unsigned* const slow = (unsigned*)take(sl);
     float* const o = out16 ? (float*)take(o16) : (float*)out;
     transpose_device("sdh_attention", v, tv, N, Skv, kvi);
     const PackRows none{};
@@ -1104,7 +1330,6 @@ bool split_attention(const float* q, const float* k, const float* v, void* out, 
             p.N = (int)Skv;
             p.K = (int)d;
             p.steps = (int)dsteps;
-            p.slow = slow;
             p.part = (float*)s;
             launch_mm<kDense>(sized(p1, p), p);
             auto soft = skp <= 512    ? k_softmax_split<64, 1>

@@ -263,3 +263,54 @@ def test_small_arena():
                        env=dict(os.environ, SDH_ARENA_MB="160", SDH_ARENA_LIMIT_MB="160"))
     print(r.stdout, r.stderr[-3000:])
     assert r.returncode == 0 and "small arena ok" in r.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,acc", [
+    (3000, 5000, 160, True), (4097, 2049, 128, False), (1024, 1032, 1000, False),  # 256, 128 and 64 wide tiles
+    (700, 260, 8192, True),  # parts of K
+])
+def test_gemm_one_bad_row_and_column(be, orc, M, N, K, acc):
+    """A NaN in a row of A and infinities in a row of W: the blocks of their
+    results by fp32 FMAs, every other result untouched, also where C is added."""
+    def edit(A, W):
+        A[M // 2, K // 3] = np.nan
+        W[N // 3] = np.abs(W[N // 3])
+        W[N // 3, 5] = np.inf
+        A[:, 5] = np.abs(A[:, 5]) + 0.1
+
+    got, A, W, b, c0 = run_gemm(be, orc, M, N, K, 5200 + K, acc=acc, edit=edit)
+    rows = np.unique(np.concatenate([np.arange(0, M, max(1, M // 50)), np.arange(M // 2 - 3, M // 2 + 4), [M - 1]]))
+    A2 = A.copy()
+    A2[M // 2, K // 3] = 0
+    W2 = W.copy()
+    W2[N // 3, 5] = 0
+    want, S = orc.gemm_nt_f32(A2[rows], W2, b, c0[rows] if acc else None, acc)
+    got = got[rows]
+    at = list(rows).index(M // 2)
+    assert np.all(np.isnan(got[at]))
+    fine = np.ones(got.shape, bool)
+    fine[at] = fine[:, N // 3] = False
+    assert np.all(np.isposinf(np.delete(got[:, N // 3], at)))
+    assert_gemm(got[fine], want[fine], S[fine], K + 2, f"beside bad rows {M}x{N}x{K}")
+
+
+@pytest.mark.gpu
+def test_conv_one_bad_pixel_in_parts(be, orc):
+    """An infinity in one pixel and a NaN in one output channel's weights where
+    K is cut into parts: nine pixels of every channel, all pixels of one."""
+    N, Cin, H, W, Cout = 2, 260, 8, 8, 300
+    x = orc.randn((N, Cin, H, W), 5300)
+    w = orc.randn((Cout, Cin, 3, 3), 5301, 0.0, 0.02)
+    want, S = orc.conv2d(x, w, None, 1, 1)
+    x[1, 100, 3, 4] = np.inf
+    w[77, 9, 1, 1] = np.nan
+    out = be.empty((N, Cout, H, W))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, 3, 3, None, 1, 1, out, H, W)
+    got = out.download()
+    bad = np.zeros(got.shape, bool)
+    bad[:, 77] = True
+    bad[1, :, 2:5, 3:6] = True
+    assert np.array_equal(~np.isfinite(got), bad)
+    assert np.all(np.isnan(got[:, 77]))
+    assert_gemm(got[~bad], want[~bad], S[~bad], Cin * 9 + 2, "beside a bad pixel and channel")
