@@ -107,7 +107,10 @@ int sdh_gemm_nt_bf16_packed(int64_t M, int64_t N, int64_t K, const uint16_t* A, 
 /* ---- GEMM with fp32 weights --------------------------------------------- */
 /* backend_cuda.h:38-40 gemm_nt_f32(): C[M,N] = A[M,K] * B[N,K]^T (+ C when
  * accumulate) (+ bias[N]), all fp32, row-major with leading dimensions in
- * elements; bias may be NULL. The linear layers whose weights stay fp32. */
+ * elements; bias may be NULL. The linear layers whose weights stay fp32. Large
+ * products run on fp16 pairs: each operand is within 2^-22 of its value, and of
+ * values below 2^-17 of their row's largest within 2^-39 of that one; a result
+ * that the latter could move by more than 2^-22 of itself is computed in fp32. */
 int sdh_gemm_nt_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb,
                     float* C, int64_t ldc, const float* bias, int accumulate);
 /* backend_cuda.h:45-47 conv2d(); tensor.h:159 (tensor.cpp:520-560).
@@ -227,7 +230,9 @@ int sdh_swiglu_bf16(const float* gate, const float* up, uint16_t* y, int64_t n);
  * head h / (heads / kv_heads); causal keeps keys 0..i for query i.
  * kv_heads <= 0 means kv_heads = heads. out must not overlap the inputs.
  * Fused on the MFMA units (no score matrix in memory) for d <= 128; above, with
- * more than 64 keys, blocks of the score matrix in library scratch. */
+ * more than 64 keys, blocks of the score matrix in library scratch, its products
+ * as sdh_gemm_nt_f32's large ones; softmax weights below 2^-17 of their row's
+ * largest are held within 2^-39 of that one. */
 int sdh_attention(const float* q, const float* k, const float* v, float* out, int64_t N, int64_t Sq, int64_t Skv,
                   int heads, int kv_heads, int64_t d, int causal);
 /* FUSED: out = bf16 bits of attention(q, k, v): sdh_attention then the bf16

@@ -10,6 +10,13 @@
 // fp32 accumulation: three fp16 MFMAs per fp32 product. |x - hi - lo| is at most
 // 2^-23 |x| while |x| >= 2^-16 of the block's largest value and at most 2^-39
 // of that value below it; the dropped lo_a lo_b is at most 2^-24 of the product.
+// Where the values that lose bits this way could matter, fp32 takes over: the
+// pack counts, row by row, the values below 2^-17 of the row's largest that were
+// not held exactly, and a result stands only if its magnitude is at least 2^22
+// times what they can have cost it (kPerTail); else it is computed by fp32
+// FMAs from the original operands. Ordinary rows have no such value or one, and
+// about one result in 10^7 is computed again; a row of unlike groups of
+// channels met by weights that ignore the large ones gives what fp32 gives.
 // Against 64-bit results the products come out closer than the fp32 MFMA's,
 // whose K additions round one by one where these round once per 16 products.
 //   linear  a block is one row of A, one row of B (one output feature)
@@ -52,6 +59,10 @@ constexpr int kStep = 32;            // K per step
 constexpr int kRowBytes = 128;       // one row of one step: 32 hi, 32 lo
 constexpr int kBad = 1 << 20;        // exponent of a row that holds an infinity or a NaN
 constexpr unsigned kInf = 0x7F800000u;
+constexpr unsigned kNotFinite = 1u << 31;  // in a row's count: it holds an infinity or a NaN
+// A scaled value below 2^-3 is off by at most 2^-25 and meets one below 2^15: 2^-10 of a result
+// before the exponents, and 2^22 times that must be reached.
+constexpr float kPerTail = 4096.f;
 constexpr int kBufferWord3 = 0x00020000;  // raw buffer resource, 32-bit data format
 constexpr int kPixBlock = 256, kChanBlock = 32;  // conv2d: x's maxima are kept per this many pixels and channels
 
@@ -71,15 +82,38 @@ __device__ __forceinline__ unsigned wave_umax(unsigned v) {
     return v;
 }
 
-// Eight values scaled by 2^s and split.
-__device__ __forceinline__ void split8(const float* x, int s, h8& hi, h8& lo) {
+__device__ __forceinline__ unsigned wave_usum(unsigned v) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) v += (unsigned)__shfl_xor((int)v, o, 64);
+    return v;
+}
+
+// Eight values scaled by 2^s and split; how many of them are small (see kPerTail)
+// and not held exactly, which few waves have to count.
+__device__ __forceinline__ int split8(const float* x, int s, h8& hi, h8& lo) {
+    constexpr float kSmall = 0.125f;
+    float least = INFINITY;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const float v = __builtin_amdgcn_ldexpf(x[e], s);
+        least = fminf(least, fabsf(v));
         hi[e] = (_Float16)v;
         lo[e] = (_Float16)(v - (float)hi[e]);
     }
+    int n = 0;
+    if (__any(least < kSmall)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float v = __builtin_amdgcn_ldexpf(x[e], s);
+            const float back = (float)hi[e] + (float)lo[e];  // exact for small v; v may have vanished in the scaling
+            n += fabsf(v) < kSmall && (back != v || (v == 0.f) != (x[e] == 0.f));
+        }
+    }
+    return n;
 }
+
+// What a row's count asks of a result's magnitude.
+__device__ __forceinline__ float limit_of(unsigned tail) { return tail >= kNotFinite ? INFINITY : (float)tail * kPerTail; }
 
 // ---------------------------------------------------------------------------
 // Pack of dense rows: X [rows, K] (ld) -> planes, exps. One wave per row: the
@@ -90,6 +124,7 @@ struct PackRows {
     int64_t ld;
     u16* P;
     int* exps;
+    unsigned* tails;  // see kPerTail
     int rows, K;
     // further matrices of the same sizes: matrix i starts at X + (i / inner) outer_ld + (i % inner) inner_ld
     int inner;
@@ -99,23 +134,24 @@ struct PackRows {
 __device__ __forceinline__ unsigned umax4(const f4& v) {
     return max(max(absbits(v.x), absbits(v.y)), max(absbits(v.z), absbits(v.w)));
 }
-__device__ __forceinline__ void store_split(u16* o, const float* v, int s) {
+__device__ __forceinline__ int store_split(u16* o, const float* v, int s) {
     h8 hi, lo;
-    split8(v, s, hi, lo);
+    const int n = split8(v, s, hi, lo);
     *(h8*)o = hi;
     *(h8*)(o + kStep) = lo;
+    return n;
 }
-
 // A row of LANES threads' values to steps. TURNS > 0: float4 loads (K, ld and X
 // aligned for them) of at most 8 LANES TURNS values, all in flight at once and
 // kept in registers. TURNS = 0: any row, read twice.
 template <int LANES, int TURNS>
-__device__ __forceinline__ void pack_row(const PackRows& a, const float* x, u16* P, int* exps, int row, int lane,
-                                         unsigned* red) {
+__device__ __forceinline__ void pack_row(const PackRows& a, const float* x, u16* P, int* exps, unsigned* tails, int row,
+                                         int lane, unsigned* red) {
     const int kp = (a.K + kStep - 1) / kStep * kStep;
     auto out = [&](int k) __attribute__((always_inline)) {
         return P + ((int64_t)(k / kStep) * a.rows + row) * (kRowBytes / 2) + (k % kStep);
     };
+    bool bad = false;
     auto exponent = [&](unsigned m) __attribute__((always_inline)) {
         m = wave_umax(m);
         if constexpr (LANES > 64) {
@@ -125,9 +161,11 @@ __device__ __forceinline__ void pack_row(const PackRows& a, const float* x, u16*
         }
         const int e = exp_of(m);
         if (lane == 0) exps[row] = e;
-        return e == kBad ? 0 : -e;
+        bad = e == kBad;
+        return bad ? 0 : -e;
     };
     unsigned m = 0;
+    int n = 0;
     if constexpr (TURNS > 0) {
         f4 v[TURNS][2];
 #pragma unroll
@@ -146,7 +184,7 @@ __device__ __forceinline__ void pack_row(const PackRows& a, const float* x, u16*
             float f[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) f[i] = k + i < a.K ? v[j][i / 4][i % 4] : 0.f;
-            store_split(out(k), f, e);
+            n += store_split(out(k), f, e);
         }
     } else {
 #pragma unroll 4
@@ -156,17 +194,24 @@ __device__ __forceinline__ void pack_row(const PackRows& a, const float* x, u16*
             float f[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) f[i] = k + i < a.K ? x[k + i] : 0.f;
-            store_split(out(k), f, e);
+            n += store_split(out(k), f, e);
         }
     }
+    unsigned tail = __any(n) ? wave_usum((unsigned)n) : 0u;
+    if constexpr (LANES > 64) {
+        if ((lane & 63) == 0) red[4 + (lane >> 6)] = tail;
+        __syncthreads();
+        tail = (red[4] + red[5]) + (red[6] + red[7]);
+    }
+    if (lane == 0) tails[row] = bad ? kNotFinite : tail;
 }
 
 // Two operands in one launch: the first ba workgroups take a's rows, the rest
 // b's. Four rows per workgroup, a wave each, or (LANES 256) one. grid.y: the matrices.
 template <int LANES, int TURNS>
-__global__ __launch_bounds__(256) void k_split_pack(PackRows a, PackRows b, int ba) {
+__global__ __launch_bounds__(256, TURNS < 4 ? 8 : 4) void k_split_pack(PackRows a, PackRows b, int ba) {
     constexpr int ROWS = 256 / LANES;
-    __shared__ unsigned red[4];
+    __shared__ unsigned red[8];
     const bool first = (int)blockIdx.x < ba;
     const PackRows& p = first ? a : b;
     const int row = ((int)blockIdx.x - (first ? 0 : ba)) * ROWS + (int)threadIdx.x / LANES;
@@ -174,8 +219,8 @@ __global__ __launch_bounds__(256) void k_split_pack(PackRows a, PackRows b, int 
     const int i = blockIdx.y;
     const int64_t steps = (p.K + kStep - 1) / kStep;
     const float* x = p.X + (i / p.inner) * p.outer_ld + (i % p.inner) * p.inner_ld + (int64_t)row * p.ld;
-    pack_row<LANES, TURNS>(p, x, p.P + i * steps * p.rows * (kRowBytes / 2), p.exps + (int64_t)i * p.rows, row,
-                           threadIdx.x % LANES, red);
+    pack_row<LANES, TURNS>(p, x, p.P + i * steps * p.rows * (kRowBytes / 2), p.exps + (int64_t)i * p.rows,
+                           p.tails + (int64_t)i * p.rows, row, threadIdx.x % LANES, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -322,6 +367,8 @@ struct SplitArgs {
     int rowA;                // bytes from one row of A's step to the next
     const int* ea;           // per row
     const int* eb;           // per column; conv2d: per sample
+    const unsigned* ta;      // counts per row (kDense), per column (not conv2d): see kPerTail
+    const unsigned* tb;
     float* C;
     int64_t ldc;
     const float* bias;       // per column; conv2d: per row
@@ -520,14 +567,14 @@ __device__ __forceinline__ void element_fp32(const SplitArgs& p, int row, int co
     __syncthreads();
 }
 
-// 1024 elements by the workgroup: 32 x 32 from (row0, col0) on, or (!SQUARE) 4 x 256.
-// Each wave sums a part of K for all of them, sixteen per lane; `sums`: 1024 floats of LDS.
-template <Kind KIND, int T, bool SQUARE>
+// 32 x 32 elements from (row0, col0) on by the workgroup: each wave sums a part
+// of K for all of them, sixteen per lane; `sums`: 1024 floats of LDS.
+template <Kind KIND, int T>
 __device__ __forceinline__ void block_fp32(const SplitArgs& p, int row0, int col0, float* sums) {
     constexpr int NW = T / 64;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    auto row_of = [&](int l, int r) __attribute__((always_inline)) { return row0 + (SQUARE ? (l >> 3) + 8 * r : r); };
-    auto col_of = [&](int l, int c) __attribute__((always_inline)) { return col0 + (SQUARE ? (l & 7) + 8 * c : l + 64 * c); };
+    auto row_of = [&](int l, int r) __attribute__((always_inline)) { return row0 + (l >> 3) + 8 * r; };
+    auto col_of = [&](int l, int c) __attribute__((always_inline)) { return col0 + (l & 7) + 8 * c; };
     int row[4], col[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -588,7 +635,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     __shared__ __attribute__((aligned(16))) float slr[BM];
     __shared__ float slc[BN];
     constexpr int NB = (BM / 32) * (BN / 32), kAlone = 16;
-    __shared__ int blocks[NB], alone[NB * kAlone], nalone;
+    __shared__ int alone[NB * kAlone], whole[NB], nalone, nwhole;
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = w / (BN / WN), wn = w % (BN / WN);
     const int fr = lane & 31, fh = lane >> 5;
@@ -604,6 +651,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
         p.B = (const u16*)((const char*)p.B + b * p.matB);
         p.ea += (int64_t)z * p.M;
         p.eb += (int64_t)b * p.N;
+        if (KIND == kDense) p.ta += (int64_t)z * p.M;
+        p.tb += (int64_t)b * p.N;
         p.C += o * p.outC + h * p.inC;
         if (KIND == kDense) p.A0 += o * p.outA0 + h * p.inA0;
         p.B0 += o * p.outB0 + (h / p.group) * p.inB0;
@@ -681,16 +730,16 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
 
     // the rows' and columns' exponents and limits
     bool watch = false;
-    auto limit = [&](bool bad) __attribute__((always_inline)) {
-        watch |= bad;
-        return bad ? INFINITY : 0.f;
+    auto limit = [&](unsigned tail) __attribute__((always_inline)) {
+        watch |= tail != 0;
+        return limit_of(tail);
     };
-    if (t == 0) nalone = 0;
+    if (t == 0) nalone = nwhole = 0;
     for (int i = t; i < BM; i += T) {
         const int row = min(m0 + i, p.M - 1), e = p.ea[row];
         sea[i] = e;
         if (CONV) sbias[i] = p.bias ? p.bias[row] : 0.f;
-        slr[i] = limit(e == kBad);
+        slr[i] = limit(KIND == kDense ? p.ta[row] : e == kBad ? kNotFinite : 0u);
     }
     for (int i = t; i < BN; i += T) {
         const int col = min(n0 + i, p.N - 1);
@@ -705,13 +754,13 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
                 for (int b = (iy * p.W + xa) / kPixBlock; b <= (iy * p.W + xb) / kPixBlock; ++b)
                     bad |= p.bad[n * p.npb + b] != 0;
             }
-            slc[i] = limit(bad);
+            slc[i] = limit(bad ? kNotFinite : 0u);
             if (p.splits > 1 && z == 0 && mt == 0 && n0 + i < p.N) p.limc[col] = slc[i];
         } else {
             const int e = p.eb[col];
             seb[i] = e;
             sbias[i] = p.bias ? p.bias[col] : 0.f;
-            slc[i] = limit(e == kBad);
+            slc[i] = limit(p.tb[col]);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -834,29 +883,42 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
     }
     // the elements that the fp32 path takes: one bit for each of a lane's
     unsigned low[RA * RB] = {};
+    bool look = false;
     if (watch) {
+        // most waves' smallest result reaches the largest limits that they have
+        float top = 0.f, topc = 0.f, least = INFINITY;
 #pragma unroll
-        for (int b = 0; b < RB; ++b) {
+        for (int i = 0; i < WM; i += 64) top = fmaxf(top, slr[wm * WM + (i + lane) % WM]);
+#pragma unroll
+        for (int i = 0; i < WN; i += 64) topc = fmaxf(topc, slc[wn * WN + (i + lane) % WN]);
+        top = dev::wave_max(top) + dev::wave_max(topc);
+#pragma unroll
+        for (int a = 0; a < RA; ++a)
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) least = fminf(least, fabsf(acc[a][b][i]));
+        look = __any(!(least >= top));
+#pragma unroll
+        for (int b = 0; b < RB && look; ++b) {
             const float lc = slc[wn * WN + b * 32 + fr];
 #pragma unroll
             for (int a = 0; a < RA; ++a) {
                 const int rl = wm * WM + a * 32;
                 unsigned m = 0;
-                int n = 0;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const f4 lr = *(const f4*)(slr + rl + g * 8 + fh * 4);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const bool is = !(fabsf(acc[a][b][g * 4 + i]) >= lr[i] + lc);
-                        m |= (unsigned)is << (g * 4 + i);
-                        n += __builtin_popcountll(__ballot(is));
-                    }
+                    for (int i = 0; i < 4; ++i)
+                        m |= (unsigned)!(fabsf(acc[a][b][g * 4 + i]) >= lr[i] + lc) << (g * 4 + i);
                 }
-                const bool whole = n > kAlone;
-                low[a * RB + b] = whole ? 0xFFFFu : m;
-                if (lane == 0) blocks[(rl / 32) * (BN / 32) + wn * RB + b] = whole;
-                if (!whole && m) {
+                if (!__any(m != 0)) continue;
+                if (wave_usum(__builtin_popcount(m)) > kAlone) {
+                    low[a * RB + b] = 0xFFFFu;
+                    if (lane == 0) whole[atomicAdd(&nwhole, 1)] = (rl << 16) | (wn * WN + b * 32);
+                } else if (m) {
+                    low[a * RB + b] = m;
                     int at = atomicAdd(&nalone, __builtin_popcount(m));
                     for (; m; m &= m - 1) {
                         const int i = __builtin_ctz(m);
@@ -866,45 +928,53 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
             }
         }
     }
+    auto store_all = [&](auto some) __attribute__((always_inline)) {
+        constexpr bool SOME = decltype(some)::value;
 #pragma unroll
-    for (int b = 0; b < RB; ++b) {
-        const int cl = wn * WN + b * 32 + fr, col = n0 + cl;
-        if (col >= p.N) continue;
-        const int ec = seb[cl];
-        const float bc = CONV ? 0.f : sbias[cl];
-        float* cp = place<CONV>(p, m0 + wm * WM + fh * 4, col);
-        const int64_t ld = CONV ? p.HWo : p.ldc;
+        for (int b = 0; b < RB; ++b) {
+            const int cl = wn * WN + b * 32 + fr, col = n0 + cl;
+            if (col >= p.N) continue;
+            const int ec = seb[cl];
+            const float bc = CONV ? 0.f : sbias[cl];
+            float* cp = place<CONV>(p, m0 + wm * WM + fh * 4, col);
+            const int64_t ld = CONV ? p.HWo : p.ldc;
 #pragma unroll
-        for (int a = 0; a < RA; ++a)
+            for (int a = 0; a < RA; ++a)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int rl = wm * WM + a * 32 + g * 8 + fh * 4;  // four rows from here
-                const int4 er = *(const int4*)(sea + rl);
-                f4 v = {__builtin_amdgcn_ldexpf(acc[a][b][g * 4], er.x + ec),
-                        __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 1], er.y + ec),
-                        __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 2], er.z + ec),
-                        __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 3], er.w + ec)};
-                float* q = cp + (a * 32 + g * 8) * ld;
-                const int left = p.M - m0 - rl;
-                if (!CONV && p.accumulate) {
+                for (int g = 0; g < 4; ++g) {
+                    const int rl = wm * WM + a * 32 + g * 8 + fh * 4;  // four rows from here
+                    const int4 er = *(const int4*)(sea + rl);
+                    f4 v = {__builtin_amdgcn_ldexpf(acc[a][b][g * 4], er.x + ec),
+                            __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 1], er.y + ec),
+                            __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 2], er.z + ec),
+                            __builtin_amdgcn_ldexpf(acc[a][b][g * 4 + 3], er.w + ec)};
+                    float* q = cp + (a * 32 + g * 8) * ld;
+                    const int left = p.M - m0 - rl;
+                    if (!CONV && p.accumulate) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] += q[min(i, max(left - 1, 0)) * ld];
+                        for (int i = 0; i < 4; ++i) v[i] += q[min(i, max(left - 1, 0)) * ld];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (i < left && !(SOME && low[a * RB + b] >> (g * 4 + i) & 1)) q[i * ld] = v[i] + (CONV ? sbias[rl + i] : bc);
                 }
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (i < left && !(low[a * RB + b] >> (g * 4 + i) & 1)) q[i * ld] = v[i] + (CONV ? sbias[rl + i] : bc);
-            }
-    }
+        }
+    };
+    if (look)
+        store_all(std::true_type());
+    else
+        store_all(std::false_type());
     if (!watch) return;
     __syncthreads();
+    if (nalone + nwhole == 0) return;
     float* sums = (float*)sA0;  // every fragment has been read
     for (int i = 0; i < nalone; ++i) {
         const int row = m0 + (alone[i] >> 16), col = n0 + (alone[i] & 0xFFFF);
         if (row < p.M && col < p.N) element_fp32<KIND, T>(p, row, col, sums);
     }
-    for (int i = 0; i < NB; ++i) {
-        const int row0 = m0 + i / (BN / 32) * 32, col0 = n0 + i % (BN / 32) * 32;
-        if (blocks[i] && row0 < p.M && col0 < p.N) block_fp32<KIND, T, true>(p, row0, col0, sums);
+    for (int i = 0; i < nwhole; ++i) {
+        const int row0 = m0 + (whole[i] >> 16), col0 = n0 + (whole[i] & 0xFFFF);
+        if (row0 < p.M && col0 < p.N) block_fp32<KIND, T>(p, row0, col0, sums);
     }
 }
 
@@ -913,10 +983,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
 template <Kind KIND>
 __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) {
     constexpr bool CONV = KIND == kConv;
-    __shared__ float sums[1024];
-    __shared__ int alone[64], nalone;
-    const int t = threadIdx.x, row0 = blockIdx.y * 4, col = min((int)blockIdx.x * 256 + t, p.N - 1);
-    const bool mine = (int)blockIdx.x * 256 + t < p.N;
+    const int lane = threadIdx.x & 63, row0 = blockIdx.y * 4, mine = blockIdx.x * 256 + threadIdx.x;
+    const int col = min(mine, p.N - 1);
     const int64_t ld = (int64_t)p.tn * BN, plane = (int64_t)p.tm * BM * ld;
     const float* s = p.part + row0 * ld + col;  // whole tiles: rows past the matrix are there
     float v[4] = {s[0], s[ld], s[2 * ld], s[3 * ld]};
@@ -925,33 +993,24 @@ __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] += s[z * plane + i * ld];
     const int ec = p.eb[CONV ? col / p.HWo : col];
-    const float lc = CONV ? p.limc[col] : ec == kBad ? INFINITY : 0.f;
-    int er[4];
-    unsigned low = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        er[i] = p.ea[min(row0 + i, p.M - 1)];
-        const bool is = mine && row0 + i < p.M && !(fabsf(v[i]) >= lc + (er[i] == kBad ? INFINITY : 0.f));
-        low |= (unsigned)is << i;
-    }
-    const int n = __syncthreads_count(low);  // threads with such an element
-    if (n > 16) {
-        block_fp32<KIND, 256, false>(p, row0, (int)blockIdx.x * 256, sums);
-        return;
-    }
+    const float lc = CONV ? p.limc[col] : limit_of(p.tb[col]);
     float* q = place<CONV>(p, row0, col);
     const int64_t ldo = CONV ? p.HWo : p.ldc;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (mine && row0 + i < p.M && !(low >> i & 1))
-            store<CONV>(p, row0 + i, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], er[i] + ec));
-    if (!n) return;
-    if (t == 0) nalone = 0;
-    __syncthreads();
-    for (; low; low &= low - 1) alone[atomicAdd(&nalone, 1)] = (__builtin_ctz(low) << 16) | t;
-    __syncthreads();
-    for (int i = 0; i < nalone; ++i)
-        element_fp32<KIND, 256>(p, row0 + (alone[i] >> 16), (int)blockIdx.x * 256 + (alone[i] & 0xFFFF), sums);
+    for (int i = 0; i < 4; ++i) {
+        const int row = row0 + i;
+        if (row >= p.M) break;
+        const int er = p.ea[row];
+        const float lr = limit_of(KIND == kDense ? p.ta[row] : er == kBad ? kNotFinite : 0u);
+        const bool low = !(fabsf(v[i]) >= lr + lc);
+        if (mine < p.N && !low) store<CONV>(p, row, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], er + ec));
+        // the fp32 path, element by element, a wave's lanes along K
+        for (uint64_t left = __ballot(mine < p.N && low); left; left &= left - 1) {
+            const int l = __builtin_ctzll(left), c = mine - lane + l;
+            const float f = dev::wave_sum(dot_share<KIND>(p, row, c, lane, 64));
+            if (lane == l) store<CONV>(p, row, c, q + i * ldo, f);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1121,11 +1180,12 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     if ((int64_t)q.tm * q.tn * q.splits * 512 >= kMost) return false;
     const size_t pa = up((size_t)steps * M * kRowBytes), pb = up((size_t)steps * N * kRowBytes);
     const size_t ea = up((size_t)M * 4), eb = up((size_t)N * 4);
-    char* s = (char*)try_scratch(pa + pb + ea + eb + q.part_bytes());
+    char* s = (char*)try_scratch(pa + pb + 2 * (ea + eb) + q.part_bytes());
     if (!s) return false;
     SplitArgs p{};
-    const PackRows ra{A, lda, (u16*)s, (int*)(s + pa + pb), (int)M, (int)K, 1, 0, 0};
-    const PackRows rb{B, ldb, (u16*)(s + pa), (int*)(s + pa + pb + ea), (int)N, (int)K, 1, 0, 0};
+    char* const x = s + pa + pb;
+    const PackRows ra{A, lda, (u16*)s, (int*)x, (unsigned*)(x + ea + eb), (int)M, (int)K, 1, 0, 0};
+    const PackRows rb{B, ldb, (u16*)(s + pa), (int*)(x + ea), (unsigned*)(x + 2 * ea + eb), (int)N, (int)K, 1, 0, 0};
     launch_pack(ra, rb, 1);
     p.A = ra.P;
     p.B = rb.P;
@@ -1134,6 +1194,8 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     p.rowA = kRowBytes;
     p.ea = ra.exps;
     p.eb = rb.exps;
+    p.ta = ra.tails;
+    p.tb = rb.tails;
     p.C = C;
     p.ldc = ldc;
     p.bias = bias;
@@ -1145,7 +1207,7 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
     p.tm = q.tm;
     p.tn = q.tn;
     p.splits = q.splits;
-    p.part = (float*)(s + pa + pb + ea + eb);
+    p.part = (float*)(x + 2 * (ea + eb));
     p.A0 = A;
     p.B0 = B;
     p.lda = lda;
@@ -1265,17 +1327,17 @@ bool split_attention(const float* q, const float* k, const float* v, void* out, 
     const size_t eq = up((size_t)qn * Sq * 4), ek = up((size_t)kn * Skv * 4), ev = up((size_t)kn * d * 4);
     const size_t ep = up((size_t)qn * Sq * 4);  // for any round, so that the budget alone decides what a call holds
     const size_t parts = std::max(p1.part_bytes(), p2.part_bytes()), o16 = out16 ? up((size_t)N * Sq * inner * 4) : 0;
-    char* s = (char*)try_scratch(pq + pk + pv + vt + sc + eq + ek + ev + ep + o16 + parts);
+    char* s = (char*)try_scratch(pq + pk + pv + vt + sc + 2 * (eq + ek + ev) + ep + o16 + parts);
     if (!s) return false;
     auto take = [&](size_t n) {
         char* r = s;
         s += n;
         return r;
     };
-    const PackRows rq{q, inner, (u16*)take(pq), (int*)take(eq), (int)Sq, (int)d, heads, Sq * inner, d};
-    const PackRows rk{k, kvi, (u16*)take(pk), (int*)take(ek), (int)Skv, (int)d, kv_heads, Skv * kvi, d};
+    const PackRows rq{q, inner, (u16*)take(pq), (int*)take(eq), (unsigned*)take(eq), (int)Sq, (int)d, heads, Sq * inner, d};
+    const PackRows rk{k, kvi, (u16*)take(pk), (int*)take(ek), (unsigned*)take(ek), (int)Skv, (int)d, kv_heads, Skv * kvi, d};
     float* const tv = (float*)take(vt);
-    const PackRows rv{tv, Skv, (u16*)take(pv), (int*)take(ev), (int)d, (int)Skv, 1, d * Skv, 0};
+    const PackRows rv{tv, Skv, (u16*)take(pv), (int*)take(ev), (unsigned*)take(ev), (int)d, (int)Skv, 1, d * Skv, 0};
     float* const S = (float*)take(sc);
     int* const exps = (int*)take(ep);
     float* const o = out16 ? (float*)take(o16) : (float*)out;
@@ -1314,6 +1376,8 @@ bool split_attention(const float* q, const float* k, const float* v, void* out, 
             p.rowA = kRowBytes;
             p.ea = rq.exps + b0 * Sq + r0;
             p.eb = rk.exps + kb * Skv;
+            p.ta = rq.tails + b0 * Sq + r0;
+            p.tb = rk.tails + kb * Skv;
             p.C = S;
             p.ldc = skp;
             p.outC = heads * m * skp;
@@ -1350,6 +1414,7 @@ bool split_attention(const float* q, const float* k, const float* v, void* out, 
             p.matB = ssteps * d * kRowBytes;
             p.planeB = d * kRowBytes;
             p.eb = rv.exps + kb * d;
+            p.tb = rv.tails + kb * d;
             p.C = o + (n0 * Sq + r0) * inner + h0 * d;
             p.ldc = inner;
             p.outC = Sq * inner;

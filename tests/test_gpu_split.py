@@ -41,6 +41,8 @@ def run_gemm(be, orc, M, N, K, seed, lda=None, bias=True, acc=False, edit=None):
     (700, 260, 8192, None, False, False),    # parts of K
     (4097, 2049, 128, None, True, False),    # 128 x 128, one past the tiles (unaligned C rows)
     (3000, 5000, 160, None, True, True),     # 256 x 256 with remainders
+    # rows that are not a multiple of 16 bytes: the split product at the sizes above that the library takes when aligned
+    (1024, 1032, 1000, 1005, True, True), (130, 4100, 2052, 2053, True, False), (700, 260, 8191, None, False, False),
 ])
 def test_gemm(be, orc, M, N, K, lda, bias, acc):
     got, A, W, b, c0 = run_gemm(be, orc, M, N, K, 4000 + M + K, lda, bias, acc)
@@ -267,8 +269,8 @@ def test_small_arena():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,acc", [
-    (3000, 5000, 160, True), (4097, 2049, 128, False), (1024, 1032, 1000, False),  # 256, 128 and 64 wide tiles
-    (700, 260, 8192, True),  # parts of K
+    (3000, 5000, 160, True), (4097, 2049, 128, False), (1024, 1033, 1000, False),  # 256, 128 and 64 wide tiles
+    (700, 260, 8191, True),  # parts of K
 ])
 def test_gemm_one_bad_row_and_column(be, orc, M, N, K, acc):
     """A NaN in a row of A and infinities in a row of W: the blocks of their
@@ -314,3 +316,56 @@ def test_conv_one_bad_pixel_in_parts(be, orc):
     assert np.array_equal(~np.isfinite(got), bad)
     assert np.all(np.isnan(got[:, 77]))
     assert_gemm(got[~bad], want[~bad], S[~bad], Cin * 9 + 2, "beside a bad pixel and channel")
+
+
+def unlike_groups(orc, shape, axis, seed, spread, pattern):
+    """Values whose channels (along axis) fall into a large and a small group,
+    2^spread apart: interleaved, or two halves."""
+    x = orc.randn(shape, seed)
+    n = shape[axis]
+    large = np.arange(n) % 2 == 0 if pattern == "interleaved" else np.arange(n) < n // 2
+    scale = np.where(large, np.float32(2.0) ** spread, np.float32(1))
+    return x * scale.reshape([-1 if i == axis else 1 for i in range(len(shape))]), large
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spread", [12, 20, 24, 28, 60])
+@pytest.mark.parametrize("pattern", ["interleaved", "halves"])
+@pytest.mark.parametrize("M,N,K", [(300, 333, 641), (2048, 1024, 640), (300, 260, 8191)])
+def test_gemm_unlike_channels(be, orc, M, N, K, pattern, spread):
+    """Rows whose channels differ by 2^spread, met by weights that ignore the
+    large group in every other output and are its reciprocal in some: within
+    the error of fp32 sums of the result's own terms. Bound: K roundings of
+    2^-24 each of partial sums no larger than the result in the mean, which
+    add up as their squares do, 2^-24 sqrt(K) of the result's norm."""
+    def edit(A, W):
+        scaled, large = unlike_groups(orc, A.shape, 1, 5400, spread, pattern)
+        A[:] = scaled
+        W[::2, large] = 0
+        W[1::4, large] *= np.float32(2.0) ** -spread
+
+    got, A, W, _, _ = run_gemm(be, orc, M, N, K, 5400 + K, bias=False, edit=edit)
+    want = A.astype(np.float64) @ W.astype(np.float64).T
+    for part in (np.s_[:, ::2], np.s_[:, 1::4], np.s_[:, 3::4]):
+        err = np.linalg.norm(got[part] - want[part]) / np.linalg.norm(want[part])
+        assert err <= 2.0 ** -24 * np.sqrt(K), (part, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [160, 512])
+def test_wide_attention_unlike_channels(be, orc, d):
+    """Queries whose channels differ by 2^24 and keys that ignore the large
+    ones, values of one channel spread by 2^24 over the keys: scores and
+    outputs as fp32 gives them."""
+    S = 200
+    q, large = unlike_groups(orc, (1, S, d), 2, 5500, 24, "interleaved")
+    k, v = orc.randn((1, S, d), 5501), orc.randn((1, S, d), 5502)
+    k[:, :, large] = 0
+    k[:, :, ~large] *= 2
+    v[0, :, 7] *= np.where(np.arange(S) % 2 == 0, np.float32(2.0 ** 24), 1)
+    out = be.empty((1, S, d))
+    be.attention(be.array(q), be.array(k), be.array(v), out, 1, S, S, 1, 1, d, False)
+    want = orc.attention(q, k, v, 1, False, 1)
+    got = out.download()
+    assert np.max(np.abs(np.delete(got - want, 7, 2))) <= 1e-4
+    assert np.max(np.abs(got[..., 7] - want[..., 7])) <= 1e-5 * 2.0 ** 24
