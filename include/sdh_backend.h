@@ -108,17 +108,21 @@ int sdh_gemm_nt_bf16_packed(int64_t M, int64_t N, int64_t K, const uint16_t* A, 
 /* backend_cuda.h:38-40 gemm_nt_f32(): C[M,N] = A[M,K] * B[N,K]^T (+ C when
  * accumulate) (+ bias[N]), all fp32, row-major with leading dimensions in
  * elements; bias may be NULL. The linear layers whose weights stay fp32. Large
- * products run on fp16 pairs: each operand is within 2^-22 of its value, and of
- * values below 2^-17 of their row's largest within 2^-39 of that one; a result
- * that the latter could move by more than 2^-22 of itself is computed in fp32. */
+ * products run on fp16 pairs: each operand is within 2^-22 of its value, or below
+ * 2^-17 of its row's largest within 2^-39 of that one; a result that values below
+ * 2^-19 could move by more than 2^-20 of itself is computed in fp32. */
 int sdh_gemm_nt_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb,
                     float* C, int64_t ldc, const float* bias, int accumulate);
 /* backend_cuda.h:45-47 conv2d(); tensor.h:159 (tensor.cpp:520-560).
  * x [N, Cin, H, W], w [Cout, Cin, kh, kw] fp32, bias [Cout] or NULL,
  * out [N, Cout, Ho, Wo] with Ho = (H + 2 pad - kh) / stride + 1 (and Wo
- * alike); zero padding. out must not overlap the inputs. An implicit GEMM with
- * fp32 accuracy; it takes scratch of about the size of x and w, or at most
- * 128 MB where the arena has no more. */
+ * alike); zero padding. out must not overlap the inputs. An implicit GEMM on
+ * fp16 pairs, with sdh_gemm_nt_f32's rule for results that the spread of an
+ * operand could cost bits; the spread between blocks of 32 input channels costs
+ * none up to 2^34. It takes ceil(Cin / 32) * 128 bytes of scratch per pixel of x
+ * and per (output channel, tap), and up to 16 times the output where that has few
+ * tiles; where the arena has no room for that, at most 128 MB for gathered
+ * patches. The scratch is kept until an allocation needs the room. */
 int sdh_conv2d(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, const float* w, int64_t Cout, int64_t kh,
                int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo);
 /* Tensor::to_bf16 (tensor.cpp:131-137) on device memory: y[i] = bf16 bits of

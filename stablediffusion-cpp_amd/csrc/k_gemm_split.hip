@@ -11,21 +11,21 @@
 // 2^-23 |x| while |x| >= 2^-16 of the block's largest value and at most 2^-39
 // of that value below it; the dropped lo_a lo_b is at most 2^-24 of the product.
 // Where the values that lose bits this way could matter, fp32 takes over: the
-// pack counts, row by row, the values below 2^-17 of the row's largest that were
-// not held exactly, and a result stands only if its magnitude is at least 2^22
-// times what they can have cost it (kPerTail); else it is computed by fp32
-// FMAs from the original operands. Ordinary rows have no such value or one, and
-// about one result in 10^7 is computed again; a row of unlike groups of
-// channels met by weights that ignore the large ones gives what fp32 gives.
+// pack counts, row by row, the values below 2^-19 of the row's largest that were
+// not held exactly, and a result stands only if its magnitude is at least 2^20
+// times the most that they can have cost it (kPerTail; as a rule they cost a
+// tenth of that); else it is computed by fp32 FMAs from the original operands.
+// Few ordinary rows have such a value, and about one result in 10^8 is computed
+// again; a row of unlike groups of channels met by weights that ignore the
+// large ones gives what fp32 gives.
 // Against 64-bit results the products come out closer than the fp32 MFMA's,
 // whose K additions round one by one where these round once per 16 products.
 //   linear  a block is one row of A, one row of B (one output feature)
-//   conv2d  a block is one output channel's weights; one sample of x
+//   conv2d  a block is one output channel's weights, or 32 channels of a sample
+//           of x (whose scale the weights take over, see the pack)
 // The exponents are exact and are applied to the accumulators at the end.
-// A result whose row or column holds an infinity or a NaN, or (conv2d) sees a run
-// of 256 pixels whose values are all below 2^-14 of the sample's largest (where
-// the bound above would be looser than fp32's), is computed by plain fp32
-// FMAs from the original operands instead, so such inputs give what fp32 gives.
+// A result whose row or column (conv2d: one of its pixels) holds an infinity or a
+// NaN is computed by those FMAs too, so such inputs give what fp32 gives.
 //
 // Packed operands (library scratch): K is cut into steps of 32; a step of a row
 // is 128 bytes, 32 hi halves then 32 lo halves, and all rows of a step lie
@@ -42,6 +42,7 @@
 // v_mfma_f32_32x32x16_f16: lane l holds row l % 32 of A and of B, k (l / 32) * 8 .. + 7;
 // result column l % 32, rows (i / 4) * 8 + (l / 32) * 4 + i % 4.
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "sdh_internal.hpp"
@@ -60,11 +61,10 @@ constexpr int kRowBytes = 128;       // one row of one step: 32 hi, 32 lo
 constexpr int kBad = 1 << 20;        // exponent of a row that holds an infinity or a NaN
 constexpr unsigned kInf = 0x7F800000u;
 constexpr unsigned kNotFinite = 1u << 31;  // in a row's count: it holds an infinity or a NaN
-// A scaled value below 2^-3 is off by at most 2^-25 and meets one below 2^15: 2^-10 of a result
-// before the exponents, and 2^22 times that must be reached.
-constexpr float kPerTail = 4096.f;
+// A scaled value is off by at most 2^-25, which for one below kSmall can be more than 2^-20 of it.
+// It meets one below 2^15: 2^-10 of a result before the exponents, and 2^20 times that must be reached.
+constexpr float kSmall = 0x1p-5f, kPerTail = 1024.f;
 constexpr int kBufferWord3 = 0x00020000;  // raw buffer resource, 32-bit data format
-constexpr int kPixBlock = 256, kChanBlock = 32;  // conv2d: x's maxima are kept per this many pixels and channels
 
 __device__ __forceinline__ unsigned absbits(float x) { return __float_as_uint(x) & 0x7FFFFFFFu; }
 
@@ -91,7 +91,6 @@ __device__ __forceinline__ unsigned wave_usum(unsigned v) {
 // Eight values scaled by 2^s and split; how many of them are small (see kPerTail)
 // and not held exactly, which few waves have to count.
 __device__ __forceinline__ int split8(const float* x, int s, h8& hi, h8& lo) {
-    constexpr float kSmall = 0.125f;
     float least = INFINITY;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -224,134 +223,264 @@ __global__ __launch_bounds__(256, TURNS < 4 ? 8 : 4) void k_split_pack(PackRows 
 }
 
 // ---------------------------------------------------------------------------
-// conv2d's pack. Launch 1: the maxima of x per (sample, 32 channels, 256
-// pixels), and the weights. Launch 2: the pixels, with the sample's exponent.
+// conv2d's pack. Launch 1: the largest values of the weights per row and 32
+// channels, and of x per sample, 32 channels and part of the pixels. Every
+// workgroup of launch 2 reads all of x's, so there are at most kMaxima, or kTable
+// where samples and channels alone are more. Launch 2: the exponents, then the
+// weights and the pixels.
+//
+// Channels of unlike scale: chunk c of 32 channels has an exponent ec of its own
+// besides the sample's es, and the weights of these channels take 2^ec before
+// their row's exponent is found, so that x w keeps its value. With f the largest
+// over the samples of (chunk's exponent - sample's), ec is f / 2: x and w share
+// the spread, and neither loses bits while it is below 2^34, whether the weights
+// are alike, reciprocal to it, or zero where x is large.
 // ---------------------------------------------------------------------------
+constexpr int kTable = 2048, kMaxima = 256;
+
 struct ConvPack {
     const float* x;       // [N, Cin, HW]
     const float* w;       // [Cout, Cin, taps]
-    unsigned* maxima;     // [N, ncb, npb]
+    unsigned* maxima;     // [N, chunks, parts], of finite values
+    unsigned* wmaxima;    // [Cout, chunks]; kInf: not all finite
     u16* X;               // planes of N * HW + 1 pixels
     u16* Wp;              // planes of Cout rows
     int* ex;              // [N]
     int* ew;              // [Cout]
-    unsigned* bad;        // [N, npb]: this run of pixels needs the fp32 path
+    unsigned* tx;         // [N * HW + 1]: counts of the pixels, see kPerTail
+    unsigned* tw;         // [Cout]
     int N, Cin, HW, Cout, taps;
-    int ncb, npb, chunks;  // 32-channel blocks, 256-pixel blocks, 32-channel steps
-    int per;               // 32-channel steps that a workgroup of launch 2 packs
+    int chunks, parts;    // 32-channel steps; parts of the pixels, a power of two
+    int per, groups;      // steps that a workgroup of launch 2 packs; such groups of steps
+    int tiles, run, runs; // 64-pixel tiles of a sample; tiles that a workgroup packs; such runs
 };
 
-__global__ __launch_bounds__(256) void k_conv_prep(ConvPack a, int nmax, int in_lds) {
-    extern __shared__ float row[];
+__global__ __launch_bounds__(256) void k_conv_max(ConvPack a) {
     __shared__ unsigned red[4];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    unsigned m = 0;
-    if ((int)blockIdx.x < nmax) {
-        const int pb = blockIdx.x % a.npb, cb = blockIdx.x / a.npb % a.ncb, n = blockIdx.x / (a.npb * a.ncb);
-        const int c0 = cb * kChanBlock, p = min(pb * kPixBlock + t, a.HW - 1);  // past the last pixel: that one again
-        const float* x = a.x + ((int64_t)n * a.Cin + c0) * a.HW + p;
-        float v[kChanBlock];
+    const int t = threadIdx.x, lane = t & 63, nx = gridDim.x - a.Cout, b = (int)blockIdx.x - a.Cout;
+    if (b < 0) {  // an output channel: a wave per 32 channels
+        const int K = a.Cin * a.taps, chunk = kStep * a.taps, co = blockIdx.x;
+        const float* w = a.w + (int64_t)co * K;
+        constexpr int U = 8;  // loads of a lane on their way at once: 512 weights of a chunk, the next chunk's behind them
+        float v[U], x[U];
+        if (a.taps == 1) {  // half a wave per chunk
+            for (int k0 = t; k0 - lane < a.chunks * kStep; k0 += U * 256) {
 #pragma unroll
-        for (int c = 0; c < kChanBlock; ++c) v[c] = x[(int64_t)min(c, a.Cin - 1 - c0) * a.HW];
+                for (int u = 0; u < U; ++u) v[u] = w[min(k0 + u * 256, K - 1)];
 #pragma unroll
-        for (int c = 0; c < kChanBlock; ++c) m = max(m, absbits(v[c]));
-        m = wave_umax(m);
-        if (lane == 0) red[wv] = m;
-        __syncthreads();
-        if (t == 0) a.maxima[blockIdx.x] = max(max(red[0], red[1]), max(red[2], red[3]));
+                for (int u = 0; u < U; ++u) {
+                    const int c = (k0 + u * 256) / kStep;
+                    const uint64_t bad = __ballot(absbits(v[u]) >= kInf) >> (lane & 32) << 32;
+                    float f = dev::group_max<16>(fabsf(v[u]));
+                    f = fmaxf(f, __shfl_xor(f, 16, 64));
+                    const unsigned m = __float_as_uint(f);
+                    if ((lane & 31) == 0 && c < a.chunks) a.wmaxima[(int64_t)co * a.chunks + c] = bad ? kInf : m;
+                }
+            }
+            return;
+        }
+        auto load = [&](int c, int k0) __attribute__((always_inline)) {  // past the chunk or the row: its last one again
+            const int last = min(K, (c + 1) * chunk) - 1;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k0 + u * 64 < chunk) v[u] = w[min(c * chunk + k0 + u * 64 + lane, last)];
+        };
+        int c = __builtin_amdgcn_readfirstlane(t >> 6);
+        if (c < a.chunks) load(c, 0);
+        for (; c < a.chunks; c += 4) {
+            unsigned m = 0;
+            for (int k0 = 0; k0 < chunk; k0 += U * 64) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) x[u] = v[u];
+                if (k0 + U * 64 < chunk) load(c, k0 + U * 64);
+                else if (c + 4 < a.chunks) load(c + 4, 0);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (k0 + u * 64 < chunk) m = max(m, absbits(x[u]));
+            }
+            const bool bad = __any(m >= kInf);
+            m = __float_as_uint(dev::wave_max(__uint_as_float(m)));
+            if (lane == 0) a.wmaxima[(int64_t)co * a.chunks + c] = bad ? kInf : m;
+        }
         return;
     }
-    // one output channel's weights: [Cin][taps] -> steps (32 channels, tap),
-    // through LDS where the launch gave it room for them
-    const int co = blockIdx.x - nmax, K = a.Cin * a.taps;
-    const float* w = a.w + (int64_t)co * K;
-    if (in_lds) {
-#pragma unroll 8
-        for (int k = t; k < K; k += 256) {
-            const float v = w[k];
-            row[k] = v;
-            m = max(m, absbits(v));
+    for (int i = b * 256 + t; i <= a.N * a.HW; i += nx * 256) a.tx[i] = 0;
+    const int part = b % a.parts, c0 = b / a.parts % a.chunks * kStep, n = b / (a.parts * a.chunks);
+    const float* x = a.x + ((int64_t)n * a.Cin + c0) * a.HW;
+    unsigned m = 0;
+    for (int64_t p0 = part * 256; p0 < a.HW; p0 += a.parts * 256) {
+        const int p = min((int)p0 + t, a.HW - 1);  // past the last pixel: that one again
+        float v[kStep];
+#pragma unroll
+        for (int c = 0; c < kStep; ++c) v[c] = x[(int64_t)min(c, a.Cin - 1 - c0) * a.HW + p];
+#pragma unroll
+        for (int c = 0; c < kStep; ++c) {
+            const unsigned b = absbits(v[c]);
+            m = max(m, b < kInf ? b : 0u);
         }
-    } else {
-#pragma unroll 8
-        for (int k = t; k < K; k += 256) m = max(m, absbits(w[k]));
     }
     m = wave_umax(m);
-    if (lane == 0) red[wv] = m;
+    if ((t & 63) == 0) red[t >> 6] = m;
     __syncthreads();
-    const int e = exp_of(max(max(red[0], red[1]), max(red[2], red[3])));
-    if (t == 0) a.ew[co] = e;
+    if (t == 0) a.maxima[b] = max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
+// Exponents from the maxima: E [N, chunks], the chunks' biased ones (bits >> 23, at
+// least 1; 0: all zero), and ec [chunks]. By the whole workgroup.
+__device__ __forceinline__ int wave_imax(int v) { return (int)dev::wave_max((float)v); }  // |v| < 2^24
+__device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) {
+    constexpr int kNone = -1000;
+    const int t = threadIdx.x, lane = t & 63, words = a.N * a.chunks * a.parts;
+    for (int i0 = t - lane; i0 < words; i0 += 256) {
+        const int i = i0 + lane;
+        unsigned m = i < words ? a.maxima[i] : 0u;
+        for (int o = 1; o < a.parts; o <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
+        if (lane % a.parts == 0 && i < words) E[i / a.parts] = m ? max((int)(m >> 23), 1) : 0;
+    }
+    for (int c = t; c < a.chunks; c += 256) ec[c] = kNone;
+    __syncthreads();
+    // a chunk's largest (own - sample's) over the samples; many chunks have few samples (kTable)
+    if (a.chunks <= 32) {  // a lane per sample
+        for (int n0 = t - lane; n0 < a.N; n0 += 256) {
+            const int n = min(n0 + lane, a.N - 1);
+            int whole = 0;
+            for (int c = 0; c < a.chunks; ++c) whole = max(whole, E[n * a.chunks + c]);
+            for (int c = 0; c < a.chunks; ++c) {
+                const int own = E[n * a.chunks + c], f = wave_imax(own ? own - whole : kNone);
+                if (lane == 0) atomicMax(ec + c, f);
+            }
+        }
+    } else {  // a thread per chunk
+        for (int n = 0; n < a.N; ++n) {
+            int whole = 0;
+            for (int c = lane; c < a.chunks; c += 64) whole = max(whole, E[n * a.chunks + c]);
+            whole = wave_imax(whole);
+            for (int c = t; c < a.chunks; c += 256) {
+                const int own = E[n * a.chunks + c];
+                if (own) ec[c] = max(ec[c], own - whole);
+            }
+        }
+    }
+    __syncthreads();
+    for (int c = t; c < a.chunks; c += 256) ec[c] = ec[c] == kNone ? 0 : ec[c] / 2;  // from -126 on
+    __syncthreads();
+}
+// A sample's exponent beside those: its scaled values lie below 2^15.
+__device__ __forceinline__ int conv_sample_exp(const ConvPack& a, const int* E, const int* ec, int n) {
+    constexpr int kNone = -1000;
+    int e = kNone;
+    for (int c = threadIdx.x & 63; c < a.chunks; c += 64) {
+        const int own = E[n * a.chunks + c];
+        e = max(e, own ? own - 141 - ec[c] : kNone);
+    }
+    e = wave_imax(e);
+    return e == kNone ? 0 : e;
+}
+
+// One output channel's weights: [Cin][taps] -> steps (32 channels, tap).
+__device__ __forceinline__ void conv_pack_weights(const ConvPack& a, int co, const int* ec, unsigned* red) {
+    const int t = threadIdx.x, lane = t & 63, K = a.Cin * a.taps;
+    const float* w = a.w + (int64_t)co * K;
+    // its exponent: every wave finds it; a chunk of zeros counts as the smallest weights
+    int m = -1000;
+    bool bad = false;
+    for (int c = lane; c < a.chunks; c += 64) {
+        const unsigned b = a.wmaxima[(int64_t)co * a.chunks + c];
+        bad |= b >= kInf;
+        m = max(m, (int)(b >> 23) + ec[c]);
+    }
+    bad = __any(bad);
+    const int e = wave_imax(m) - 141;  // scaled by 2^(ec - e) the largest lies below 2^15
+    if (t == 0) a.ew[co] = bad ? kBad : e;
     const int tasks = a.chunks * a.taps * 4;
+    unsigned tail = 0;
     for (int i = t; i < tasks; i += 256) {  // eight channels of one step
-        const int g = i & 3, step = i >> 2, chunk = step / a.taps, tap = step - chunk * a.taps, c0 = chunk * kStep + g * 8;
+        const int g = i & 3, step = i >> 2, c = step / a.taps, tap = step - c * a.taps, c0 = c * kStep + g * 8;
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int k = (c0 + j) * a.taps + tap;
-            v[j] = c0 + j < a.Cin ? (in_lds ? row[k] : w[k]) : 0.f;
+            const float x = w[min((c0 + j) * a.taps + tap, K - 1)];
+            v[j] = c0 + j < a.Cin ? x : 0.f;
         }
-        store_split(a.Wp + ((int64_t)step * a.Cout + co) * (kRowBytes / 2) + g * 8, v, e == kBad ? 0 : -e);
+        tail += store_split(a.Wp + ((int64_t)step * a.Cout + co) * (kRowBytes / 2) + g * 8, v, bad ? 0 : ec[c] - e);
+    }
+    tail = __any(tail != 0) ? wave_usum(tail) : 0u;
+    if (lane == 0) red[t >> 6] = tail;
+    __syncthreads();
+    if (t == 0) a.tw[co] = bad ? kNotFinite : (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// `run` times 64 pixels of a sample, `per` steps of 32 channels; each step through
+// LDS, so that x is read in runs of 64 pixels and a step of 64 pixels is written
+// as 8 KB in a row.
+template <class Scales>
+__device__ __forceinline__ void conv_pack_pixels(const ConvPack& a, int b, const int* E, const int* ec, u16* tile,
+                                                 Scales&& scales) {
+    const int t = threadIdx.x, lane = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int run = b % a.runs, group = b / a.runs % a.groups, n = b / (a.runs * a.groups);
+    const int s0 = group * a.per, s1 = min(a.chunks, s0 + a.per);
+    float v[8];
+    auto load = [&](int p, int s) __attribute__((always_inline)) {  // channels past the last: that one again, dropped below
+        const int c0 = s * kStep + g * 8;
+        const float* x = a.x + (int64_t)n * a.Cin * a.HW;
+        const int pix = min(p * 64 + lane, a.HW - 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = x[(int64_t)min(c0 + j, a.Cin - 1) * a.HW + pix];
+    };
+    load(run * a.run, s0);
+    scales();  // behind the first loads
+    const int e = conv_sample_exp(a, E, ec, n);
+    if (run == 0 && group == 0 && t == 0) a.ex[n] = e;
+    const int64_t prows = (int64_t)a.N * a.HW + 1;
+    const int p1 = min(a.tiles, (run + 1) * a.run);
+    for (int p = run * a.run; p < p1; ++p) {
+        const int p0 = p * 64, pix = p0 + lane;
+        unsigned tail = 0;
+        for (int s = s0; s < s1; ++s) {
+            const int c0 = s * kStep + g * 8;
+            unsigned m = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                v[j] = c0 + j < a.Cin ? v[j] : 0.f;
+                m = max(m, absbits(v[j]));
+            }
+            h8 hi, lo;
+            const unsigned c = split8(v, -(e + ec[s]), hi, lo);
+            tail = (tail + c) | (m >= kInf ? kNotFinite : 0u);  // the count stays far below the mark
+            const bool last = s + 1 == s1;
+            if (!last || p + 1 < p1) load(last ? p + 1 : p, last ? s0 : s + 1);
+            __syncthreads();  // the previous step's tile is read
+            *(h8*)(tile + lane * 64 + ((g ^ (lane & 7)) << 3)) = hi;
+            *(h8*)(tile + lane * 64 + (((g + 4) ^ (lane & 7)) << 3)) = lo;
+            __syncthreads();
+            u16* out = a.X + ((int64_t)s * prows + (int64_t)n * a.HW + p0) * 64;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int i = t + j * 256, r = i >> 3, k = i & 7;
+                if (p0 + r < a.HW) *(h8*)(out + i * 8) = *(const h8*)(tile + r * 64 + ((k ^ (r & 7)) << 3));
+            }
+            if (n == a.N - 1 && p0 + 64 >= a.HW && t < 8)  // the row of zeros
+                *(u32x4*)(a.X + ((int64_t)s * prows + prows - 1) * 64 + t * 8) = u32x4{0, 0, 0, 0};
+        }
+        if (tail && pix < a.HW) {  // rare; whole numbers, so that the order does not matter
+            unsigned* at = a.tx + (int64_t)n * a.HW + pix;
+            if (tail >= kNotFinite) atomicOr(at, kNotFinite);
+            else atomicAdd(at, tail);
+        }
     }
 }
 
-// One workgroup: 64 pixels of a sample, `per` steps of 32 channels; each step
-// through LDS, so that x is read in runs of 64 pixels and a step of 64 pixels is
-// written as 8 KB in a row. Grid: (pixel tiles, channel groups, samples).
 __global__ __launch_bounds__(256) void k_conv_pack(ConvPack a) {
+    extern __shared__ int lds[];
     __shared__ unsigned red[4];
     __shared__ __attribute__((aligned(16))) u16 tile[64 * 64];
-    const int t = threadIdx.x, lane = t & 63, g = t >> 6, n = blockIdx.z;
-    const unsigned* mx = a.maxima + (int64_t)n * a.ncb * a.npb;
-    unsigned m = 0;
-    for (int i = t; i < a.ncb * a.npb; i += 256) {
-        const unsigned v = mx[i];
-        if (v < kInf) m = max(m, v);
-    }
-    m = wave_umax(m);
-    if (lane == 0) red[g] = m;
-    __syncthreads();
-    m = max(max(red[0], red[1]), max(red[2], red[3]));
-    const int e = exp_of(m);
-    const int p0 = blockIdx.x * 64, pix = p0 + lane;
-    if (blockIdx.y == 0 && t == 0) {
-        if (p0 == 0) a.ex[n] = e;
-        if (p0 % kPixBlock == 0) {
-            const int pb = p0 / kPixBlock;
-            unsigned b = 0;
-            for (int c = 0; c < a.ncb; ++c) b = max(b, mx[c * a.npb + pb]);
-            // not finite, or all of it below 2^-14 of the sample's largest (14 << 23 in exponent bits)
-            a.bad[n * a.npb + pb] = b >= kInf || (b != 0 && b + (14u << 23) < m) ? 1u : 0u;
-        }
-    }
-    const int64_t prows = (int64_t)a.N * a.HW + 1;
-    const int s0 = blockIdx.y * a.per, s1 = min(a.chunks, s0 + a.per);
-    float v[8];
-    auto load = [&](int s) __attribute__((always_inline)) {  // channels past the last: that one again, dropped below
-        const int c0 = s * kStep + g * 8;
-        const float* x = a.x + (int64_t)n * a.Cin * a.HW + min(pix, a.HW - 1);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = x[(int64_t)min(c0 + j, a.Cin - 1) * a.HW];
-    };
-    load(s0);
-    for (int s = s0; s < s1; ++s) {
-        const int c0 = s * kStep + g * 8;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = c0 + j < a.Cin ? v[j] : 0.f;
-        h8 hi, lo;
-        split8(v, -e, hi, lo);
-        if (s + 1 < s1) load(s + 1);
-        __syncthreads();  // the previous step's tile is read
-        *(h8*)(tile + lane * 64 + ((g ^ (lane & 7)) << 3)) = hi;
-        *(h8*)(tile + lane * 64 + (((g + 4) ^ (lane & 7)) << 3)) = lo;
-        __syncthreads();
-        u16* out = a.X + ((int64_t)s * prows + (int64_t)n * a.HW + p0) * 64;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int i = t + j * 256, r = i >> 3, c = i & 7;
-            if (p0 + r < a.HW) *(h8*)(out + i * 8) = *(const h8*)(tile + r * 64 + ((c ^ (r & 7)) << 3));
-        }
-        if (n == a.N - 1 && p0 + 64 >= a.HW && t < 8)  // the row of zeros
-            *(u32x4*)(a.X + ((int64_t)s * prows + prows - 1) * 64 + t * 8) = u32x4{0, 0, 0, 0};
+    int *E = lds, *ec = E + a.N * a.chunks;
+    auto scales = [&]() __attribute__((always_inline)) { conv_scales(a, E, ec); };
+    if ((int)blockIdx.x < a.Cout) {
+        scales();
+        conv_pack_weights(a, blockIdx.x, ec, red);
+    } else {
+        conv_pack_pixels(a, blockIdx.x - a.Cout, E, ec, tile, scales);
     }
 }
 
@@ -367,7 +496,7 @@ struct SplitArgs {
     int rowA;                // bytes from one row of A's step to the next
     const int* ea;           // per row
     const int* eb;           // per column; conv2d: per sample
-    const unsigned* ta;      // counts per row (kDense), per column (not conv2d): see kPerTail
+    const unsigned* ta;      // counts per row (not kWeights), per column; conv2d: per pixel: see kPerTail
     const unsigned* tb;
     float* C;
     int64_t ldc;
@@ -387,8 +516,7 @@ struct SplitArgs {
     const float* B0;
     int64_t lda, ldb;
     // conv2d
-    const unsigned* bad;
-    int H, W, Wo, HWo, kh, kw, stride, pad, taps, Cin, Cout, npb, zero;
+    int H, W, Wo, HWo, kh, kw, stride, pad, taps, Cin, Cout, zero;
 };
 
 // Where element (row, col) lies, and what is added to it.
@@ -452,12 +580,12 @@ __device__ __forceinline__ float dot_share(const SplitArgs& p, int row, int col,
         const int e = p.ea[row], end = weights_of(p, row);
         if (e == kBad) return __builtin_nanf("");
         const float* b = p.B0 + (int64_t)col * p.ldb;
-#pragma unroll 4
+#pragma unroll 8
         for (int k = t; k < end; k += T) s = fmaf(packed_weight(p, row, e, k), b[k], s);
     } else {
         const float* a = p.A0 + (int64_t)row * p.lda;
         const float* b = p.B0 + (int64_t)col * p.ldb;
-#pragma unroll 4
+#pragma unroll 8
         for (int k = t; k < p.K; k += T) s = fmaf(a[k], b[k], s);
     }
     return s;
@@ -739,22 +867,25 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
         const int row = min(m0 + i, p.M - 1), e = p.ea[row];
         sea[i] = e;
         if (CONV) sbias[i] = p.bias ? p.bias[row] : 0.f;
-        slr[i] = limit(KIND == kDense ? p.ta[row] : e == kBad ? kNotFinite : 0u);
+        slr[i] = limit(KIND == kWeights ? (e == kBad ? kNotFinite : 0u) : p.ta[row]);
     }
     for (int i = t; i < BN; i += T) {
         const int col = min(n0 + i, p.N - 1);
         if constexpr (CONV) {
             const int n = col / p.HWo, q = col - n * p.HWo, oy = q / p.Wo, ox = q - oy * p.Wo;
             seb[i] = p.eb[n];
-            const int xa = min(max(ox * p.stride - p.pad, 0), p.W - 1);
-            const int xb = min(max(ox * p.stride - p.pad + p.kw - 1, 0), p.W - 1);
-            bool bad = false;
-            for (int ky = 0; ky < p.kh; ++ky) {
-                const int iy = min(max(oy * p.stride - p.pad + ky, 0), p.H - 1);
-                for (int b = (iy * p.W + xa) / kPixBlock; b <= (iy * p.W + xb) / kPixBlock; ++b)
-                    bad |= p.bad[n * p.npb + b] != 0;
+            unsigned tail = 0, bad = 0;  // of all pixels that the column sees
+            int ky = 0, kx = 0;
+#pragma unroll 4
+            for (int tap = 0; tap < p.taps; ++tap) {
+                const int iy = oy * p.stride - p.pad + ky, ix = ox * p.stride - p.pad + kx;
+                const bool in = (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
+                const unsigned c = p.tb[in ? (n * p.H + iy) * p.W + ix : p.zero];
+                tail += c & ~kNotFinite;
+                bad |= c & kNotFinite;
+                if (++kx == p.kw) kx = 0, ++ky;
             }
-            slc[i] = limit(bad ? kNotFinite : 0u);
+            slc[i] = limit(bad ? kNotFinite : tail);
             if (p.splits > 1 && z == 0 && mt == 0 && n0 + i < p.N) p.limc[col] = slc[i];
         } else {
             const int e = p.eb[col];
@@ -983,7 +1114,9 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), BM * BN > 128 * 128 ? 1
 template <Kind KIND>
 __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) {
     constexpr bool CONV = KIND == kConv;
-    const int lane = threadIdx.x & 63, row0 = blockIdx.y * 4, mine = blockIdx.x * 256 + threadIdx.x;
+    __shared__ float sums[4];
+    __shared__ uint64_t left[4][4];  // the lanes of wave w whose row i the fp32 path takes
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, row0 = blockIdx.y * 4, mine = blockIdx.x * 256 + threadIdx.x;
     const int col = min(mine, p.N - 1);
     const int64_t ld = (int64_t)p.tn * BN, plane = (int64_t)p.tm * BM * ld;
     const float* s = p.part + row0 * ld + col;  // whole tiles: rows past the matrix are there
@@ -998,19 +1131,19 @@ __global__ __launch_bounds__(256) void k_split_sum(SplitArgs p, int BM, int BN) 
     const int64_t ldo = CONV ? p.HWo : p.ldc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int row = row0 + i;
-        if (row >= p.M) break;
-        const int er = p.ea[row];
-        const float lr = limit_of(KIND == kDense ? p.ta[row] : er == kBad ? kNotFinite : 0u);
-        const bool low = !(fabsf(v[i]) >= lr + lc);
-        if (mine < p.N && !low) store<CONV>(p, row, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], er + ec));
-        // the fp32 path, element by element, a wave's lanes along K
-        for (uint64_t left = __ballot(mine < p.N && low); left; left &= left - 1) {
-            const int l = __builtin_ctzll(left), c = mine - lane + l;
-            const float f = dev::wave_sum(dot_share<KIND>(p, row, c, lane, 64));
-            if (lane == l) store<CONV>(p, row, c, q + i * ldo, f);
-        }
+        const int row = row0 + i, at = min(row, p.M - 1), er = p.ea[at];
+        const float lr = limit_of(KIND == kWeights ? (er == kBad ? kNotFinite : 0u) : p.ta[at]);
+        const bool in = mine < p.N && row < p.M, low = !(fabsf(v[i]) >= lr + lc);
+        if (in && !low) store<CONV>(p, row, col, q + i * ldo, __builtin_amdgcn_ldexpf(v[i], er + ec));
+        const uint64_t b = __ballot(in && low);
+        if (lane == 0) left[wv][i] = b;
     }
+    __syncthreads();
+    if (!__any(lane < 16 && left[lane >> 2 & 3][lane & 3])) return;
+    for (int w = 0; w < 4; ++w)
+        for (int i = 0; i < 4; ++i)
+            for (uint64_t b = left[w][i]; b; b &= b - 1)
+                element_fp32<KIND, 256>(p, row0 + i, (int)blockIdx.x * 256 + w * 64 + __builtin_ctzll(b), sums);
 }
 
 // ---------------------------------------------------------------------------
@@ -1164,7 +1297,6 @@ void launch_pack(const PackRows& a, const PackRows& b, int64_t batches) {
     go<<<dim3(ba + bb, (unsigned)batches), 256, 0, stream()>>>(a, b, (int)ba);
 }
 
-constexpr size_t kRowLds = 48 << 10;  // weights of one output channel that k_conv_prep takes through LDS
 constexpr int64_t kMost = int64_t(1) << 31;
 
 }  // namespace
@@ -1220,79 +1352,95 @@ bool split_gemm(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, co
 bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, const float* w, int64_t Cout, int64_t kh,
                 int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo) {
     const int64_t HW = H * W, HWo = Ho * Wo, taps = kh * kw, chunks = (Cin + kStep - 1) / kStep, steps = chunks * taps;
-    const int64_t cols = N * HWo, prows = N * HW + 1;
+    const int64_t cols = N * HWo;
     // 32-bit offsets, also of a padded tile's first pixel
     if ((N * HW + (int64_t)pad * (W + 1) + 1) * kRowBytes >= kMost || cols >= kMost - 256 || Cout * kRowBytes >= kMost ||
         steps >= kMost || Cin * taps >= kMost || N > 65535 || N * Cin * HW >= kMost * 64)
         return false;
-    const Plan q = plan_of(Cout, cols, steps);
-    if ((int64_t)q.tm * q.tn * q.splits * 512 >= kMost) return false;
-    ConvPack a{};
-    a.ncb = (int)((Cin + kChanBlock - 1) / kChanBlock);
-    a.npb = (int)((HW + kPixBlock - 1) / kPixBlock);
+    // samples at a time: the exponents' table of one call of the pack is bounded
+    const int64_t most = std::min(N, kTable / chunks);
+    if (most == 0) return false;
+    const auto plan = [&](int64_t ns) { return plan_of(Cout, ns * HWo, steps); };
+    const auto grid = [](const Plan& q) { return (int64_t)q.tm * q.tn * q.splits; };
+    const Plan whole = plan(most), rest = plan(N % most ? N % most : most);
+    if (std::max(grid(whole), grid(rest)) * 512 >= kMost) return false;
+    const int64_t prows = most * HW + 1;
     const size_t px = up((size_t)chunks * prows * kRowBytes), pw = up((size_t)steps * Cout * kRowBytes);
-    const size_t mx = up((size_t)N * a.ncb * a.npb * 4), bd = up((size_t)N * a.npb * 4);
-    const size_t ex = up((size_t)N * 4), ew = up((size_t)Cout * 4), lc = q.splits > 1 ? up((size_t)cols * 4) : 0;
-    char* s = (char*)try_scratch(px + pw + mx + bd + ex + ew + lc + q.part_bytes());
+    const size_t mx = up((size_t)kTable * 4), wm = up((size_t)(Cout * chunks) * 4), tx = up((size_t)prows * 4), ex = up((size_t)most * 4);
+    const size_t ew = up((size_t)Cout * 4), lc = up((size_t)most * HWo * 4);
+    char* s = (char*)try_scratch(px + pw + mx + wm + tx + ex + 2 * ew + lc + std::max(whole.part_bytes(), rest.part_bytes()));
     if (!s) return false;
-    a.x = x;
+    ConvPack a{};
     a.w = w;
     a.X = (u16*)s;
     a.Wp = (u16*)(s += px);
     a.maxima = (unsigned*)(s += pw);
-    a.bad = (unsigned*)(s += mx);
-    a.ex = (int*)(s += bd);
+    a.wmaxima = (unsigned*)(s += mx);
+    a.tx = (unsigned*)(s += wm);
+    a.ex = (int*)(s += tx);
     a.ew = (int*)(s += ex);
-    a.N = (int)N;
+    a.tw = (unsigned*)(s += ew);
+    float* const limc = (float*)(s += ew);
+    float* const part = (float*)(s + lc);
     a.Cin = (int)Cin;
     a.HW = (int)HW;
     a.Cout = (int)Cout;
     a.taps = (int)taps;
     a.chunks = (int)chunks;
-    const int nmax = (int)(N * a.ncb * a.npb), pt = (int)((HW + 63) / 64);
-    // all channels of a pixel tile in one workgroup where that leaves at least four workgroups per CU
-    const int64_t groups = std::min<int64_t>(chunks, std::max<int64_t>(1, (4 * num_cus() + pt * N - 1) / (pt * N)));
-    a.per = (int)((chunks + groups - 1) / groups);
-    const size_t row = (size_t)(Cin * taps) * 4;
-    const bool in_lds = row <= kRowLds;
-    k_conv_prep<<<(unsigned)(nmax + Cout), 256, in_lds ? row : 0, stream()>>>(a, nmax, in_lds ? 1 : 0);
-    k_conv_pack<<<dim3((unsigned)pt, (unsigned)((chunks + a.per - 1) / a.per), (unsigned)N), 256, 0, stream()>>>(a);
-    SplitArgs p{};
-    p.A = a.Wp;
-    p.B = a.X;
-    p.planeA = Cout * kRowBytes;
-    p.planeB = prows * kRowBytes;
-    p.rowA = kRowBytes;
-    p.ea = a.ew;
-    p.eb = a.ex;
-    p.C = out;
-    p.bias = bias;
-    p.M = (int)Cout;
-    p.N = (int)cols;
-    p.K = (int)(Cin * taps);
-    p.steps = (int)steps;
-    p.tm = q.tm;
-    p.tn = q.tn;
-    p.splits = q.splits;
-    p.limc = (float*)(s += ew);
-    p.part = (float*)(s + lc);
-    p.A0 = w;
-    p.B0 = x;
-    p.bad = a.bad;
-    p.H = (int)H;
-    p.W = (int)W;
-    p.Wo = (int)Wo;
-    p.HWo = (int)HWo;
-    p.kh = (int)kh;
-    p.kw = (int)kw;
-    p.stride = stride;
-    p.pad = pad;
-    p.taps = (int)taps;
-    p.Cin = (int)Cin;
-    p.Cout = (int)Cout;
-    p.npb = a.npb;
-    p.zero = (int)(prows - 1);
-    launch_mm<kConv>(q, p);
+    a.tiles = (int)((HW + 63) / 64);
+    in_pieces(N, most, [&](int64_t n0, int64_t ns) {
+        const Plan& q = ns == most ? whole : rest;
+        a.x = x + n0 * Cin * HW;
+        a.N = (int)ns;
+        a.parts = 1;
+        while (a.parts < 64 && a.parts * 256 < HW && ns * chunks * a.parts * 2 <= kMaxima) a.parts *= 2;
+        // all channels of a pixel tile in one workgroup where that leaves at least four workgroups per
+        // CU, and several tiles where it leaves sixteen rounds of those
+        const int64_t pt = a.tiles * ns;
+        a.groups = (int)std::min<int64_t>(chunks, std::max<int64_t>(1, (4 * num_cus() + pt - 1) / pt));
+        a.per = (int)((chunks + a.groups - 1) / a.groups);
+        a.groups = (int)((chunks + a.per - 1) / a.per);
+        a.run = (int)std::max<int64_t>(1, pt * a.groups / (64 * num_cus()));
+        a.runs = (a.tiles + a.run - 1) / a.run;
+        k_conv_max<<<(unsigned)(Cout + ns * chunks * a.parts), 256, 0, stream()>>>(a);
+        k_conv_pack<<<(unsigned)(Cout + (int64_t)a.runs * a.groups * ns), 256, (size_t)((ns + 1) * chunks) * 4, stream()>>>(a);
+        SplitArgs p{};
+        p.A = a.Wp;
+        p.B = a.X;
+        p.planeA = Cout * kRowBytes;
+        p.planeB = (ns * HW + 1) * kRowBytes;
+        p.rowA = kRowBytes;
+        p.ea = a.ew;
+        p.eb = a.ex;
+        p.ta = a.tw;
+        p.tb = a.tx;
+        p.C = out + n0 * Cout * HWo;
+        p.bias = bias;
+        p.M = (int)Cout;
+        p.N = (int)(ns * HWo);
+        p.K = (int)(Cin * taps);
+        p.steps = (int)steps;
+        p.tm = q.tm;
+        p.tn = q.tn;
+        p.splits = q.splits;
+        p.limc = limc;
+        p.part = part;
+        p.A0 = w;
+        p.B0 = a.x;
+        p.H = (int)H;
+        p.W = (int)W;
+        p.Wo = (int)Wo;
+        p.HWo = (int)HWo;
+        p.kh = (int)kh;
+        p.kw = (int)kw;
+        p.stride = stride;
+        p.pad = pad;
+        p.taps = (int)taps;
+        p.Cin = (int)Cin;
+        p.Cout = (int)Cout;
+        p.zero = (int)(ns * HW);
+        launch_mm<kConv>(q, p);
+    });
     return true;
 }
 

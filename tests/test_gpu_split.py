@@ -369,3 +369,95 @@ def test_wide_attention_unlike_channels(be, orc, d):
     got = out.download()
     assert np.max(np.abs(np.delete(got - want, 7, 2))) <= 1e-4
     assert np.max(np.abs(got[..., 7] - want[..., 7])) <= 1e-5 * 2.0 ** 24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spread", [12, 20, 28, 60])
+@pytest.mark.parametrize("pattern", ["interleaved", "halves", "dim chunk"])
+@pytest.mark.parametrize("N,Cin,H,W,Cout,k", [(1, 128, 20, 24, 70, 3), (3, 96, 9, 8, 66, 1), (2, 640, 8, 8, 260, 3)])
+def test_conv_unlike_channels(be, orc, N, Cin, H, W, Cout, k, pattern, spread):
+    """Channels that differ by 2^spread (within a chunk of 32, between chunks,
+    one small chunk), met by weights that ignore the large ones, are their
+    reciprocal, or are alike: the bound of test_gemm_unlike_channels."""
+    if pattern == "dim chunk":
+        x = orc.randn((N, Cin, H, W), 5600)
+        large = np.arange(Cin) >= 32
+        x[:, large] *= np.float32(2.0) ** spread
+    else:
+        x, large = unlike_groups(orc, (N, Cin, H, W), 1, 5600, spread, pattern)
+    w = orc.randn((Cout, Cin, k, k), 5601, 0.0, 0.1)
+    w[::3, large] = 0
+    w[1::3, large] *= np.float32(2.0) ** -spread
+    out = be.empty((N, Cout, H, W))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, k, k, None, 1, k // 2, out, H, W)
+    want, _ = orc.conv2d(x, w, None, 1, k // 2)
+    got = out.download()
+    for part in range(3):
+        err = np.linalg.norm(got[:, part::3] - want[:, part::3]) / np.linalg.norm(want[:, part::3])
+        assert err <= 2.0 ** -24 * np.sqrt(Cin * k * k), (part, err)
+
+
+@pytest.mark.gpu
+def test_conv_unlike_pixels(be, orc):
+    """Image rows 2^26 apart inside one run of 256 pixels, a zero chunk of
+    channels, a zero sample: each output within the error of its own terms."""
+    N, Cin, H, W, Cout = 3, 96, 32, 16, 40
+    x = orc.randn((N, Cin, H, W), 5700)
+    x[:, :, 8:] *= np.float32(2.0 ** -26)
+    x[:, 32:64] = 0
+    x[2] = 0
+    w = orc.randn((Cout, Cin, 3, 3), 5701, 0.0, 0.1)
+    out = be.empty((N, Cout, H, W))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, 3, 3, None, 1, 1, out, H, W)
+    want, _ = orc.conv2d(x, w, None, 1, 1)
+    got = out.download()
+    assert np.all(got[2] == 0)
+    for part in (np.s_[:2, :, :8], np.s_[:2, :, 9:]):
+        err = np.linalg.norm(got[part] - want[part]) / np.linalg.norm(want[part])
+        assert err <= 2.0 ** -24 * np.sqrt(Cin * 9), (part, err)
+
+
+@pytest.mark.gpu
+def test_conv_many_samples(be, orc):
+    """More samples than the pack's table of exponents takes at once."""
+    N, Cin, H, W, Cout = 700, 130, 3, 5, 24  # 5 chunks: 409 samples at a time, then 291
+    x = orc.randn((N, Cin, H, W), 5800) * np.exp2(np.arange(N, dtype=np.float32) % 40)[:, None, None, None]
+    w = orc.randn((Cout, Cin, 3, 3), 5801, 0.0, 0.03)
+    b = orc.randn((Cout,), 5802)
+    out = be.empty((N, Cout, H, W))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, 3, 3, be.array(b), 1, 1, out, H, W)
+    want, S = orc.conv2d(x, w, b, 1, 1)
+    assert_gemm(out.download(), want, S, Cin * 9 + 2, "many samples")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Cin,H,W,Cout,k", [(1, 70, 9, 11, 5, 1), (1, 2100, 3, 4, 9, 1), (2, 33, 6, 5, 7, 3),
+                                              (1, 20, 24, 23, 6, 23), (1, 2000, 4, 4, 10, 3)])
+def test_conv_weights_of_any_scale(be, orc, N, Cin, H, W, Cout, k):
+    """Each output channel's weights have their own exponent, found per 32
+    channels: 2^+-60, one large weight at the row's either end, zeros, subnormal
+    weights, and rows that hold an infinity or NaN at either end."""
+    x = orc.randn((N, Cin, H, W), 5900)
+    w = orc.randn((Cout, Cin, k, k), 5901, 0.0, 0.1)
+    flat = w.reshape(Cout, -1)
+    flat[0] *= np.float32(2.0 ** 60)
+    flat[1] *= np.float32(2.0 ** -60)
+    flat[2, -1], flat[3, 0] = 1000, -1000
+    flat[4] = 0
+    bad = {}
+    if Cout > 6:
+        flat[5] = np.float32(2.0 ** -140) * np.rint(flat[5] * 1000)
+    if Cout > 8:
+        flat[7, -1], flat[8, 0] = np.inf, np.nan
+        bad = {7, 8}
+    out = be.empty((N, Cout, H, W))
+    be.conv2d(be.array(x), N, Cin, H, W, be.array(w), Cout, k, k, None, 1, k // 2, out, H, W)
+    got = out.download()
+    with np.errstate(invalid="ignore"):
+        want, S = orc.conv2d(x, w, None, 1, k // 2)
+    for co in range(Cout):
+        if co in bad:
+            assert np.array_equal(np.isnan(got[:, co]), np.isnan(want[:, co]))
+            assert not np.any(np.isfinite(got[:, co]) & ~np.isfinite(want[:, co]))
+        else:
+            assert_gemm(got[:, co], want[:, co], S[:, co] + 2.0 ** -126, Cin * k * k + 2, f"channel {co}")
