@@ -1062,7 +1062,8 @@ void run_attention(const float* q, const float* k, const float* v, void* out, bo
         // library GEMMs that took long sequences of aligned rows): [2,64,8x160]
         // 16 / 24, [2,256,8x160] to 77 keys 41 / 28, [2,256,8x160] 138 / 35, [1,450,512]
         // 244 / 33, [1,2745,512] 2997 / 108, [1,4096,512] 329* / 151, [1,16384,512]
-        // 4124* / 1875 (293 TFLOP/s).
+        // 4124* / 1875 (293 TFLOP/s). Few queries to few keys stay for the smaller error
+        // ([1,64,8x160] to 77 keys 20 / 24 us, 4.1e-7 / 2.7e-7 off).
         launched(op);
         reserve_blaslt();
     } else if (!(Sq * Skv >= (int64_t(1) << 18) &&

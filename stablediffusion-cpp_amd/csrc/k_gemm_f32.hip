@@ -134,11 +134,15 @@ void run_gemm_f32(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, 
     // only tall ones, whose packed weights many rows share: [6400,320] x [640,320]
     // 24.5 / 23.9, [2400,512] x [1024,512] 35 / 21, [4800,512] x [512,512] 36 / 23 to 29;
     // below, [4096,512] x [512,512] 19.5 / 21.4, [1024,1024] x [1024,1024] 18.8 / 22.8,
-    // [330,640] x [5120,640] 23 / 28. Operands that the library path does not take: from
-    // the size where the kernel below is slower ([130,33] x [70,33] 8.6 / 9.3, [257,321] x
-    // [300,321] 31.6 / 10.8).
+    // [330,640] x [5120,640] 23 / 28. Not with under 256 columns ([8192,2048] x [128,2048]
+    // 38 / 47) or a K that the pack cannot hold in registers ([512,65536] x [128,65536] 74 /
+    // 223), nor a short one of few rows ([300,128] x [40000,128] 37 / 42) or, from 2.4 GFLOP, one
+    // longer than the row that it makes ([2048,1200] x [512,1200] 26 / 29). Operands that the library
+    // path does not take: from the size where the kernel below is slower ([130,33] x [70,33]
+    // 8.6 / 9.3, [257,321] x [300,321] 31.6 / 10.8).
     const double flops = 2.0 * (double)M * (double)N * (double)K;
-    const bool large = N >= 128 && ((flops >= 3e9 && M >= 256) || (flops >= 2.4e9 && M >= 2048));
+    const bool large = N >= 256 && K <= 16384 &&
+                       ((flops >= 3e9 && M >= 256 && (M >= 512 || K >= 256)) || (flops >= 2.4e9 && M >= 2048 && K <= N));
     if (K > 0 && apart && (lt ? large : K >= 64 && M >= 16 && N >= 16) &&
         split_gemm(M, N, K, A, lda, B, ldb, C, ldc, bias, accumulate)) {
         launched(op);

@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void k_conv_max(ConvPack a) {
         const int p = min((int)p0 + t, a.HW - 1);  // past the last pixel: that one again
         float v[kStep];
 #pragma unroll
-        for (int c = 0; c < kStep; ++c) v[c] = x[(int64_t)min(c, a.Cin - 1 - c0) * a.HW + p];
+        for (int c = 0; c < kStep; ++c) v[c] = x[(int64_t)min(c, a.Cin - 1 - c0) * a.HW + p];  // likewise
 #pragma unroll
         for (int c = 0; c < kStep; ++c) {
             const unsigned b = absbits(v[c]);
@@ -331,11 +331,20 @@ __device__ __forceinline__ int wave_imax(int v) { return (int)dev::wave_max((flo
 __device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) {
     constexpr int kNone = -1000;
     const int t = threadIdx.x, lane = t & 63, words = a.N * a.chunks * a.parts;
+    if (a.parts > 64) {  // at most kMaxima / 128 entries
+        if (t < a.N * a.chunks) E[t] = 0;
+        __syncthreads();
+    }
     for (int i0 = t - lane; i0 < words; i0 += 256) {
         const int i = i0 + lane;
         unsigned m = i < words ? a.maxima[i] : 0u;
-        for (int o = 1; o < a.parts; o <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-        if (lane % a.parts == 0 && i < words) E[i / a.parts] = m ? max((int)(m >> 23), 1) : 0;
+        for (int o = 1; o < min(a.parts, 64); o <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
+        const int e = m ? max((int)(m >> 23), 1) : 0;
+        if (a.parts <= 64) {
+            if (lane % a.parts == 0 && i < words) E[i / a.parts] = e;
+        } else if (lane == 0) {
+            atomicMax(E + i / a.parts, e);
+        }
     }
     for (int c = t; c < a.chunks; c += 256) ec[c] = kNone;
     __syncthreads();
@@ -1393,7 +1402,7 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
         a.x = x + n0 * Cin * HW;
         a.N = (int)ns;
         a.parts = 1;
-        while (a.parts < 64 && a.parts * 256 < HW && ns * chunks * a.parts * 2 <= kMaxima) a.parts *= 2;
+        while (a.parts * 256 < HW && ns * chunks * a.parts * 2 <= kMaxima) a.parts *= 2;
         // all channels of a pixel tile in one workgroup where that leaves at least four workgroups per
         // CU, and several tiles where it leaves sixteen rounds of those
         const int64_t pt = a.tiles * ns;

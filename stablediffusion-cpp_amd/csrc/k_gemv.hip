@@ -144,8 +144,10 @@ void launch(const float* A, int64_t lda, const B* W, int64_t ldb, float* C, int6
 template <class B>
 bool run(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const B* W, int64_t ldb, float* C, int64_t ldc,
          const float* bias, bool accumulate) {
-    // the library's tiles take large layers of five to eight rows (see above)
-    if (M > 8 || (M > 4 && N * K > (int64_t(1) << 22)) || K >= (1 << 30) || N * 64 >= kMaxGridItems) return false;
+    // the library's tiles take large layers of five to eight rows (see above), and very large
+    // bf16 ones of three or four ([4,1024] x [151936,1024] 58 us there, 106 here; [4,11008] x
+    // [4096,11008] 23 and 28; [4,4096] x [4096,4096] still gains)
+    if (M > 8 || (M > 4 && N * K > (int64_t(1) << 22)) || (M > 2 && sizeof(B) == 2 && N * K > (int64_t(1) << 25)) || K >= (1 << 30) || N * 64 >= kMaxGridItems) return false;
     const int m = (int)M;
     if (m == 1) launch<B, 1>(A, lda, W, ldb, C, ldc, bias, m, N, (int)K, accumulate);
     else if (m == 2) launch<B, 2>(A, lda, W, ldb, C, ldc, bias, m, N, (int)K, accumulate);
