@@ -348,8 +348,8 @@ __device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) 
     }
     for (int c = t; c < a.chunks; c += 256) ec[c] = kNone;
     __syncthreads();
-    // a chunk's largest (own - sample's) over the samples; many chunks have few samples (kTable)
-    if (a.chunks <= 32) {  // a lane per sample
+    // a chunk's largest (own - sample's) over the samples, the shorter way (at most 45 turns: kTable)
+    if (a.chunks < a.N) {  // a lane per sample
         for (int n0 = t - lane; n0 < a.N; n0 += 256) {
             const int n = min(n0 + lane, a.N - 1);
             int whole = 0;
@@ -589,7 +589,7 @@ __device__ __forceinline__ float dot_share(const SplitArgs& p, int row, int col,
         const int e = p.ea[row], end = weights_of(p, row);
         if (e == kBad) return __builtin_nanf("");
         const float* b = p.B0 + (int64_t)col * p.ldb;
-#pragma unroll 8
+#pragma unroll 4
         for (int k = t; k < end; k += T) s = fmaf(packed_weight(p, row, e, k), b[k], s);
     } else {
         const float* a = p.A0 + (int64_t)row * p.lda;
@@ -1226,10 +1226,8 @@ size_t up(size_t n) { return (n + 255) / 256 * 256; }
 // `cu` workgroups of a tile; a round of workgroups takes `full` us per step with
 // every CU full, `idle` us with few workgroups, and `once` us to start and to
 // store; parts of K add a launch and the traffic of their sums. The constants are
-// a fit (6 % rms) to 270 timings of 33 shapes, M and N from 64 to 262144 and 3 to
-// 720 steps, under every tile and 1 to 8 parts: over these shapes the tile and
-// the parts with the lowest estimate were the fastest measured, or within 4 % of
-// it in 30 and 13 % in all. Measured at the ends of the range, best tile in
+// a fit to timings of every tile with 1 to 8 parts, M and N from 64 to 262144 and
+// 3 to 720 steps. Measured at the ends of the range, best tile in
 // front: [4096,320] x [320,320] 14.6 us with 64 x 64, 20.0 with 128 x 128;
 // conv [1,256,256,256] to 256 channels 226 us with 256 x 256, 246 with 128 x 256,
 // 273 with 128 x 128; conv [2,2560,8,8] to 1280 channels 119 us with 64 x 64 in
