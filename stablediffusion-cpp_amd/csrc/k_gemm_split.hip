@@ -1360,6 +1360,7 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
                 int64_t kw, const float* bias, int stride, int pad, float* out, int64_t Ho, int64_t Wo) {
     const int64_t HW = H * W, HWo = Ho * Wo, taps = kh * kw, chunks = (Cin + kStep - 1) / kStep, steps = chunks * taps;
     const int64_t cols = N * HWo;
+    if (HW == 0) return false;  // outputs that see padding only
     // 32-bit offsets, also of a padded tile's first pixel
     if ((N * HW + (int64_t)pad * (W + 1) + 1) * kRowBytes >= kMost || cols >= kMost - 256 || Cout * kRowBytes >= kMost ||
         steps >= kMost || Cin * taps >= kMost || N > 65535 || N * Cin * HW >= kMost * 64)

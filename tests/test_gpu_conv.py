@@ -67,3 +67,14 @@ def test_conv2d_in_place(be, orc):
         be.conv2d(dx, N, C, H, W, be.array(w), C, k, k, None, 1, k // 2, dx, H, W)
         want, S = orc.conv2d(x, w, None, 1, k // 2)
         assert_gemm(dx.download(), want, S, C * k * k + 2, f"in place {k}x{k}")
+
+
+@pytest.mark.parametrize("H,W", [(0, 5), (4, 0), (0, 0)])
+def test_conv2d_of_no_pixels(be, orc, H, W):
+    """An image without pixels under padding: every output is the bias."""
+    N, Cin, Cout, k, pad = 2, 3, 4, 3, 2
+    Ho, Wo = H + 2 * pad - k + 1, W + 2 * pad - k + 1
+    b = orc.randn((Cout,), 8201)
+    out = be.empty((N, Cout, Ho, Wo))
+    be.conv2d(be.empty((1,)), N, Cin, H, W, be.randn((Cout, Cin, k, k), 8202), Cout, k, k, be.array(b), 1, pad, out, Ho, Wo)
+    assert np.array_equal(out.download(), np.broadcast_to(b[None, :, None, None], (N, Cout, Ho, Wo)))
