@@ -223,26 +223,27 @@ __global__ __launch_bounds__(256, TURNS < 4 ? 8 : 4) void k_split_pack(PackRows 
 }
 
 // ---------------------------------------------------------------------------
-// conv2d's pack. Launch 1: the largest values of the weights per row and 32
-// channels, and of x per sample, 32 channels and part of the pixels. Every
-// workgroup of launch 2 reads all of x's, so there are at most kMaxima, or kTable
-// where samples and channels alone are more. Launch 2: the exponents, then the
-// weights and the pixels.
-//
+// conv2d's pack. Launch 1: the weights, and the largest values of x per sample, 32
+// channels and part of the pixels. Every workgroup of launch 2 reads all of these,
+// so there are at most kMaxima, or kTable where samples and channels alone are
+// more. Launch 2: the exponents, then the pixels, and the weights once more where
+// they take over some of x's scale.
 // Channels of unlike scale: chunk c of 32 channels has an exponent ec of its own
 // besides the sample's es, and the weights of these channels take 2^ec before
 // their row's exponent is found, so that x w keeps its value. With f the largest
-// over the samples of (chunk's exponent - sample's), ec is f / 2: x and w share
-// the spread, and neither loses bits while it is below 2^34, whether the weights
-// are alike, reciprocal to it, or zero where x is large.
+// over the samples of (chunk's exponent - sample's), ec is f / 2 from -kNear on: x
+// and w share the spread, and neither loses bits while it is below 2^34, whether the
+// weights are alike, reciprocal to it, or zero where x is large. Chunks nearer to
+// their sample, as a rule all of them, leave the weights as launch 1 packed them:
+// packing them after the maxima, or reading them twice, took 3 to 9 us more
+// ([1280,1280,3,3]: 59 MB).
 // ---------------------------------------------------------------------------
-constexpr int kTable = 2048, kMaxima = 256;
+constexpr int kTable = 2048, kMaxima = 256, kNear = 8;
 
 struct ConvPack {
     const float* x;       // [N, Cin, HW]
     const float* w;       // [Cout, Cin, taps]
     unsigned* maxima;     // [N, chunks, parts], of finite values
-    unsigned* wmaxima;    // [Cout, chunks]; kInf: not all finite
     u16* X;               // planes of N * HW + 1 pixels
     u16* Wp;              // planes of Cout rows
     int* ex;              // [N]
@@ -255,53 +256,72 @@ struct ConvPack {
     int tiles, run, runs; // 64-pixel tiles of a sample; tiles that a workgroup packs; such runs
 };
 
-__global__ __launch_bounds__(256) void k_conv_max(ConvPack a) {
-    __shared__ unsigned red[4];
-    const int t = threadIdx.x, lane = t & 63, nx = gridDim.x - a.Cout, b = (int)blockIdx.x - a.Cout;
-    if (b < 0) {  // an output channel: a wave per 32 channels
-        const int K = a.Cin * a.taps, chunk = kStep * a.taps, co = blockIdx.x;
-        const float* w = a.w + (int64_t)co * K;
-        constexpr int U = 8;  // loads of a lane on their way at once: 512 weights of a chunk, the next chunk's behind them
-        float v[U], x[U];
-        if (a.taps == 1) {  // half a wave per chunk
-            for (int k0 = t; k0 - lane < a.chunks * kStep; k0 += U * 256) {
+// One output channel's weights: [Cin][taps] -> steps (32 channels, tap), through
+// LDS where there is room for them at `row`. FOLD: with 2^ec.
+template <bool FOLD>
+__device__ __forceinline__ void conv_pack_weights(const ConvPack& a, int co, const int* ec, float* row, unsigned* red) {
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, K = a.Cin * a.taps, chunk = kStep * a.taps;
+    const float* w = a.w + (int64_t)co * K;
+    // the largest |w| 2^ec by its bits with ec added to the exponent: floor(that / 2^23) bounds the
+    // magnitude also where the exponent falls below 1, or the weight is subnormal or zero
+    int m = INT_MIN, top = 0;
+    int c = t / chunk, r = t - c * chunk;  // FOLD: the weight's chunk, its place there
+    const int dc = 256 / chunk, dr = 256 - dc * chunk;
+    constexpr int U = 8;
+    for (int k0 = t; k0 < K; k0 += U * 256) {
+        float v[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = w[min(k0 + u * 256, K - 1)];
+        for (int u = 0; u < U; ++u) v[u] = w[min(k0 + u * 256, K - 1)];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int c = (k0 + u * 256) / kStep;
-                    const uint64_t bad = __ballot(absbits(v[u]) >= kInf) >> (lane & 32) << 32;
-                    float f = dev::group_max<16>(fabsf(v[u]));
-                    f = fmaxf(f, __shfl_xor(f, 16, 64));
-                    const unsigned m = __float_as_uint(f);
-                    if ((lane & 31) == 0 && c < a.chunks) a.wmaxima[(int64_t)co * a.chunks + c] = bad ? kInf : m;
-                }
+        for (int u = 0; u < U; ++u) {
+            if (k0 + u * 256 >= K) break;
+            if (row) row[k0 + u * 256] = v[u];
+            const int b = (int)absbits(v[u]);
+            top = max(top, b);
+            if constexpr (FOLD) {
+                m = max(m, b + ec[c] * (1 << 23));
+                r += dr;
+                const int over = r >= chunk ? 1 : 0;
+                c += dc + over;
+                r -= over ? chunk : 0;
             }
-            return;
         }
-        auto load = [&](int c, int k0) __attribute__((always_inline)) {  // past the chunk or the row: its last one again
-            const int last = min(K, (c + 1) * chunk) - 1;
+    }
+    if constexpr (!FOLD) m = top;
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (k0 + u * 64 < chunk) v[u] = w[min(c * chunk + k0 + u * 64 + lane, last)];
-        };
-        int c = __builtin_amdgcn_readfirstlane(t >> 6);
-        if (c < a.chunks) load(c, 0);
-        for (; c < a.chunks; c += 4) {
-            unsigned m = 0;
-            for (int k0 = 0; k0 < chunk; k0 += U * 64) {
+    for (int o = 32; o; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+    if (lane == 0) red[wv] = (unsigned)m;
+    const bool bad = __syncthreads_or(top >= (int)kInf);
+    m = max(max((int)red[0], (int)red[1]), max((int)red[2], (int)red[3]));
+    const int e = (m >> 23) - 141;  // scaled by 2^(ec - e) the largest lies below 2^15
+    if (t == 0) a.ew[co] = bad ? kBad : e;
+    const int tasks = a.chunks * a.taps * 4;
+    unsigned tail = 0;
+    for (int i = t; i < tasks; i += 256) {  // eight channels of one step
+        const int g = i & 3, step = i >> 2, cc = step / a.taps, tap = step - cc * a.taps, c0 = cc * kStep + g * 8;
+        float v[8];
 #pragma unroll
-                for (int u = 0; u < U; ++u) x[u] = v[u];
-                if (k0 + U * 64 < chunk) load(c, k0 + U * 64);
-                else if (c + 4 < a.chunks) load(c + 4, 0);
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (k0 + u * 64 < chunk) m = max(m, absbits(x[u]));
-            }
-            const bool bad = __any(m >= kInf);
-            m = __float_as_uint(dev::wave_max(__uint_as_float(m)));
-            if (lane == 0) a.wmaxima[(int64_t)co * a.chunks + c] = bad ? kInf : m;
+        for (int j = 0; j < 8; ++j) {
+            const int k = min((c0 + j) * a.taps + tap, K - 1);
+            const float x = row ? row[k] : w[k];
+            v[j] = c0 + j < a.Cin ? x : 0.f;
         }
+        const int shift = (FOLD ? ec[cc] : 0) - e;
+        tail += store_split(a.Wp + ((int64_t)step * a.Cout + co) * (kRowBytes / 2) + g * 8, v, bad ? 0 : shift);
+    }
+    tail = __any(tail != 0) ? wave_usum(tail) : 0u;
+    if (lane == 0) red[4 + wv] = tail;
+    __syncthreads();
+    if (t == 0) a.tw[co] = bad ? kNotFinite : (red[4] + red[5]) + (red[6] + red[7]);
+}
+
+__global__ __launch_bounds__(256) void k_conv_prep(ConvPack a, int in_lds) {
+    extern __shared__ float row[];
+    __shared__ unsigned red[8];
+    const int t = threadIdx.x, nx = gridDim.x - a.Cout, b = (int)blockIdx.x - a.Cout;
+    if (b < 0) {
+        if (in_lds) conv_pack_weights<false>(a, blockIdx.x, nullptr, row, red);
+        else conv_pack_weights<false>(a, blockIdx.x, nullptr, nullptr, red);
         return;
     }
     for (int i = b * 256 + t; i <= a.N * a.HW; i += nx * 256) a.tx[i] = 0;
@@ -371,7 +391,7 @@ __device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) 
         }
     }
     __syncthreads();
-    for (int c = t; c < a.chunks; c += 256) ec[c] = ec[c] == kNone ? 0 : ec[c] / 2;  // from -126 on
+    for (int c = t; c < a.chunks; c += 256) ec[c] = ec[c] == kNone || ec[c] > -kNear ? 0 : ec[c] / 2;  // from -126 on
     __syncthreads();
 }
 // A sample's exponent beside those: its scaled values lie below 2^15.
@@ -384,39 +404,6 @@ __device__ __forceinline__ int conv_sample_exp(const ConvPack& a, const int* E, 
     }
     e = wave_imax(e);
     return e == kNone ? 0 : e;
-}
-
-// One output channel's weights: [Cin][taps] -> steps (32 channels, tap).
-__device__ __forceinline__ void conv_pack_weights(const ConvPack& a, int co, const int* ec, unsigned* red) {
-    const int t = threadIdx.x, lane = t & 63, K = a.Cin * a.taps;
-    const float* w = a.w + (int64_t)co * K;
-    // its exponent: every wave finds it; a chunk of zeros counts as the smallest weights
-    int m = -1000;
-    bool bad = false;
-    for (int c = lane; c < a.chunks; c += 64) {
-        const unsigned b = a.wmaxima[(int64_t)co * a.chunks + c];
-        bad |= b >= kInf;
-        m = max(m, (int)(b >> 23) + ec[c]);
-    }
-    bad = __any(bad);
-    const int e = wave_imax(m) - 141;  // scaled by 2^(ec - e) the largest lies below 2^15
-    if (t == 0) a.ew[co] = bad ? kBad : e;
-    const int tasks = a.chunks * a.taps * 4;
-    unsigned tail = 0;
-    for (int i = t; i < tasks; i += 256) {  // eight channels of one step
-        const int g = i & 3, step = i >> 2, c = step / a.taps, tap = step - c * a.taps, c0 = c * kStep + g * 8;
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float x = w[min((c0 + j) * a.taps + tap, K - 1)];
-            v[j] = c0 + j < a.Cin ? x : 0.f;
-        }
-        tail += store_split(a.Wp + ((int64_t)step * a.Cout + co) * (kRowBytes / 2) + g * 8, v, bad ? 0 : ec[c] - e);
-    }
-    tail = __any(tail != 0) ? wave_usum(tail) : 0u;
-    if (lane == 0) red[t >> 6] = tail;
-    __syncthreads();
-    if (t == 0) a.tw[co] = bad ? kNotFinite : (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // `run` times 64 pixels of a sample, `per` steps of 32 channels; each step through
@@ -481,16 +468,19 @@ __device__ __forceinline__ void conv_pack_pixels(const ConvPack& a, int b, const
 
 __global__ __launch_bounds__(256) void k_conv_pack(ConvPack a) {
     extern __shared__ int lds[];
-    __shared__ unsigned red[4];
+    __shared__ unsigned red[8];
     __shared__ __attribute__((aligned(16))) u16 tile[64 * 64];
     int *E = lds, *ec = E + a.N * a.chunks;
     auto scales = [&]() __attribute__((always_inline)) { conv_scales(a, E, ec); };
-    if ((int)blockIdx.x < a.Cout) {
-        scales();
-        conv_pack_weights(a, blockIdx.x, ec, red);
-    } else {
-        conv_pack_pixels(a, blockIdx.x - a.Cout, E, ec, tile, scales);
+    const int pixels = a.runs * a.groups * a.N;
+    if ((int)blockIdx.x < pixels) {
+        conv_pack_pixels(a, blockIdx.x, E, ec, tile, scales);
+        return;
     }
+    scales();
+    bool fold = false;
+    for (int c = threadIdx.x; c < a.chunks; c += 256) fold |= ec[c] != 0;
+    if (__syncthreads_or(fold)) conv_pack_weights<true>(a, blockIdx.x - pixels, ec, nullptr, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1304,6 +1294,7 @@ void launch_pack(const PackRows& a, const PackRows& b, int64_t batches) {
     go<<<dim3(ba + bb, (unsigned)batches), 256, 0, stream()>>>(a, b, (int)ba);
 }
 
+constexpr size_t kRowLds = 48 << 10;  // weights of one output channel that k_conv_prep takes through LDS
 constexpr int64_t kMost = int64_t(1) << 31;
 
 }  // namespace
@@ -1374,17 +1365,16 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
     if (std::max(grid(whole), grid(rest)) * 512 >= kMost) return false;
     const int64_t prows = most * HW + 1;
     const size_t px = up((size_t)chunks * prows * kRowBytes), pw = up((size_t)steps * Cout * kRowBytes);
-    const size_t mx = up((size_t)kTable * 4), wm = up((size_t)(Cout * chunks) * 4), tx = up((size_t)prows * 4), ex = up((size_t)most * 4);
+    const size_t mx = up((size_t)kTable * 4), tx = up((size_t)prows * 4), ex = up((size_t)most * 4);
     const size_t ew = up((size_t)Cout * 4), lc = up((size_t)most * HWo * 4);
-    char* s = (char*)try_scratch(px + pw + mx + wm + tx + ex + 2 * ew + lc + std::max(whole.part_bytes(), rest.part_bytes()));
+    char* s = (char*)try_scratch(px + pw + mx + tx + ex + 2 * ew + lc + std::max(whole.part_bytes(), rest.part_bytes()));
     if (!s) return false;
     ConvPack a{};
     a.w = w;
     a.X = (u16*)s;
     a.Wp = (u16*)(s += px);
     a.maxima = (unsigned*)(s += pw);
-    a.wmaxima = (unsigned*)(s += mx);
-    a.tx = (unsigned*)(s += wm);
+    a.tx = (unsigned*)(s += mx);
     a.ex = (int*)(s += tx);
     a.ew = (int*)(s += ex);
     a.tw = (unsigned*)(s += ew);
@@ -1410,7 +1400,9 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
         a.groups = (int)((chunks + a.per - 1) / a.per);
         a.run = (int)std::max<int64_t>(1, pt * a.groups / (64 * num_cus()));
         a.runs = (a.tiles + a.run - 1) / a.run;
-        k_conv_max<<<(unsigned)(Cout + ns * chunks * a.parts), 256, 0, stream()>>>(a);
+        const size_t row = (size_t)(Cin * taps) * 4;
+        const bool in_lds = row <= kRowLds;
+        k_conv_prep<<<(unsigned)(Cout + ns * chunks * a.parts), 256, in_lds ? row : 0, stream()>>>(a, in_lds ? 1 : 0);
         k_conv_pack<<<(unsigned)(Cout + (int64_t)a.runs * a.groups * ns), 256, (size_t)((ns + 1) * chunks) * 4, stream()>>>(a);
         SplitArgs p{};
         p.A = a.Wp;
