@@ -3,7 +3,7 @@
 // The implicit GEMM on split fp16 operands (k_gemm_split.hip) takes it: [1,256,512,512]
 // to 256 channels, 3x3: 6.4 ms with the path below, 0.90-0.96 ms there; [2,4,64,64] to 320: 32
 // and 22 us. One sample of few pixels and many channels is slower there (3x3, 8x8, 1280 to
-// 1280: 29 and 58 us; 1x1, 16x16, 1280 to 1280: 19 and 31) and stays for its smaller error
+// 1280: 29 and 50 us; 1x1, 16x16, 1280 to 1280: 19 and 28) and stays for its smaller error
 // (4e-7 where the path below gives 1.1e-6). What follows runs where that
 // one's scratch (see sdh_conv2d) does not fit the arena or would have
 // to grow during a capture, in at most 128 MB: per sample, pixels in chunks of at

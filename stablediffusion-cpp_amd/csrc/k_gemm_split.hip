@@ -346,9 +346,9 @@ __global__ __launch_bounds__(256) void k_conv_prep(ConvPack a, int in_lds) {
 }
 
 // Exponents from the maxima: E [N, chunks], the chunks' biased ones (bits >> 23, at
-// least 1; 0: all zero), and ec [chunks]. By the whole workgroup.
+// least 1; 0: all zero), and ec [chunks]; S [N]: the samples'. By the whole workgroup.
 __device__ __forceinline__ int wave_imax(int v) { return (int)dev::wave_max((float)v); }  // |v| < 2^24
-__device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) {
+__device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* S, int* ec) {
     constexpr int kNone = -1000;
     const int t = threadIdx.x, lane = t & 63, words = a.N * a.chunks * a.parts;
     if (a.parts > 64) {  // at most kMaxima / 128 entries
@@ -366,10 +366,12 @@ __device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) 
             atomicMax(E + i / a.parts, e);
         }
     }
-    for (int c = t; c < a.chunks; c += 256) ec[c] = kNone;
+    if (a.chunks < a.N)
+        for (int c = t; c < a.chunks; c += 256) ec[c] = kNone;
     __syncthreads();
-    // a chunk's largest (own - sample's) over the samples, the shorter way (at most 45 turns: kTable)
-    if (a.chunks < a.N) {  // a lane per sample
+    // f, a chunk's largest (own - sample's) over the samples
+    auto folded = [](int f) __attribute__((always_inline)) { return f == kNone || f > -kNear ? 0 : f / 2; };  // from -126 on
+    if (a.chunks < a.N) {  // a lane per sample, at most 45 chunks (kTable)
         for (int n0 = t - lane; n0 < a.N; n0 += 256) {
             const int n = min(n0 + lane, a.N - 1);
             int whole = 0;
@@ -379,19 +381,25 @@ __device__ __forceinline__ void conv_scales(const ConvPack& a, int* E, int* ec) 
                 if (lane == 0) atomicMax(ec + c, f);
             }
         }
-    } else {  // a thread per chunk
-        for (int n = 0; n < a.N; ++n) {
+        __syncthreads();
+        for (int c = t; c < a.chunks; c += 256) ec[c] = folded(ec[c]);
+    } else {  // a thread per chunk; a wave finds every fourth sample's, of one sample each wave for itself
+        for (int n = a.N > 1 ? t >> 6 : 0; n < a.N; n += 4) {
             int whole = 0;
             for (int c = lane; c < a.chunks; c += 64) whole = max(whole, E[n * a.chunks + c]);
-            whole = wave_imax(whole);
-            for (int c = t; c < a.chunks; c += 256) {
+            S[n] = wave_imax(whole);  // the same from every lane
+        }
+        if (a.N > 1) __syncthreads();
+        for (int c = t; c < a.chunks; c += 256) {
+            int f = kNone;
+#pragma unroll 4
+            for (int n = 0; n < a.N; ++n) {
                 const int own = E[n * a.chunks + c];
-                if (own) ec[c] = max(ec[c], own - whole);
+                f = max(f, own ? own - S[n] : kNone);
             }
+            ec[c] = folded(f);
         }
     }
-    __syncthreads();
-    for (int c = t; c < a.chunks; c += 256) ec[c] = ec[c] == kNone || ec[c] > -kNear ? 0 : ec[c] / 2;  // from -126 on
     __syncthreads();
 }
 // A sample's exponent beside those: its scaled values lie below 2^15.
@@ -470,8 +478,8 @@ __global__ __launch_bounds__(256) void k_conv_pack(ConvPack a) {
     extern __shared__ int lds[];
     __shared__ unsigned red[8];
     __shared__ __attribute__((aligned(16))) u16 tile[64 * 64];
-    int *E = lds, *ec = E + a.N * a.chunks;
-    auto scales = [&]() __attribute__((always_inline)) { conv_scales(a, E, ec); };
+    int *E = lds, *ec = E + a.N * a.chunks, *S = ec + a.chunks;
+    auto scales = [&]() __attribute__((always_inline)) { conv_scales(a, E, S, ec); };
     const int pixels = a.runs * a.groups * a.N;
     if ((int)blockIdx.x < pixels) {
         conv_pack_pixels(a, blockIdx.x, E, ec, tile, scales);
@@ -1403,7 +1411,7 @@ bool split_conv(const float* x, int64_t N, int64_t Cin, int64_t H, int64_t W, co
         const size_t row = (size_t)(Cin * taps) * 4;
         const bool in_lds = row <= kRowLds;
         k_conv_prep<<<(unsigned)(Cout + ns * chunks * a.parts), 256, in_lds ? row : 0, stream()>>>(a, in_lds ? 1 : 0);
-        k_conv_pack<<<(unsigned)(Cout + (int64_t)a.runs * a.groups * ns), 256, (size_t)((ns + 1) * chunks) * 4, stream()>>>(a);
+        k_conv_pack<<<(unsigned)(Cout + (int64_t)a.runs * a.groups * ns), 256, (size_t)(ns * chunks + chunks + ns) * 4, stream()>>>(a);
         SplitArgs p{};
         p.A = a.Wp;
         p.B = a.X;
